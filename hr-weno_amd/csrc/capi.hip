@@ -941,7 +941,7 @@ static int run_stage_sets(const hrw_problem_s *p, const unsigned long long *ain,
         a.h = h;
         a.stage = stage;
         a.ty = p->ty;
-        const int sw = strip_width(p->k, p->arith == HRW_ARITH_FAST);
+        const int sw = strip_width(p->k);
         a.nstrips = (p->n1 + sw - 1) / sw;
         launch_stage2d(p, a, s);
     }

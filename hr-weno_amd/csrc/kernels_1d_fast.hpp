@@ -31,22 +31,6 @@
 
 namespace hrw {
 
-// 1/x to ~1 ulp: hardware estimate + two Newton steps.
-__device__ __forceinline__ double rcp_nr(double x)
-{
-    double r = __builtin_amdgcn_rcp(x);
-    double e = fma_(-x, r, 1.0);
-    r = fma_(r, e, r);
-    e = fma_(-x, r, 1.0);
-    return fma_(r, e, r);
-}
-
-// Shared pieces of the triple (a, b, c) = (v_m, v_m+1, v_m+2) for K = 3.
-struct Tri3 {
-    double bA, bB, bC;       // 12*beta_0(m), 12*beta_1(m+1), 12*beta_2(m+2)
-    double Pm, P0, P1, P2;   // 6*c(:,-1).T, 6*c(:,0).T, 6*c(:,1).T, 6*c(:,2).T
-};
-
 // With D = a - 2b + c, E = a - c, X = 2D + E, Y = 2D - E:  12 beta = 13 D^2 + 3 E^2 (middle),
 // 13 D^2 + 3 X^2, 13 D^2 + 3 Y^2; and the candidates follow from P0 = 2a + 5b - c by one term
 // each: P1 = P0 - 3E, Pm = P0 + 3X, P2 = P1 + 3Y (18 operations instead of 23).
@@ -107,9 +91,6 @@ __device__ __forceinline__ void recon3(double eps12, const Tri3 &t2, const Tri3 
 
 // K = 2: pair (a, b) = (v_m, v_m+1) gives beta_0(m) = beta_1(m+1) = (b-a)^2 and the
 // candidates 2*vrr0(m) = a+b = 2*vlr1(m+1), 2*vrr1(m+1) = 3b-a, 2*vlr0(m) = 3a-b.
-struct Pair2 {
-    double B, S, Rr, Lr;
-};
 __device__ __forceinline__ Pair2 pair2(double a, double b)
 {
     Pair2 p;

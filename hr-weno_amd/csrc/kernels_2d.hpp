@@ -8,7 +8,7 @@
 // along x2 (a window sliding down the column in registers) and along x1 (its window gathered
 // from the neighbouring lanes' column values by lane shifts, plus K-1 halo values loaded by
 // the edge lanes).  Interface fluxes along x1 pass between neighbouring lanes the same way, so
-// lanes 1..62 own output cells.  (K = 3, FAST: columns X0-2 .. X0+61, lanes 2..61 own, and the
+// lanes 1..62 own output cells.  (K = 3: columns X0-2 .. X0+61, lanes 2..61 own, and the
 // x1 smoothness triples are shared between lanes -- strip_width.)  Each cell value is read
 // from HBM once per row band.
 #pragma once
@@ -33,24 +33,43 @@ struct Stage2DArgs {
 };
 
 constexpr int kStrip = 62;
-// Output columns of a wavefront's strip.  K = 3 in the FAST form: 60, with two halo lanes each
+// Output columns of a wavefront's strip.  K = 3: 60, with two halo lanes each
 // side, so that every lane forms only the smoothness triple centred on its own column and takes
 // the triples of its neighbours' columns by lane shifts (the outer halo lanes' centred triples
 // feed lanes 1 and 62, whose reconstructions give the strip's two outer fluxes).
-__host__ __device__ constexpr int strip_width(int K, bool fast) { return (K == 3 && fast) ? 60 : kStrip; }
+__host__ __device__ constexpr int strip_width(int K) { return K == 3 ? 60 : kStrip; }
+
+// The shared pieces and their reconstruction in either arithmetic form.
+template <bool FAST> __device__ __forceinline__ Tri3 triple(double a, double b, double c)
+{
+    if constexpr (FAST) return tri3(a, b, c);
+    else return tri3_exact(a, b, c);
+}
+template <bool FAST>
+__device__ __forceinline__ void recon_triples(double eps, const Tri3 &t2, const Tri3 &t1,
+                                              const Tri3 &t0, double &vl, double &vr)
+{
+    if constexpr (FAST) recon3<false, true>(12.0 * eps, t2, t1, t0, vl, vr);
+    else recon3_exact(eps, t2, t1, t0, vl, vr);
+}
+template <bool FAST> __device__ __forceinline__ Pair2 pair(double a, double b)
+{
+    if constexpr (FAST) return pair2(a, b);
+    else return pair2_exact(a, b);
+}
+template <bool FAST>
+__device__ __forceinline__ void recon_pairs(double eps, const Pair2 &p1, const Pair2 &p0,
+                                            double &vl, double &vr)
+{
+    if constexpr (FAST) recon2(eps, p1, p0, vl, vr);
+    else recon2_exact(eps, p1, p0, vl, vr);
+}
 
 template <int K, bool FAST>
 __device__ __forceinline__ void recon(const double *x, double eps, double &vl, double &vr)
 {
-    if constexpr (!FAST) {
-        weno_cell_exact<K>(x, eps, nullptr, vl, vr);
-    } else if constexpr (K == 3) {   // the 1D kernel's form (scaled triples, reciprocals)
-        recon3<false, true>(12.0 * eps, tri3(x[0], x[1], x[2]), tri3(x[1], x[2], x[3]), tri3(x[2], x[3], x[4]), vl, vr);
-    } else if constexpr (K == 2) {
-        recon2(eps, pair2(x[0], x[1]), pair2(x[1], x[2]), vl, vr);
-    } else {
-        vl = vr = x[0];
-    }
+    if constexpr (K == 2) recon_pairs<FAST>(eps, pair<FAST>(x[0], x[1]), pair<FAST>(x[1], x[2]), vl, vr);
+    else vl = vr = FAST ? x[0] : 0.0 + x[0];
 }
 
 // The x2 reconstruction marching down a column: the pieces of each triple (pair) of rows are
@@ -58,30 +77,30 @@ __device__ __forceinline__ void recon(const double *x, double eps, double &vl, d
 template <int K, bool FAST>
 struct ColumnRecon {
     double cw[2 * K - 1];                // u(i, r-K+1 .. r+K-1) for the current row r
-    [[maybe_unused]] Tri3 t2, t1;        // K = 3, FAST: T(r-2), T(r-1)
-    [[maybe_unused]] Pair2 p1;           // K = 2, FAST: pair (r-1, r)
+    [[maybe_unused]] Tri3 t2, t1;        // K = 3: T(r-2), T(r-1)
+    [[maybe_unused]] Pair2 p1;           // K = 2: pair (r-1, r)
 
     __device__ __forceinline__ void start(double eps)
     {
         (void)eps;
-        if constexpr (FAST && K == 3) {
-            t2 = tri3(cw[0], cw[1], cw[2]);
-            t1 = tri3(cw[1], cw[2], cw[3]);
-        } else if constexpr (FAST && K == 2) {
-            p1 = pair2(cw[0], cw[1]);
+        if constexpr (K == 3) {
+            t2 = triple<FAST>(cw[0], cw[1], cw[2]);
+            t1 = triple<FAST>(cw[1], cw[2], cw[3]);
+        } else if constexpr (K == 2) {
+            p1 = pair<FAST>(cw[0], cw[1]);
         }
     }
     // reconstruction of the window now in cw (the triples of its lower part already formed)
     __device__ __forceinline__ void recon_current(double eps, double &vl, double &vr)
     {
-        if constexpr (FAST && K == 3) {
-            const Tri3 t0 = tri3(cw[2], cw[3], cw[4]);
-            recon3<false, true>(12.0 * eps, t2, t1, t0, vl, vr);
+        if constexpr (K == 3) {
+            const Tri3 t0 = triple<FAST>(cw[2], cw[3], cw[4]);
+            recon_triples<FAST>(eps, t2, t1, t0, vl, vr);
             t2 = t1;
             t1 = t0;
-        } else if constexpr (FAST && K == 2) {
-            const Pair2 p0 = pair2(cw[1], cw[2]);
-            recon2(eps, p1, p0, vl, vr);
+        } else if constexpr (K == 2) {
+            const Pair2 p0 = pair<FAST>(cw[1], cw[2]);
+            recon_pairs<FAST>(eps, p1, p0, vl, vr);
             p1 = p0;
         } else {
             recon<K, FAST>(cw, eps, vl, vr);
@@ -136,9 +155,9 @@ __device__ __forceinline__ unsigned xcd_major(unsigned b, unsigned nb)
     return x < r ? x * (q + 1) + loc : r * (q + 1) + (x - r) * q + loc;
 }
 
-// The x1 window of row j, u(clamp(i+m), j) for m = -(K-1)..K-1, from the lanes' centre values
-// c = u(clamp(i), j) and the halo values: lanes 0..K-2 hold u(clamp(i-(K-1)), j) and lanes
-// 64-(K-1)..63 hold u(clamp(i+(K-1)), j).
+// The x1 window of row j for K <= 2, u(clamp(i+m), j) for m = -(K-1)..K-1, from the lanes'
+// centre values c = u(clamp(i), j) and the halo values: lane 0 holds u(clamp(i-(K-1)), j) and
+// lane 63 u(clamp(i+(K-1)), j).
 template <int K>
 __device__ __forceinline__ void x1_window(double c, double halo, double *x)
 {
@@ -146,11 +165,6 @@ __device__ __forceinline__ void x1_window(double c, double halo, double *x)
     if constexpr (K == 2) {
         x[0] = from_left(halo, c);
         x[2] = from_right(halo, c);
-    } else if constexpr (K == 3) {
-        x[1] = from_left(from_right(0.0, halo), c);    // lane 0: lane 1's halo
-        x[0] = from_left(halo, x[1]);                  // lane 0: its own halo
-        x[3] = from_right(from_left(0.0, halo), c);    // lane 63: lane 62's halo
-        x[4] = from_right(halo, x[3]);                 // lane 63: its own halo
     }
 }
 
@@ -171,8 +185,8 @@ __device__ __forceinline__ void pbe2d_wave(const Stage2DArgs &a)
     const long long Y0 = sy * a.ty;
     if (Y0 >= n2) return;                               // whole wavefront leaves together
     const int Y1 = (int)min((long long)n2, Y0 + a.ty);
-    constexpr bool SHARE = K == 3 && FAST;             // centred triples shared between lanes
-    constexpr int S = strip_width(K, FAST), H0 = SHARE ? 2 : 1;   // output columns, left halo lanes
+    constexpr bool SHARE = K == 3;                     // centred triples shared between lanes
+    constexpr int S = strip_width(K), H0 = SHARE ? 2 : 1;   // output columns, left halo lanes
     const int i = sx * S - H0 + lane;                   // column of this lane (may be < 0 or >= n1)
     auto colc = [n1](int c) { return c < 0 ? 0 : (c >= n1 ? n1 - 1 : c); };
     const int ic = colc(i);                             // clamped column for loads
@@ -249,7 +263,7 @@ __device__ __forceinline__ void pbe2d_wave(const Stage2DArgs &a)
         if constexpr (SHARE) {
             // T(i-1) = (u(i-1), u(i), u(i+1)) here; T(i-2) and T(i) are the neighbours' own
             const double xl = from_left(o.halo, uc), xr = from_right(o.halo, uc);
-            const Tri3 tm = tri3(xl, uc, xr);
+            const Tri3 tm = triple<FAST>(xl, uc, xr);
             Tri3 tl{}, tr{};
             tl.bC = from_left(tm.bC, tm.bC);
             tl.P2 = from_left(tm.P2, tm.P2);
@@ -257,7 +271,7 @@ __device__ __forceinline__ void pbe2d_wave(const Stage2DArgs &a)
             tr.bA = from_right(tm.bA, tm.bA);
             tr.P0 = from_right(tm.P0, tm.P0);
             tr.Pm = from_right(tm.Pm, tm.Pm);
-            recon3<false, true>(12.0 * a.eps, tl, tm, tr, vl1, vr1);
+            recon_triples<FAST>(a.eps, tl, tm, tr, vl1, vr1);
         } else {
             double xw[2 * K - 1];
             x1_window<K>(uc, o.halo, xw);
@@ -303,6 +317,9 @@ __device__ __forceinline__ void pbe2d_wave(const Stage2DArgs &a)
     }
 }
 
+// Bound by FP64 issue (EXACT: about 290 VALU operations per cell, against 62 for its bytes).
+// 2048 x 2048 cells, per RK3 stage: EXACT 81 us with a divide for every quotient and the triples
+// formed per cell, 58 us with shared triples and reciprocals (weights_exact); FAST 41 us.
 template <int K, int BC, bool FAST>
 __global__ __launch_bounds__(kBlock) void pbe2d_kernel(Stage2DArgs a)
 {

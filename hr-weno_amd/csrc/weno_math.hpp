@@ -3,9 +3,10 @@
 // Two arithmetic forms of the same mathematics are provided, selected by a template flag:
 //
 //  * Exact  : the reference's own evaluation order, operation for operation (left-to-right
-//             sums, (eps+beta)**2 as a product, 12 IEEE divides per cell for k=3).  The
-//             library is compiled with -ffp-contract=off, so no multiply-add is fused and the
-//             results are bit-identical to the reference Fortran built for baseline x86-64.
+//             sums, (eps+beta)**2 as a product, 12 correctly rounded divides per cell for k=3).
+//             The library is compiled with -ffp-contract=off, and a multiply-add is fused only
+//             where its product is exact (a power of two), so the results are bit-identical to
+//             the reference Fortran built for baseline x86-64.
 //  * Fast   : the same formulas with explicit fused multiply-adds and the nonlinear weights
 //             consolidated over a common denominator (two divides per cell instead of twelve):
 //                 w_r = d_r/q_r / sum_s d_s/q_s  =  d_r*prod_{s!=r} q_s / sum_s d_s*prod_{t!=s} q_t
@@ -81,13 +82,97 @@ template <int K> HRW_HD void beta_exact(const double *x, double *beta)
     }
 }
 
+// 1/x to within a fraction of an ulp: hardware estimate (2^-24.4) and two Newton steps.
+#if defined(__HIPCC__)
+__device__ __forceinline__ double rcp_nr(double x)
+{
+    double r = __builtin_amdgcn_rcp(x);
+    double e = fma_(-x, r, 1.0);
+    r = fma_(r, e, r);
+    e = fma_(-x, r, 1.0);
+    return fma_(r, e, r);
+}
+
+// n/d correctly rounded, given y = rcp_nr(d): the quotient estimate n*y is within an ulp, its
+// remainder n - d*q is exact in one fused operation, and one correction rounds it (Markstein,
+// "Computation of elementary functions on the IBM RISC System/6000", 1990).  That is the IEEE
+// quotient while no intermediate leaves the normal range: |n| and d between 2^-900 and 2^900,
+// their exponents less than 768 apart (n = +0 is exact too; -0 gives +0).
+__device__ __forceinline__ double quot(double n, double d, double y)
+{
+    const double q = n * y;
+    return fma_(fma_(-d, q, n), y, q);
+}
+#endif
+
+// The nonlinear weights of the right (w) and left (wt) faces from the smoothness indicators,
+// src/hrweno_weno.f90:206-214: alfa_r = d_r/(eps + beta_r)**2, w_r = alfa_r/sum(alfa).  Every
+// quotient is the correctly rounded one; on the device the quotients over one denominator share
+// its reciprocal (5 reciprocals and 11 quotients for k = 3, about 60 operations instead of the
+// 120 of the divides), which needs sum (eps + beta_r)**2 < 2^400 -- with eps > 2^-52 every
+// operand of a quotient then lies in (2^-405, 2^400).  Larger or NaN indicators take the divides.
+template <int K> HRW_HD void weights_exact(const double *beta, double eps, double *w, double *wt)
+{
+    if constexpr (K == 1) {
+        w[0] = wt[0] = 1.0;   // alfa/alfa
+        return;
+    } else {
+        double q[K], alfa[K], alfat[K];
+        double qs = 0.0;
+#pragma unroll
+        for (int r = 0; r < K; ++r) {
+            q[r] = eps + beta[r];
+            q[r] = q[r] * q[r];
+            qs += q[r];
+        }
+#if defined(__HIP_DEVICE_COMPILE__)
+        if (qs < 0x1p400) {
+#pragma unroll
+            for (int r = 0; r < K; ++r) {
+                const double y = rcp_nr(q[r]);
+                alfa[r] = quot(Tab<K>::d[r], q[r], y);
+                alfat[r] = 2 * r == K - 1 ? alfa[r] : quot(Tab<K>::d[K - 1 - r], q[r], y);
+            }
+            double sa = alfa[0], sat = alfat[0];
+#pragma unroll
+            for (int r = 1; r < K; ++r) {
+                sa = sa + alfa[r];
+                sat = sat + alfat[r];
+            }
+            const double ya = rcp_nr(sa), yt = rcp_nr(sat);
+#pragma unroll
+            for (int r = 0; r < K; ++r) {
+                w[r] = quot(alfa[r], sa, ya);
+                wt[r] = quot(alfat[r], sat, yt);
+            }
+            return;
+        }
+#endif
+#pragma unroll
+        for (int r = 0; r < K; ++r) {
+            alfa[r] = Tab<K>::d[r] / q[r];
+            alfat[r] = Tab<K>::d[K - 1 - r] / q[r];
+        }
+        double sa = 0.0, sat = 0.0;
+#pragma unroll
+        for (int r = 0; r < K; ++r) sa = sa + alfa[r];
+#pragma unroll
+        for (int r = 0; r < K; ++r) sat = sat + alfat[r];
+#pragma unroll
+        for (int r = 0; r < K; ++r) {
+            w[r] = alfa[r] / sa;
+            wt[r] = alfat[r] / sat;
+        }
+    }
+}
+
 // Exact form of one cell, src/hrweno_weno.f90:176-214.  ci == nullptr: uniform tables;
 // otherwise ci[(r+1)*K + j] == cnu(j, r, i) (non-uniform grid, eq. 2.20).
 template <int K> HRW_HD void weno_cell_exact(const double *x, double eps, const double *ci,
                                              double &vl, double &vr)
 {
     const double *v = x + (K - 1);
-    double vrr[K], vlr[K], beta[K], alfa[K], alfat[K];
+    double vrr[K], vlr[K], beta[K], w[K], wt[K];
 #pragma unroll
     for (int r = 0; r < K; ++r) {
         double s = 0.0, sl = 0.0;
@@ -105,25 +190,80 @@ template <int K> HRW_HD void weno_cell_exact(const double *x, double eps, const 
         vlr[r] = sl;
     }
     beta_exact<K>(x, beta);
-#pragma unroll
-    for (int r = 0; r < K; ++r) {
-        double q = eps + beta[r];
-        q = q * q;
-        alfa[r] = Tab<K>::d[r] / q;
-        alfat[r] = Tab<K>::d[K - 1 - r] / q;
-    }
-    double sa = 0.0, sat = 0.0;
-#pragma unroll
-    for (int r = 0; r < K; ++r) sa = sa + alfa[r];
-#pragma unroll
-    for (int r = 0; r < K; ++r) sat = sat + alfat[r];
+    weights_exact<K>(beta, eps, w, wt);
     double a = 0.0, b = 0.0;
 #pragma unroll
-    for (int r = 0; r < K; ++r) a = a + (alfa[r] / sa) * vrr[r];
+    for (int r = 0; r < K; ++r) a = a + w[r] * vrr[r];
 #pragma unroll
-    for (int r = 0; r < K; ++r) b = b + (alfat[r] / sat) * vlr[r];
+    for (int r = 0; r < K; ++r) b = b + wt[r] * vlr[r];
     vr = a;
     vl = b;
+}
+
+// Pieces of the triple (a, b, c) = (v_m, v_m+1, v_m+2) that the K = 3 reconstructions of cells
+// m, m+1 and m+2 draw on, in either arithmetic form: the smoothness indicators beta_0(m),
+// beta_1(m+1), beta_2(m+2) and the four candidates c(:,r).T, r = -1..2 (vlr0(m), vrr0(m) =
+// vlr1(m+1), vrr1(m+1) = vlr2(m+2), vrr2(m+2)).  FAST keeps 12 beta and 6 c.T.
+struct Tri3 {
+    double bA, bB, bC;
+    double Pm, P0, P1, P2;
+};
+
+// EXACT: each piece is what beta_exact and weno_cell_exact form for those cells, operation for
+// operation (a product by 2, 4 or 1/4 is exact, so fusing it with the sum it enters changes
+// nothing); formed once and used by three cells.
+HRW_HD Tri3 tri3_exact(double a, double b, double c)
+{
+    Tri3 t;
+    const double D = fma_(-2.0, b, a) + c;
+    const double dd = 13.0 / 12 * (D * D);
+    const double b0 = fma_(-4.0, b, 3 * a) + c;
+    const double b1 = a - c;
+    const double b2 = fma_(-4.0, b, a) + 3 * c;
+    t.bA = fma_(0.25, b0 * b0, dd);
+    t.bB = fma_(0.25, b1 * b1, dd);
+    t.bC = fma_(0.25, b2 * b2, dd);
+    auto cand = [&](const double *q) { return (fma_(q[0], a, 0.0) + q[1] * b) + q[2] * c; };
+    t.Pm = cand(Tab<3>::c[0]);
+    t.P0 = cand(Tab<3>::c[1]);
+    t.P1 = cand(Tab<3>::c[2]);
+    t.P2 = cand(Tab<3>::c[3]);
+    return t;
+}
+// One reconstruction from T(i-2), T(i-1), T(i): weno_cell_exact<3> from the shared pieces.
+HRW_HD void recon3_exact(double eps, const Tri3 &t2, const Tri3 &t1, const Tri3 &t0, double &vl,
+                         double &vr)
+{
+    const double beta[3] = {t0.bA, t1.bB, t2.bC};
+    double w[3], wt[3];
+    weights_exact<3>(beta, eps, w, wt);
+    vr = (fma_(w[0], t0.P0, 0.0) + w[1] * t1.P1) + w[2] * t2.P2;
+    vl = (fma_(wt[0], t0.Pm, 0.0) + wt[1] * t1.P0) + wt[2] * t2.P1;
+}
+
+// The same of a pair (a, b) = (v_m, v_m+1) for K = 2: beta_0(m) = beta_1(m+1), and the
+// candidates S = vrr0(m) = vlr1(m+1), Rr = vrr1(m+1), Lr = vlr0(m) (FAST keeps twice those).
+struct Pair2 {
+    double B, S, Rr, Lr;
+};
+HRW_HD Pair2 pair2_exact(double a, double b)
+{
+    Pair2 p;
+    const double d = b - a;
+    p.B = d * d;
+    auto cand = [&](const double *q) { return fma_(q[0], a, 0.0) + q[1] * b; };
+    p.Lr = cand(Tab<2>::c[0]);
+    p.S = cand(Tab<2>::c[1]);
+    p.Rr = cand(Tab<2>::c[2]);
+    return p;
+}
+HRW_HD void recon2_exact(double eps, const Pair2 &p1, const Pair2 &p0, double &vl, double &vr)
+{
+    const double beta[2] = {p0.B, p1.B};
+    double w[2], wt[2];
+    weights_exact<2>(beta, eps, w, wt);
+    vr = fma_(w[0], p0.S, 0.0) + w[1] * p1.Rr;
+    vl = fma_(wt[0], p0.Lr, 0.0) + wt[1] * p1.S;
 }
 
 // Fast form of one cell on a uniform grid (see the header comment).

@@ -9,6 +9,7 @@
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
 #include <algorithm>
 #include <climits>
@@ -64,6 +65,8 @@ static int fail(int code, const char *fmt, ...)
     } while (0)
 
 static inline hipStream_t S(hrw_stream_t s) { return reinterpret_cast<hipStream_t>(s); }
+
+constexpr int kMaxDevices = 64;
 
 static bool is_done(double t, double tout, double dt)   // src/hrweno_tvdode.f90:273-284
 {
@@ -829,15 +832,19 @@ static bool exact_linear_grid(double xmin, double rx, long long n)
     return big < std::ldexp(1.0L, 53 + e);
 }
 
+// Edges within 1e8 cell widths of the origin: the FAST kernels' 1/width is one Newton step from
+// 1/rx.
+static bool near_linear_grid(double xmin, double rx, long long n)
+{
+    return std::max(std::fabs(xmin), std::fabs(xmin + rx * (double)n)) <= 1e8 * rx;
+}
+
 static void launch_stage1d(const hrw_problem_s *p, const Stage1DArgs &a, hipStream_t s)
 {
     const bool amax0 = p->alphamax();
-    // the register-blocked kernels take linear grids whose edges stay within 1e8 cell widths
-    // of the origin (their 1/width is one Newton step from 1/rx); a width array, a non-uniform
+    // the register-blocked kernels take linear grids near the origin; a width array, a non-uniform
     // grid's coefficients or a grid far from the origin go to the tile kernel
-    const bool linear_near = !a.cnu && !a.width &&
-                             std::max(std::fabs(a.xmin), std::fabs(a.xmin + a.rx * (double)a.n)) <=
-                                 1e8 * a.rx;
+    const bool linear_near = !a.cnu && !a.width && near_linear_grid(a.xmin, a.rx, a.n);
     if (p->arith == HRW_ARITH_FAST && p->variant != 1 && linear_near &&
         a.n < (1LL << 31) - (1LL << 20) &&
         aligned16(a.us) && aligned16(a.u0) && aligned16(a.uo) && aligned16(a.uo4) &&
@@ -1128,6 +1135,13 @@ struct hrw_ode_s {
     GenScratch gen;
     bool check_finite = true;              // integrate ends with a scan of u for NaN/Inf
     unsigned long long *d_bad = nullptr;   // the scan's result word
+    // whole-integration kernel: its exchange words (kResWords, behind the slots), the next exchange
+    // number, whether words and result word are clear, whether it ran in this call and its result's
+    // scan, the polls of a wait (about 0.2 s; HRW_RESIDENT_POLLS at creation sets them for tests)
+    unsigned long long *res_words = nullptr, res_bad = 0;
+    unsigned res_tag = 0;
+    bool res_clear = false, res_ran = false;
+    int res_polls = 1 << 18;
     ~hrw_ode_s();
 };
 // Drop the recording; keep_storage: its blocks go to the pool for the next recording.
@@ -1174,7 +1188,11 @@ static int ode_alloc(hrw_ode_s *o)
         for (auto &b : o->ring_u) CALL(dalloc(&b, o->neq));
         for (auto &b : o->ring_L) CALL(dalloc(&b, o->neq));
     }
-    CALL(dalloc(&o->slots, (size_t)3 * kNSlot * kSlotStride));
+    // (the exchange words of a line of several blocks, behind the slots)
+    const bool exchange = o->p && o->method == METHOD_RK && o->p->kind == PROB_BURGERS1D && o->neq > 10 * kOutLanes;
+    const size_t slots = (size_t)3 * kNSlot * kSlotStride;
+    CALL(dalloc(&o->slots, slots + (exchange ? kResWords : 0)));
+    if (exchange) o->res_words = o->slots + slots;
     CALL(dalloc(&o->d_bad, 1));
     return HRW_OK;
 }
@@ -1202,6 +1220,7 @@ static int ode_new(int method, int order, hrw_problem_s *p, hrw_integrand_fn fu,
         return rc;
     }
     o->istate = 1;   // :93, :199
+    if (const char *e = std::getenv("HRW_RESIDENT_POLLS")) o->res_polls = std::atoi(e);
     *out = o;
     return HRW_OK;
 }
@@ -1316,6 +1335,155 @@ static int rk_step(hrw_ode_s *o, int &seq, double t, double dt, double *u, doubl
     return HRW_OK;
 }
 
+// The steps the loop control takes from t to tout (strict is_done, t by repeated addition); t ends
+// where the loop leaves it.
+static int64_t count_steps(double &t, double tout, double dt)
+{
+    int64_t n = 0;
+    do {
+        t = t + dt;
+        ++n;
+    } while (!is_done(t, tout, dt));
+    return n;
+}
+
+// The result word of a scan or of the whole-integration kernel, once the stream is done.
+static int ode_read_status(hrw_ode_s *o, unsigned long long *bad)
+{
+    HIP_TRY(hipMemcpyAsync(bad, o->d_bad, sizeof *bad, hipMemcpyDeviceToHost, o->stream));
+    HIP_TRY(hipStreamSynchronize(o->stream));
+    if (*bad) o->res_clear = false;   // cleared before the next whole-integration launch
+    return HRW_OK;
+}
+
+// ---- the whole integration in one launch (resident_kernel) ----
+// How a line of n cells is split: cells per lane r, wavefronts per block, blocks.  Measured on 40
+// RK3 steps, us per stage against one launch per stage (FAST Lax-Friedrichs with alpha = max|u|):
+// 300 cells 1.0 / 4.9, 1000 1.6 / 5.2, 16,000 2.2 / 5.2, 64,000 2.4 / 5.3, 250,000 2.9 / 5.6,
+// 950,000 4.4 / 8.0; EXACT 8,000 2.3 / 8.0, 250,000 3.3 / 8.3, 950,000 6.9 / 14.  One block (no
+// exchange) as long as it beats the exchange of several; then about 7 wavefronts of one cell per
+// lane per block, which hide each other's latency; more blocks cost alpha's exchange more (64:
+// 1.6 us, 128: 1.7, 256: 2.3), so with it and the FAST form, whose cells are cheap, two cells per
+// lane come in earlier.  False: the line does not fit.
+static bool resident_split(long long n, bool exact, bool amax, bool nonuniform, ResPlan *pl)
+{
+    const int most_waves = kResThreads / 64;
+    auto one = [&](int r) {
+        pl->r = r;
+        pl->blocks = 1;
+        pl->waves = (int)((n + kOutLanes * r - 1) / (kOutLanes * r));
+        return pl->waves <= most_waves;
+    };
+    if (n <= 10 * kOutLanes) return one(1);
+    if (!exact && !nonuniform && n <= (amax ? 12 : 9) * 2 * kOutLanes) return one(2);
+    // blocks of `waves` wavefronts, at most `blocks` of them; or, with `blocks` of them, as many
+    // wavefronts as it takes, at most `waves`
+    auto several = [&](int r, int waves, int blocks) {
+        const long long per = (long long)waves * kOutLanes * r, nb = (n + per - 1) / per;
+        if (nb > blocks) return false;
+        const long long m = (n + nb - 1) / nb;   // cells per block
+        pl->r = r;
+        pl->blocks = (int)((n + m - 1) / m);
+        pl->waves = (int)((m + kOutLanes * r - 1) / (kOutLanes * r));
+        return n - m * (pl->blocks - 1) >= kResHalo;
+    };
+    const int cap = most_waves - (amax ? 1 : 0);
+    auto widen = [&](int r, int waves) {   // all blocks, `waves` wavefronts at most
+        const long long w = (n + (long long)kResMaxBlocks * kOutLanes * r - 1) / ((long long)kResMaxBlocks * kOutLanes * r);
+        return w <= waves && several(r, (int)w, kResMaxBlocks);
+    };
+    if (nonuniform) return several(1, 7, kResMaxBlocks) || widen(1, cap);
+    if (amax && !exact)
+        return several(1, 7, 96) || several(2, 7, 96) || several(2, 12, 160) || widen(2, cap) || widen(4, cap);
+    return several(1, 7, kResMaxBlocks) || widen(1, exact ? 12 : cap) || widen(2, cap) || widen(4, cap);
+}
+
+// Whether nsteps steps of o take it, and how.  Left to the launches per stage: problems tuned to a
+// kernel, cell widths without their coefficients and FAST lines far from the origin (the tile
+// kernel's arithmetic), and calls under stream capture.
+static bool resident_plan(const hrw_ode_s *o, int64_t nsteps, ResPlan *pl)
+{
+    const hrw_problem_s *p = o->p;
+    if (p->kind != PROB_BURGERS1D || p->variant != 0 || p->cells_per_lane != 0) return false;
+    const bool exact = p->arith != HRW_ARITH_FAST;
+    if (!p->d_cnu && (p->d_width || (!exact && !near_linear_grid(p->xmin, p->rx, p->neq)))) return false;
+    if (p->neq < 8 || !resident_split(p->neq, exact, p->alphamax(), p->d_cnu != nullptr, pl)) return false;
+    // (a launch's first stage must not be its last: blocks read each other's initial cells)
+    if (pl->blocks > device_cus() || (pl->blocks > 1 && !o->res_words) || nsteps * o->order < 2 || nsteps >= (1 << 26)) return false;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(o->stream, &cs) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return cs == hipStreamCaptureStatusNone;
+}
+
+// Held while a launch whose blocks wait for each other is in flight on the device: two of them at
+// once could each hold CUs the other's missing blocks need.  A call that finds it taken (another
+// thread is in such an integrate) uses one launch per stage.
+static std::mutex g_resident_mu[kMaxDevices];
+
+// nsteps steps of o on u by resident_kernel.  *ran = false, and u as it was, when the device is
+// taken or refuses the launch, or when the blocks waited for each other in vain (another process's
+// kernels kept some of them off the device).
+static int rk_resident(hrw_ode_s *o, const ResPlan &pl, double *u, int64_t nsteps, double dt, bool *ran)
+{
+    *ran = false;
+    std::unique_lock<std::mutex> alone;
+    if (pl.blocks > 1) {
+        int dev = 0;
+        HIP_TRY(hipGetDevice(&dev));
+        if (dev < 0 || dev >= kMaxDevices) return HRW_OK;
+        alone = std::unique_lock<std::mutex>(g_resident_mu[dev], std::try_to_lock);
+        if (!alone.owns_lock()) return HRW_OK;
+    }
+    const hrw_problem_s *p = o->p;
+    ResArgs a{};
+    a.u = u;
+    a.saved = o->ui;
+    a.n = p->neq;
+    a.M = (int)((p->neq + pl.blocks - 1) / pl.blocks);
+    a.order = o->order;
+    a.nsteps = (int)nsteps;
+    a.periodic = p->bc == HRW_BC_PERIODIC;
+    a.amax = p->alphamax();
+    static const int stage_id[3][3] = {{RK1, RK1, RK1}, {RK2_1, RK2_2, RK2_2}, {RK3_1, RK3_2, RK3_3}};
+    for (int i = 0; i < 3; ++i) a.coef[i] = res_coef(stage_id[o->order - 1][i], dt);
+    a.eps = p->eps;
+    a.alpha = p->alpha;
+    a.xmin = p->xmin;
+    a.rx = p->rx;
+    a.width = p->d_width;
+    a.cnu = p->d_cnu;
+    a.words = o->res_words;
+    a.status = o->d_bad;
+    a.polls = o->res_polls;
+    const unsigned used = (unsigned)a.nsteps * (unsigned)o->order;
+    if (!o->res_clear || o->res_tag > 0xffffffffu - used) {
+        if (o->res_words)
+            fill_u64_kernel<<<grid_for((long long)kResWords, 256, 64), 256, 0, o->stream>>>(o->res_words, kResWords);
+        fill_u64_kernel<<<1, 64, 0, o->stream>>>(o->d_bad, 1);
+        o->res_tag = kResFirstTag;
+        o->res_clear = true;
+    }
+    a.tag = o->res_tag;
+    o->res_tag += used;
+    const bool fast = p->arith == HRW_ARITH_FAST;
+    const hipError_t e = p->k == 1   ? launch_resident_k1(p->numflux, fast, pl, a, o->stream)
+                         : p->k == 2 ? launch_resident_k2(p->numflux, fast, pl, a, o->stream)
+                                     : launch_resident_k3(p->numflux, fast, pl, a, o->stream);
+    if (e != hipSuccess) return HRW_OK;   // (not launched)
+    unsigned long long bad = 0;
+    CALL(ode_read_status(o, &bad));
+    if (bad & RES_TIMEOUT) {
+        HIP_TRY(hipMemcpyAsync(u, o->ui, o->neq * sizeof(double), hipMemcpyDeviceToDevice, o->stream));
+        return HRW_OK;
+    }
+    *ran = o->res_ran = true;
+    o->res_bad = bad;
+    return HRW_OK;
+}
+
 static int rk_integrate_taped(hrw_ode_s *o, double *u, double *t, double tout, double dt,
                               int itask);
 static int rk_integrate(hrw_ode_s *o, double *u, double *t, double tout, double dt, int itask)
@@ -1323,6 +1491,19 @@ static int rk_integrate(hrw_ode_s *o, double *u, double *t, double tout, double 
     if (o->istate < 1) return HRW_OK;                  // :126
     if (is_done(*t, tout, dt)) return HRW_OK;          // :127
     if (o->tape_every > 0) return rk_integrate_taped(o, u, t, tout, dt, itask);
+    if (o->p && o->check_finite && itask == 1) {
+        double t1 = *t;
+        const int64_t nsteps = count_steps(t1, tout, dt);
+        ResPlan pl;
+        bool ran = false;
+        if (resident_plan(o, nsteps, &pl)) CALL(rk_resident(o, pl, u, nsteps, dt, &ran));
+        if (ran) {
+            *t = t1;
+            o->fevals += o->order * (int)nsteps;
+            if (o->istate == 1) o->istate = 2;         // :176
+            return HRW_OK;
+        }
+    }
     int seq = 0;
     if (o->p) CALL(seed_alpha(o->p, o->slots, u, o->stream));
     double *cur = u, *other = o->ui2;
@@ -1527,12 +1708,13 @@ static __global__ __launch_bounds__(kBlock) void nonfinite_kernel(const double *
 
 static int ode_check_finite(hrw_ode_s *o, const double *u)
 {
-    fill_u64_kernel<<<1, 64, 0, o->stream>>>(o->d_bad, 1);
-    nonfinite_kernel<<<grid_for(o->neq, kBlock * 8, 4096), kBlock, 0, o->stream>>>(u, o->neq, o->d_bad);
-    LAUNCH_CHECK();
-    unsigned long long bad = 0;
-    HIP_TRY(hipMemcpyAsync(&bad, o->d_bad, sizeof bad, hipMemcpyDeviceToHost, o->stream));
-    HIP_TRY(hipStreamSynchronize(o->stream));
+    unsigned long long bad = o->res_bad;
+    if (!o->res_ran) {   // (else the integration has scanned its result)
+        fill_u64_kernel<<<1, 64, 0, o->stream>>>(o->d_bad, 1);
+        nonfinite_kernel<<<grid_for(o->neq, kBlock * 8, 4096), kBlock, 0, o->stream>>>(u, o->neq, o->d_bad);
+        LAUNCH_CHECK();
+        CALL(ode_read_status(o, &bad));
+    }
     if (bad) return fail(HRW_ERR_STATE, "non-finite state: u holds NaN or Inf after integrate");
     return HRW_OK;
 }
@@ -1547,6 +1729,7 @@ extern "C" int hrw_ode_integrate(hrw_ode_t ode, double *u, double *t, double tou
     if (!(dt != 0.0) || !std::isfinite(dt) || !std::isfinite(*t) || std::isnan(tout))
         return fail(HRW_ERR_ARG, "Invalid input 'dt', 't' or 'tout': dt must be finite and nonzero");
     const double t_in = *t;
+    ode->res_ran = false;
     int rc = ode->method == METHOD_MS ? ms_integrate(ode, u, t, tout, dt)
                                       : rk_integrate(ode, u, t, tout, dt, itask);
     if (rc == HRW_OK && ode->check_finite && *t != t_in) rc = ode_check_finite(ode, u);
@@ -1671,7 +1854,6 @@ constexpr long long kNoAllocMaxCells = 1LL << 20;
 constexpr long long kNoAllocSlotWords = 3LL * kNSlot * kSlotStride;
 static __device__ __align__(256) double scratch[2 * kNoAllocMaxCells + kNoAllocSlotWords];
 static std::mutex g_scratch_mu;
-constexpr int kMaxDevices = 64;
 static double *g_scratch_ptr[kMaxDevices] = {};
 
 // The scratch of the current device, looked up once per device with that device current.

@@ -1,0 +1,459 @@
+// kernels_resident.hpp -- a whole rktvd integration of one 1D Burgers line in one launch.
+//
+// A line that fits on the chip spends its time, with one launch per stage, on the launches: a
+// stage of 1000 cells takes 5 us of which its arithmetic is a few hundred ns.  Here the state stays
+// in LDS and registers for every step of the call (src/hrweno_tvdode.f90:136-171): block b owns M
+// consecutive cells, its lanes R consecutive cells each, and a stage reads the block's LDS copy of
+// the stage input and writes the other copy.  One block needs nothing else.  Several blocks (at
+// most one per CU, so that all come to be resident) exchange, after each stage, the three cells at
+// each of their ends with their neighbours and the block maxima of |u| (alpha = max|u|) with every
+// block.
+//
+// An exchange takes 1.4 us between neighbours and 1.6 / 1.7 / 2.3 us among 64 / 128 / 256 blocks
+// (each block's words on a cache line of their own; packed, writers and readers of one line queue
+// up: 2.3 / 2.7 / 3.1).  What does not wait for it runs beside it: the reconstruction of a stage
+// needs no alpha, so one wavefront more per block sees to the maxima while the others reconstruct,
+// and only the wavefronts that read a halo wait for the neighbours' cells.
+//
+// The exchange takes no fence.  A double travels as two 64-bit words, each half of it beside the
+// 32-bit number of the exchange; a maximum (a non-negative double) as one word with a bit of the
+// number in place of its sign.  All are stored and loaded with relaxed agent-scope atomics, so a
+// word that carries the expected number carries its data.  Words of exchange e live in buffer
+// e % 4.  A block publishes e + 4 behind the barrier that follows its reads of e + 2; its
+// neighbours (for the maxima, every block) published those behind a barrier that follows their
+// reads of e: no word is overwritten before it is read.  Numbers go on from launch to launch.  A
+// wait is bounded; a wave that runs out of polls sets a status bit and waits no more, so every
+// launch ends.  The blocks have saved the initial state by then, and the caller goes on from it
+// with one launch per stage.
+//
+// Per cell the arithmetic is that of the per-stage kernels, operation for operation
+// (kernels_1d_fast.hpp for the FAST form, weno_math.hpp for EXACT), so the results are theirs bit
+// for bit whatever the split into blocks and lanes.
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include "kernels_1d_fast.hpp"
+
+namespace hrw {
+
+constexpr int kResHalo = 3;        // cells exchanged at each end (a face needs K = 3 each side)
+constexpr int kResMaxBlocks = 256;
+constexpr int kResLine = 16;       // words per block and exchange: 12 of edge cells, 1 maximum
+constexpr int kResThreads = 1024;
+constexpr size_t kResWords = 4 * (size_t)kResMaxBlocks * kResLine;   // one object's exchange words
+constexpr unsigned kResFirstTag = 4;   // the number after which cleared words read as not arrived
+
+enum { RES_NONFINITE = 1, RES_TIMEOUT = 2 };   // status bits
+
+// A stage's combination of u0 (the state at the start of the step), its input us and L = rhs(us):
+// FAST  fma(C, L, fma(A, us - u0, u0))                        (kernels_1d_fast.hpp)
+// EXACT ((p u0 + s us) + g L) q, or the division by 3         (stage_update; p, s, q exact factors)
+// In a first stage u0 is us itself (A = 1; p = 0, s = 1).
+struct ResCoef {
+    double A, C, p, s, g, q;
+    int div3;
+};
+inline ResCoef res_coef(int stage, double h)
+{
+    const StageCoef c = stage_coef(stage, h);
+    const double post = c.div3 ? 1.0 / 3.0 : c.post;
+    ResCoef r{c.A * post, c.C * post, 0.0, 1.0, h, 1.0, 0};
+    if (stage == RK2_2) r.p = 1.0, r.q = 0.5;
+    if (stage == RK3_2) r.p = 3.0, r.q = 0.25;
+    if (stage == RK3_3) r.p = 1.0, r.s = 2.0, r.g = 2.0 * h, r.div3 = 1;
+    return r;
+}
+
+struct ResArgs {
+    double *u;                     // state, read at the start and written at the end
+    double *saved;                 // several blocks: receives the initial state
+    long long n;
+    int M;                         // cells per block (the last block: what is left, >= kResHalo)
+    int order, nsteps, periodic, amax;
+    double eps, alpha, xmin, rx;
+    ResCoef coef[3];               // of the step's stages
+    const double *width, *cnu;     // non-uniform grid, else nullptr
+    unsigned long long *words;     // kResWords words
+    unsigned long long *status;
+    unsigned tag;                  // number of the first exchange (>= kResFirstTag)
+    int polls;
+};
+
+__device__ __forceinline__ unsigned long long word_load(const unsigned long long *p)
+{
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void word_store(unsigned long long *p, unsigned long long w)
+{
+    __hip_atomic_store(p, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// The words of exchange `tag`; block b's line starts at word b*kResLine.
+__device__ __forceinline__ unsigned long long *res_words(const ResArgs &a, unsigned tag)
+{
+    return a.words + (tag & 3) * (kResMaxBlocks * kResLine);
+}
+__device__ __forceinline__ unsigned long long tag_phase(unsigned tag)   // in a maximum's sign bit
+{
+    return (unsigned long long)((tag >> 2) & 1) << 63;
+}
+
+// v_max_f64 (a NaN gives the other operand), and the maximum over each row of 16 lanes into its
+// lane 15 (non-negative values; a lane with no source keeps its own).
+__device__ __forceinline__ double max_f64(double x, double y)
+{
+    double r;
+    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(x), "v"(y));
+    return r;
+}
+template <int CTRL> __device__ __forceinline__ double dpp_own(double v)
+{
+    return __builtin_bit_cast(double, dpp_u64<CTRL, 0xF>(__builtin_bit_cast(unsigned long long, v)));
+}
+__device__ __forceinline__ double row_max(double v)
+{
+    v = max_f64(v, dpp_own<0x111>(v));
+    v = max_f64(v, dpp_own<0x112>(v));
+    v = max_f64(v, dpp_own<0x114>(v));
+    return max_f64(v, dpp_own<0x118>(v));
+}
+
+// *p = max(*p, v) in LDS for the lanes at work, completed (v non-negative, compared as bits; the
+// compiler would walk the lanes one by one first).
+__device__ __forceinline__ void lds_max(unsigned long long *p, double v)
+{
+    const unsigned at = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned long long *)p;
+    asm volatile("ds_max_u64 %0, %1\n\ts_waitcnt lgkmcnt(0)" ::"v"(at), "v"(v) : "memory");
+}
+
+// Face values vl, vr of a lane's R cells from their window v (cells -(K-1) .. R+K-2).  FAST: the
+// scaled forms of chunk_stage; CNU: each cell's own coefficients ci.
+template <int K, bool FAST, bool CNU, int R>
+__device__ __forceinline__ void lane_recon(const double *v, double eps, const double *ci, double *vl,
+                                           double *vr)
+{
+    if constexpr (CNU) {
+#pragma unroll
+        for (int t = 0; t < R; ++t) weno_cell_exact<K>(v + t, eps, ci + t * (K * (K + 1)), vl[t], vr[t]);
+    } else if constexpr (K == 3) {
+        Tri3 t2 = FAST ? tri3(v[0], v[1], v[2]) : tri3_exact(v[0], v[1], v[2]);
+        Tri3 t1 = FAST ? tri3(v[1], v[2], v[3]) : tri3_exact(v[1], v[2], v[3]);
+#pragma unroll
+        for (int t = 0; t < R; ++t) {
+            const Tri3 t0 = FAST ? tri3(v[t + 2], v[t + 3], v[t + 4]) : tri3_exact(v[t + 2], v[t + 3], v[t + 4]);
+            if constexpr (FAST) recon3<true, true>(12.0 * eps, t2, t1, t0, vl[t], vr[t]);
+            else recon3_exact(eps, t2, t1, t0, vl[t], vr[t]);
+            t2 = t1;
+            t1 = t0;
+        }
+    } else if constexpr (K == 2) {
+        Pair2 p1 = FAST ? pair2(v[0], v[1]) : pair2_exact(v[0], v[1]);
+#pragma unroll
+        for (int t = 0; t < R; ++t) {
+            const Pair2 p0 = FAST ? pair2(v[t + 1], v[t + 2]) : pair2_exact(v[t + 1], v[t + 2]);
+            if constexpr (FAST) recon2<true>(eps, p1, p0, vl[t], vr[t]);
+            else recon2_exact(eps, p1, p0, vl[t], vr[t]);
+            p1 = p0;
+        }
+    } else {
+#pragma unroll
+        for (int t = 0; t < R; ++t) vl[t] = vr[t] = FAST ? v[t] : 0.0 + v[t];
+    }
+}
+
+template <int K, int FLUX, bool FAST, bool CNU>
+__device__ __forceinline__ double face_flux(double vm, double vp, double alpha)
+{
+    if constexpr (CNU || !FAST) {
+        return burgers_numflux<FLUX, FAST>(vm, vp, alpha);
+    } else {
+        constexpr double S = K == 3 ? 6.0 : (K == 2 ? 2.0 : 1.0);
+        const double cq = 0.25 / (S * S), ca = (-0.5 / S) * alpha, cg = 0.5 / (S * S);
+        if constexpr (FLUX == GODUNOV) return godunov((vm * vm) * cg, (vp * vp) * cg, vm, vp);
+        else return fma_(cq, fma_(vm, vm, vp * vp), ca * (vp - vm));
+    }
+}
+
+// The extra wavefront's part of an exchange: publishes the block's maximum and waits for every
+// block's; false when the polls ran out.
+__device__ __forceinline__ bool gather_max(const ResArgs &a, unsigned tag, int polls, unsigned long long mine,
+                                           double *line_max)
+{
+    constexpr int N = kResMaxBlocks / 64;
+    const int lane = threadIdx.x & 63, B = gridDim.x;
+    const unsigned long long ph = tag_phase(tag);
+    unsigned long long *words = res_words(a, tag);
+    if (lane == 0) word_store(words + blockIdx.x * kResLine + 12, mine | ph);
+    for (int q = 0; q < polls; ++q) {
+        unsigned long long w[N], miss = 0;
+#pragma unroll
+        for (int i = 0; i < N; ++i)   // (lanes past the last block read its word)
+            w[i] = i == 0 || 64 * i < B ? word_load(words + min(64 * i + lane, B - 1) * kResLine + 12) : ph;
+        double x = 0.0;
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            w[i] ^= ph;
+            miss |= w[i];
+            x = max_f64(x, __builtin_bit_cast(double, w[i]));
+        }
+        if (!__any((long long)miss < 0)) {
+            *line_max = __builtin_bit_cast(double, wave_umax(__builtin_bit_cast(unsigned long long, x)));
+            return true;
+        }
+    }
+    return false;
+}
+
+// A wavefront that reads a halo waits for the neighbours' end cells and puts them around buf: lanes
+// 0..5 the left neighbour's last three cells, lanes 6..11 the right one's first three.  An end of
+// the line repeats its end cell (src/hrweno_weno.f90:171-173).  False when the polls ran out.
+__device__ __forceinline__ bool gather_halo(const ResArgs &a, unsigned tag, int polls, double *buf, int m, bool lo,
+                                            bool hi)
+{
+    const int lane = threadIdx.x & 63, b = blockIdx.x, B = gridDim.x;
+    const int left = b > 0 ? b - 1 : (a.periodic ? B - 1 : -1);
+    const int right = b + 1 < B ? b + 1 : (a.periodic ? 0 : -1);
+    const bool use = lane < 12 && (lane < 6 ? lo : hi);
+    const int nb = lane < 6 ? left : right;
+    const bool wait = use && nb >= 0;
+    const unsigned long long *p = res_words(a, tag) + (wait ? nb * kResLine + (lane < 6 ? lane + 6 : lane - 6) : 0);
+    unsigned long long w = 0;
+    bool ok = false;
+    for (int q = 0; q < polls; ++q) {
+        if (wait) w = word_load(p);
+        if (__all(!wait || (unsigned)w == tag)) {
+            ok = true;
+            break;
+        }
+    }
+    const unsigned half = (unsigned)(w >> 32);   // words 2e and 2e + 1: the halves of cell e
+    const unsigned other = (unsigned)__builtin_amdgcn_update_dpp(0, (int)half, 0xB1, 0xF, 0xF, true);   // lane ^ 1
+    if (use && !(lane & 1)) {
+        const int e = lane >> 1;
+        double x = __builtin_bit_cast(double, ((unsigned long long)other << 32) | half);
+        if (nb < 0) x = buf[lane < 6 ? 0 : m - 1];
+        buf[e < 3 ? e - 3 : m + e - 3] = x;
+    }
+    return ok;
+}
+
+// LDS: two copies of the block's cells with kResPad cells on each side (the three halo cells, and
+// room for what the wave-edge lanes read beyond them, which feeds no cell), and after each copy one
+// cell more that takes the writes of cells that are not the block's.
+template <int R> constexpr int kResPad = R + 4;
+template <int R> __host__ __device__ constexpr int res_copy(int waves) { return waves * kOutLanes * R + 2 * kResPad<R> + 2; }
+template <int R> constexpr size_t res_lds_bytes(int waves) { return 2 * (size_t)res_copy<R>(waves) * sizeof(double); }
+
+// waves: the wavefronts that own cells; with ONE false and alpha = max|u| the block has one more.
+template <int K, int FLUX, bool FAST, bool CNU, int R, bool ONE>
+__global__ __launch_bounds__(kResThreads) void resident_kernel(ResArgs a, int waves)
+{
+    constexpr int H = K - 1, PAD = kResPad<R>;
+    extern __shared__ double lds[];
+    __shared__ unsigned long long s_mx[4];   // block maxima of |u|, in turn
+    __shared__ double s_alpha;
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int cap = waves * kOutLanes * R, copy = res_copy<R>(waves);
+    double *cur = lds + PAD, *nxt = cur + copy;
+    const long long base = (long long)blockIdx.x * a.M;
+    const int m = (int)min((long long)a.M, a.n - base);
+    const int w0 = wv * kOutLanes * R, c0 = w0 + (lane - 1) * R;   // the lane's first cell in the block
+    const bool owned = lane >= 1 && lane <= kOutLanes;
+    const bool amax = FLUX == LF && a.amax != 0, per = a.periodic != 0;
+    const bool comm = !ONE && wv >= waves;   // the extra wavefront
+
+    // the initial state and its halo (other cells of the copies: zero)
+    for (int j = tid; j < 2 * copy; j += blockDim.x) lds[j] = 0.0;
+    if (tid < 4) s_mx[tid] = 0ull;
+    __syncthreads();
+    double x0 = 0.0;
+    for (int j = tid - kResHalo; j < m + kResHalo; j += blockDim.x) {
+        const double x = a.u[cell_index(base + j, a.n, per)];
+        cur[j] = x;
+        if (j >= 0 && j < m) {
+            x0 = max_f64(x0, fabs(x));
+            if constexpr (!ONE) a.saved[base + j] = x;
+        }
+    }
+    if (amax) {
+        x0 = row_max(x0);
+        if ((lane & 15) == 15) lds_max(&s_mx[0], x0);
+    }
+
+    // what does not change with the steps: cell widths (FAST: their reciprocals), the non-uniform
+    // grid's coefficients, which cells are this lane's, where it writes them (others: `spare`) and
+    // (the only block of a line) their images past its ends
+    const int spare = cap + PAD;
+    double wd[R];
+    [[maybe_unused]] double ci[CNU ? R * K * (K + 1) : 1];
+    bool mine[R];
+    int at[R];
+    [[maybe_unused]] int image[R];
+    const double inv_rx = rcp_nr(a.rx);
+#pragma unroll
+    for (int t = 0; t < R; ++t) {
+        const int j = c0 + t;
+        mine[t] = owned && j < m;
+        at[t] = mine[t] ? j : spare;
+        image[t] = !mine[t] ? spare : (per ? (j < kResHalo ? m + j : (j >= m - kResHalo ? j - m : spare)) : spare);
+        const long long g = base + j, gc = g < 0 ? 0 : (g < a.n ? g : a.n - 1);
+        if constexpr (CNU) {
+            wd[t] = a.width[gc];
+#pragma unroll
+            for (int q = 0; q < K * (K + 1); ++q) ci[t * K * (K + 1) + q] = a.cnu[gc * (K * (K + 1)) + q];
+        } else {
+            const double w = linear_edge(a.xmin, a.rx, gc + 1) - linear_edge(a.xmin, a.rx, gc);
+            wd[t] = FAST ? fma_(inv_rx, fma_(-w, inv_rx, 1.0), inv_rx) : w;
+        }
+    }
+    // zero-gradient ends (example1:103-104): the lane that holds cell 0, and cell n-1
+    const long long gl = a.n - 1 - base - c0;
+    const bool first = !per && base + c0 == 0 && owned, last = !per && owned && gl >= 0 && gl < R;
+    // this wavefront owns end cells of the block / reads halo cells / holds an end of the line
+    const bool own_end = (wv == 0 || w0 + kOutLanes * R > m - kResHalo) && w0 < m;
+    const bool read_lo = wv == 0, read_hi = w0 + 63 * R + H > m;
+    const bool line_end = __any(first || last);
+
+    const int stages = a.order * a.nsteps;
+    double u0[R];
+    double alpha = a.alpha;
+    bool bad = false;
+    int polls = a.polls, st = 0;   // stage of the step
+    for (int q = 0;; ++q) {
+        const unsigned tag = a.tag + (unsigned)q;
+        __syncthreads();   // cur and its maximum are complete
+        if (amax && tid == 0) s_mx[(q + 2) & 3] = 0ull;
+        double v[R + 2 * H], vl[R], vr[R], vr_left = 0.0, vl_right = 0.0;
+        if (!comm) {
+            if constexpr (!ONE) {
+                if (q > 0 && (read_lo || read_hi)) {
+                    // (these wavefronts first: theirs is the longer way)
+                    __builtin_amdgcn_s_setprio(2);
+                    if (!gather_halo(a, tag, polls, cur, m, read_lo, read_hi)) {
+                        polls = 1;
+                        if (lane == 0) atomicOr(a.status, (unsigned long long)RES_TIMEOUT);
+                    }
+                    __builtin_amdgcn_wave_barrier();
+                }
+            }
+#pragma unroll
+            for (int t = 0; t < R + 2 * H; ++t) v[t] = cur[c0 - H + t];
+            if (ONE && amax) alpha = __builtin_bit_cast(double, s_mx[q & 3]);
+            lane_recon<K, FAST, CNU, R>(v, a.eps, ci, vl, vr);
+            vr_left = shfl_up1(vr[R - 1]);
+            vl_right = shfl_down1(vl[0]);
+        } else {
+            double x = 0.0;
+            if (!gather_max(a, tag, polls, s_mx[q & 3], &x)) {
+                polls = 1;
+                if (lane == 0) atomicOr(a.status, (unsigned long long)RES_TIMEOUT);
+            }
+            if (lane == 0) s_alpha = x;
+        }
+        if (!ONE && amax) {
+            __syncthreads();   // the line's maximum is known
+            alpha = s_alpha;
+        }
+        if (comm) {
+            if (q + 1 == stages) break;
+            continue;
+        }
+        double f[R + 1], un[R];
+        f[0] = face_flux<K, FLUX, FAST, CNU>(vr_left, vl[0], alpha);
+#pragma unroll
+        for (int t = 1; t < R; ++t) f[t] = face_flux<K, FLUX, FAST, CNU>(vr[t - 1], vl[t], alpha);
+        f[R] = face_flux<K, FLUX, FAST, CNU>(vr[R - 1], vl_right, alpha);
+        if (line_end) {
+            if (first) f[0] = f[1];
+            if (last) {
+#pragma unroll
+                for (int t = 0; t < R; ++t)
+                    if (t == gl) f[t + 1] = f[t];
+            }
+        }
+        const ResCoef &co = a.coef[st];
+        if (st == 0) {
+#pragma unroll
+            for (int t = 0; t < R; ++t) u0[t] = v[H + t];
+        }
+#pragma unroll
+        for (int t = 0; t < R; ++t) {
+            const double us = v[H + t];
+            if constexpr (!CNU && FAST) {
+                const double L = (f[t] - f[t + 1]) * wd[t];
+                un[t] = fma_(co.C, L, fma_(co.A, us - u0[t], u0[t]));
+            } else {
+                const double L = (f[t] - f[t + 1]) / wd[t];
+                if constexpr (FAST) un[t] = fma_(co.g, L, fma_(co.p, u0[t], co.s * us));
+                else un[t] = (co.p * u0[t] + co.s * us) + co.g * L;
+            }
+        }
+        if constexpr (CNU || !FAST) {
+            if (co.div3) {
+#pragma unroll
+                for (int t = 0; t < R; ++t) un[t] = FAST ? div3_fast(un[t]) : un[t] / 3;
+            } else {
+#pragma unroll
+                for (int t = 0; t < R; ++t) un[t] = un[t] * co.q;
+            }
+        }
+        if (q + 1 == stages) {
+#pragma unroll
+            for (int t = 0; t < R; ++t)
+                if (mine[t]) {
+                    a.u[base + c0 + t] = un[t];
+                    bad |= !isfinite(un[t]);
+                }
+            break;
+        }
+#pragma unroll
+        for (int t = 0; t < R; ++t) nxt[at[t]] = un[t];
+        if (own_end) {
+            // the next stage's halos: the only block's own images, or words for the neighbours
+            if constexpr (ONE) {
+                if (per) {
+#pragma unroll
+                    for (int t = 0; t < R; ++t) nxt[image[t]] = un[t];
+                } else if (line_end) {   // (src/hrweno_weno.f90:171-173)
+                    if (first) nxt[-1] = nxt[-2] = nxt[-3] = un[0];
+                    if (last) {
+#pragma unroll
+                        for (int t = 0; t < R; ++t)
+                            if (t == gl) nxt[m] = nxt[m + 1] = nxt[m + 2] = un[t];
+                    }
+                }
+            } else {
+                unsigned long long *line = res_words(a, tag + 1) + blockIdx.x * kResLine;
+#pragma unroll
+                for (int t = 0; t < R; ++t) {
+                    const int j = c0 + t;
+                    const unsigned long long bits = __builtin_bit_cast(unsigned long long, un[t]);
+                    const unsigned long long wl = (bits << 32) | (tag + 1);
+                    const unsigned long long wh = (bits & 0xffffffff00000000ull) | (tag + 1);
+                    if (mine[t] && j < kResHalo) {
+                        word_store(line + 2 * j, wl);
+                        word_store(line + 2 * j + 1, wh);
+                    }
+                    if (mine[t] && j >= m - kResHalo) {
+                        word_store(line + 6 + 2 * (j - (m - kResHalo)), wl);
+                        word_store(line + 7 + 2 * (j - (m - kResHalo)), wh);
+                    }
+                }
+                __builtin_amdgcn_s_setprio(0);
+            }
+        }
+        if (amax) {
+            double x = 0.0;
+#pragma unroll
+            for (int t = 0; t < R; ++t) x = max_f64(x, mine[t] ? fabs(un[t]) : 0.0);
+            x = row_max(x);
+            if ((lane & 15) == 15) lds_max(&s_mx[(q + 1) & 3], x);
+        }
+        double *sw = cur;
+        cur = nxt;
+        nxt = sw;
+        if (++st == a.order) st = 0;
+    }
+    if (__any(bad) && lane == 0) atomicOr(a.status, (unsigned long long)RES_NONFINITE);
+}
+
+}  // namespace hrw

@@ -10,6 +10,7 @@
 #include "kernels_adjoint.hpp"
 #include "kernels_adjoint_general.hpp"
 #include "kernels_adjoint_blocked.hpp"
+#include "kernels_resident.hpp"
 
 namespace hrw {
 
@@ -37,6 +38,15 @@ void launch_fast_1d_k2(int flux, bool periodic, bool alphamax, bool constw, int 
                        const Stage1DArgs &a, hipStream_t s);
 void launch_fast_1d_k3(int flux, bool periodic, bool alphamax, bool constw, int form, int r,
                        const Stage1DArgs &a, hipStream_t s);
+// A whole rktvd integration in one launch (kernels_resident.hpp): r cells per lane (1, 2, 4; 1 on
+// a non-uniform grid), `waves` wavefronts per block, `blocks` blocks (at most one per CU; the caller
+// sees to it that no other launch whose blocks wait for each other is in flight on the device).
+struct ResPlan {
+    int r, waves, blocks;
+};
+hipError_t launch_resident_k1(int flux, bool fast, const ResPlan &pl, const ResArgs &a, hipStream_t s);
+hipError_t launch_resident_k2(int flux, bool fast, const ResPlan &pl, const ResArgs &a, hipStream_t s);
+hipError_t launch_resident_k3(int flux, bool fast, const ResPlan &pl, const ResArgs &a, hipStream_t s);
 // LDS-tile 1D stage (EXACT form, and the FAST LDS variant).
 void launch_tile_1d(int k, int flux, bool periodic, bool fast, bool alphamax, const Stage1DArgs &a,
                     hipStream_t s);

@@ -1,0 +1,43 @@
+// launch_resident.hip -- launcher of the whole-integration kernel for one WENO order, HRW_K (the
+// build compiles this file once per K = 1, 2, 3).
+#include "launch.hpp"
+
+#ifndef HRW_K
+#error "compile with -DHRW_K=1, 2 or 3"
+#endif
+
+namespace hrw {
+namespace {
+
+template <int FLUX, bool FAST, bool CNU, int R>
+hipError_t run(const ResPlan &pl, const ResArgs &a, hipStream_t s)
+{
+    const size_t lds = res_lds_bytes<R>(pl.waves);
+    if (pl.blocks == 1)
+        resident_kernel<HRW_K, FLUX, FAST, CNU, R, true><<<1, 64 * pl.waves, lds, s>>>(a, pl.waves);
+    else
+        resident_kernel<HRW_K, FLUX, FAST, CNU, R, false>
+            <<<pl.blocks, 64 * (pl.waves + (a.amax ? 1 : 0)), lds, s>>>(a, pl.waves);
+    return hipGetLastError();
+}
+template <int FLUX, bool FAST>
+hipError_t run_r(const ResPlan &pl, const ResArgs &a, hipStream_t s)
+{
+    if (a.cnu) return run<FLUX, FAST, true, 1>(pl, a, s);
+    if (pl.r == 1) return run<FLUX, FAST, false, 1>(pl, a, s);
+    if (pl.r == 2) return run<FLUX, FAST, false, 2>(pl, a, s);
+    return run<FLUX, FAST, false, 4>(pl, a, s);
+}
+
+}  // namespace
+
+#define HRW_CAT2(a, b) a##b
+#define HRW_CAT(a, b) HRW_CAT2(a, b)
+hipError_t HRW_CAT(launch_resident_k, HRW_K)(int flux, bool fast, const ResPlan &pl, const ResArgs &a,
+                                             hipStream_t s)
+{
+    if (flux == LF) return fast ? run_r<LF, true>(pl, a, s) : run_r<LF, false>(pl, a, s);
+    return fast ? run_r<GODUNOV, true>(pl, a, s) : run_r<GODUNOV, false>(pl, a, s);
+}
+
+}  // namespace hrw

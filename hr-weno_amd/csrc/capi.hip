@@ -1953,6 +1953,15 @@ struct hrw_batch_s {
     hipGraphExec_t graph = nullptr;
     const double *graph_u = nullptr;
     int graph_R = 0, graph_form = 0;
+    // whole-integration kernel: its block table (0 blocks: some line does not fit), cells per lane,
+    // exchange words with the count of started blocks behind them, the next exchange number; used
+    // unless a kernel was chosen (hrw_batch_set_*) or the tuner found one faster
+    ResBlock *d_rblocks = nullptr;
+    long long res_blocks = 0;
+    int res_r = 4;
+    unsigned long long *res_words = nullptr;
+    unsigned res_words_per = 0, res_tag = kResFirstTag, res_started = 0;
+    bool resident = true;
     bool alphamax() const { return numflux == HRW_FLUX_LAX_FRIEDRICHS && alpha < 0; }
     ~hrw_batch_s()
     {
@@ -1960,6 +1969,7 @@ struct hrw_batch_s {
         dfree(d_off); dfree(d_n); dfree(d_k); dfree(d_cline); dfree(d_cstart);
         dfree(d_h); dfree(d_xmin); dfree(d_rx); dfree(ui); dfree(ui2); dfree(slots);
         dfree(line_slots);
+        dfree(d_rblocks); dfree(res_words);
         if (ev_in) (void)hipEventDestroy(ev_in);
         if (ev_out) (void)hipEventDestroy(ev_out);
         if (own_stream && stream) (void)hipStreamDestroy(stream);
@@ -2016,6 +2026,90 @@ static int batch_chunks(hrw_batch_s *b, int R)
     if (b->graph) {
         (void)hipGraphExecDestroy(b->graph);
         b->graph = nullptr;
+    }
+    return HRW_OK;
+}
+
+// Block table of the whole-integration kernel: lines longer than a block first (their blocks
+// exchange, and only they have words), each over equal blocks, then the others, the longest first.
+// Measured, us per RK3 step against one launch per stage: 1024 lines of 256-65536 cells (LF) 163 /
+// 183, the same with the Godunov flux 126 / 183, 475 lines of 454-18274 cells 50 / 73, 256 of
+// 1024-16384 31 / 54, 8 of 30000-65000 13 / 33.  Short lines, which leave the chip half idle, go at
+// two cells per lane (800 lines of 64-2000 cells: 125 us per 8 steps, 140 at four).
+static int batch_resident_blocks(hrw_batch_s *b)
+{
+    const int r = b->res_r = *std::max_element(b->h_n.begin(), b->h_n.end()) <= 2048 ? 2 : 4;
+    const int waves = kBatchResWaves - (b->alphamax() ? 1 : 0);   // (one for the maxima)
+    const long long most = (long long)waves * kOutLanes * r, single = (long long)kBatchResWaves * kOutLanes * r;
+    std::vector<int> lines((size_t)b->nlines);
+    for (int l = 0; l < b->nlines; ++l) lines[(size_t)l] = l;
+    std::sort(lines.begin(), lines.end(), [b](int x, int y) { return b->h_n[x] != b->h_n[y] ? b->h_n[x] > b->h_n[y] : x < y; });
+    if (b->h_n[lines[0]] > most * kBatchResGroup) return HRW_OK;
+    std::vector<ResBlock> t;
+    long long exchanging = 0;
+    for (int l : lines) {
+        const int n = b->h_n[l];
+        const int group = n <= single ? 1 : (int)((n + most - 1) / most);
+        const int m = (n + group - 1) / group;
+        ResBlock q{};
+        q.off = b->h_off[l];
+        q.line = l;
+        q.n = n;
+        q.k = b->h_k[l];
+        q.g0 = (int)t.size();
+        q.group = group;
+        q.h = b->h_dt[l];
+        q.xmin = b->h_xmin[l];
+        q.rx = b->h_rx[l];
+        for (int i = 0; i < group; ++i) {
+            q.base = i * m;
+            q.m = std::min(m, n - i * m);
+            t.push_back(q);
+        }
+        if (group > 1) exchanging = (long long)t.size();
+    }
+    if ((long long)t.size() > (1 << 24)) return HRW_OK;
+    CALL(upload(&b->d_rblocks, t));
+    const size_t words = 4 * (size_t)exchanging * kResLine;
+    CALL(dalloc(&b->res_words, words + 1));
+    fill_u64_kernel<<<grid_for((long long)words + 1, 256, 4096), 256, 0, b->stream>>>(b->res_words, (long long)words + 1);
+    LAUNCH_CHECK();
+    HIP_TRY(hipStreamSynchronize(b->stream));
+    b->res_words_per = (unsigned)(exchanging * kResLine);
+    b->res_blocks = (long long)t.size();
+    return HRW_OK;
+}
+
+// nsteps RK3 steps of every line by batch_resident_kernel.
+static int batch_resident_steps(hrw_batch_s *b, double *u, int64_t nsteps)
+{
+    BatchResArgs a{};
+    a.u = u;
+    a.blocks = b->d_rblocks;
+    a.ticket = reinterpret_cast<unsigned *>(b->res_words + 4 * (size_t)b->res_words_per);
+    a.amax = b->alphamax();
+    a.polls = 1 << 23;   // seconds
+    a.eps = b->eps;
+    a.alpha = b->alpha;
+    a.words = b->res_words;
+    a.words_per = b->res_words_per;
+    while (nsteps > 0) {
+        // (a launch of bounded length: other streams get their turn)
+        a.nsteps = (int)std::min<int64_t>(nsteps, 64);
+        const unsigned used = 3u * (unsigned)a.nsteps;
+        if (b->res_tag > 0xffffffffu - used) {
+            const long long words = 4 * (long long)b->res_words_per;
+            fill_u64_kernel<<<grid_for(words, 256, 4096), 256, 0, b->stream>>>(b->res_words, words);
+            b->res_tag = kResFirstTag;
+        }
+        a.tag = b->res_tag;
+        a.ticket0 = b->res_started;
+        const hipError_t e = launch_batch_resident(b->numflux == HRW_FLUX_LAX_FRIEDRICHS ? LF : GODUNOV, b->res_r,
+                                                   b->res_blocks, a, b->stream);
+        if (e != hipSuccess) return fail(HRW_ERR_HIP, "kernel launch failed: %s", hipGetErrorString(e));
+        b->res_tag += used;
+        b->res_started += (unsigned)b->res_blocks;
+        nsteps -= a.nsteps;
     }
     return HRW_OK;
 }
@@ -2080,6 +2174,7 @@ extern "C" int hrw_batch_burgers_create(int64_t nlines, const int *ncells, const
     b->own_stream = true;
     HIP_TRY(hipEventCreateWithFlags(&b->ev_in, hipEventDisableTiming));
     HIP_TRY(hipEventCreateWithFlags(&b->ev_out, hipEventDisableTiming));
+    CALL(batch_resident_blocks(b));
     *out = guard.release();
     return HRW_OK;
 }
@@ -2191,8 +2286,13 @@ extern "C" int hrw_batch_step(hrw_batch_t b, double *u, int64_t nsteps, double *
     if (((uintptr_t)u & 15u) != 0) return fail(HRW_ERR_ARG, "the batch state must be 16-byte aligned");
     if (nsteps == 0) return HRW_OK;
     BatchCall order(b);
-    CALL(batch_seed(b, u));
-    if (use_graph) {
+    // (a capture would freeze the exchange numbers)
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    const bool capturing = hipStreamIsCapturing(b->stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone;
+    if (b->resident && b->res_blocks > 0 && !capturing) {
+        CALL(batch_resident_steps(b, u, nsteps));
+    } else if (use_graph) {
+        CALL(batch_seed(b, u));
         if (!b->graph || b->graph_u != u || b->graph_R != b->chunk_R || b->graph_form != b->form) {
             if (b->graph) {
                 (void)hipGraphExecDestroy(b->graph);
@@ -2213,6 +2313,7 @@ extern "C" int hrw_batch_step(hrw_batch_t b, double *u, int64_t nsteps, double *
         }
         for (int64_t s = 0; s < nsteps; ++s) HIP_TRY(hipGraphLaunch(b->graph, b->stream));
     } else {
+        CALL(batch_seed(b, u));
         for (int64_t s = 0; s < nsteps; ++s) CALL(batch_rk3_step(b, u));
     }
     if (t)
@@ -2262,8 +2363,8 @@ extern "C" int hrw_batch_step_per_line(hrw_batch_t b, double *u, int64_t nsteps,
     return HRW_OK;
 }
 
-// Autotuner: times the batched RK3 step for each kernel form and chunk width on a scratch copy
-// of the state and keeps the fastest (the result is the same for every candidate).  Each
+// Autotuner: times the batched RK3 step for each kernel form and chunk width, and three steps of
+// the whole-integration kernel, on a scratch copy of the state and keeps the fastest (the result is the same for every candidate).  Each
 // candidate is timed in two rounds, the second in reverse order, and keeps its faster one: the
 // clock drifts under the FP64 load, and a single pass in a fixed order once kept a candidate
 // 6 % slower than the best.
@@ -2310,6 +2411,24 @@ extern "C" int hrw_batch_tune(hrw_batch_t b, const double *u, int *chosen)
             best = 4 + 2 * (cand % 3);
             best_form = cand / 3;
         }
+    if (b->res_blocks > 0) {
+        float res_ms = 1e30f;
+        for (int pass = 0; pass < 3; ++pass) {   // (the first warms up)
+            (void)hipMemcpyAsync(work, u, b->total * sizeof(double), hipMemcpyDeviceToDevice, b->stream);
+            (void)hipEventRecord(e0, b->stream);
+            const int rc = batch_resident_steps(b, work, 3);
+            (void)hipEventRecord(e1, b->stream);
+            (void)hipEventSynchronize(e1);
+            if (rc != HRW_OK) {
+                dfree(work);
+                return rc;
+            }
+            float ms = 0.f;
+            (void)hipEventElapsedTime(&ms, e0, e1);
+            if (pass > 0) res_ms = std::min(res_ms, ms);
+        }
+        b->resident = res_ms < best_ms;
+    }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     dfree(work);
@@ -2326,6 +2445,7 @@ extern "C" int hrw_batch_set_cells_per_lane(hrw_batch_t b, int cells_per_lane)
     if (cells_per_lane != 4 && cells_per_lane != 6 && cells_per_lane != 8)
         return fail(HRW_ERR_ARG, "cells_per_lane must be 4, 6 or 8");
     b->R = cells_per_lane;
+    b->resident = false;
     return batch_chunks(b, cells_per_lane);
 }
 
@@ -2335,6 +2455,7 @@ extern "C" int hrw_batch_set_form(hrw_batch_t b, int form)
     if (form != HRW_BATCH_CHUNK && form != HRW_BATCH_PERSISTENT)
         return fail(HRW_ERR_ARG, "form must be HRW_BATCH_CHUNK (0) or HRW_BATCH_PERSISTENT (1)");
     b->form = form;
+    b->resident = false;
     return HRW_OK;
 }
 

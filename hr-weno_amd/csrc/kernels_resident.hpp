@@ -53,7 +53,7 @@ struct ResCoef {
     double A, C, p, s, g, q;
     int div3;
 };
-inline ResCoef res_coef(int stage, double h)
+__host__ __device__ inline ResCoef res_coef(int stage, double h)
 {
     const StageCoef c = stage_coef(stage, h);
     const double post = c.div3 ? 1.0 / 3.0 : c.post;
@@ -79,6 +79,23 @@ struct ResArgs {
     int polls;
 };
 
+// A block's part of a line: cells [base, base + m) of n, and whom it exchanges with.
+struct ResPart {
+    double *u, *saved;             // the line; saved: receives the initial state, or nullptr
+    long long n, base;
+    int m, order, nsteps;
+    bool per, amax;
+    double eps, alpha, xmin, rx;
+    const double *width, *cnu;
+    unsigned long long *words;     // lines of kResLine words, words_per per buffer
+    unsigned words_per;
+    int self, left, right;         // the block's line, its neighbours' (-1: an end of the line)
+    int g0, group;                 // the line's blocks: lines [g0, g0 + group)
+    unsigned tag;
+    int polls;
+    unsigned long long *status;    // or nullptr
+};
+
 __device__ __forceinline__ unsigned long long word_load(const unsigned long long *p)
 {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -88,9 +105,9 @@ __device__ __forceinline__ void word_store(unsigned long long *p, unsigned long 
     __hip_atomic_store(p, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 // The words of exchange `tag`; block b's line starts at word b*kResLine.
-__device__ __forceinline__ unsigned long long *res_words(const ResArgs &a, unsigned tag)
+__device__ __forceinline__ unsigned long long *res_words(const ResPart &a, unsigned tag)
 {
-    return a.words + (tag & 3) * (kResMaxBlocks * kResLine);
+    return a.words + (tag & 3) * (size_t)a.words_per;
 }
 __device__ __forceinline__ unsigned long long tag_phase(unsigned tag)   // in a maximum's sign bit
 {
@@ -174,15 +191,17 @@ __device__ __forceinline__ double face_flux(double vm, double vp, double alpha)
 }
 
 // The extra wavefront's part of an exchange: publishes the block's maximum and waits for every
-// block's; false when the polls ran out.
-__device__ __forceinline__ bool gather_max(const ResArgs &a, unsigned tag, int polls, unsigned long long mine,
+// block's of the line (at most GROUP); false when the polls ran out.
+template <int GROUP>
+__device__ __forceinline__ bool gather_max(const ResPart &a, unsigned tag, int polls, unsigned long long mine,
                                            double *line_max)
 {
-    constexpr int N = kResMaxBlocks / 64;
-    const int lane = threadIdx.x & 63, B = gridDim.x;
+    constexpr int N = GROUP / 64;
+    const int lane = threadIdx.x & 63, B = a.group;
     const unsigned long long ph = tag_phase(tag);
-    unsigned long long *words = res_words(a, tag);
-    if (lane == 0) word_store(words + blockIdx.x * kResLine + 12, mine | ph);
+    unsigned long long *all = res_words(a, tag);
+    if (lane == 0) word_store(all + a.self * kResLine + 12, mine | ph);
+    const unsigned long long *words = all + a.g0 * kResLine;
     for (int q = 0; q < polls; ++q) {
         unsigned long long w[N], miss = 0;
 #pragma unroll
@@ -206,14 +225,11 @@ __device__ __forceinline__ bool gather_max(const ResArgs &a, unsigned tag, int p
 // A wavefront that reads a halo waits for the neighbours' end cells and puts them around buf: lanes
 // 0..5 the left neighbour's last three cells, lanes 6..11 the right one's first three.  An end of
 // the line repeats its end cell (src/hrweno_weno.f90:171-173).  False when the polls ran out.
-__device__ __forceinline__ bool gather_halo(const ResArgs &a, unsigned tag, int polls, double *buf, int m, bool lo,
-                                            bool hi)
+__device__ __forceinline__ bool gather_halo(const ResPart &a, unsigned tag, int polls, double *buf, bool lo, bool hi)
 {
-    const int lane = threadIdx.x & 63, b = blockIdx.x, B = gridDim.x;
-    const int left = b > 0 ? b - 1 : (a.periodic ? B - 1 : -1);
-    const int right = b + 1 < B ? b + 1 : (a.periodic ? 0 : -1);
+    const int lane = threadIdx.x & 63, m = a.m;
     const bool use = lane < 12 && (lane < 6 ? lo : hi);
-    const int nb = lane < 6 ? left : right;
+    const int nb = lane < 6 ? a.left : a.right;
     const bool wait = use && nb >= 0;
     const unsigned long long *p = res_words(a, tag) + (wait ? nb * kResLine + (lane < 6 ? lane + 6 : lane - 6) : 0);
     unsigned long long w = 0;
@@ -231,6 +247,7 @@ __device__ __forceinline__ bool gather_halo(const ResArgs &a, unsigned tag, int 
         const int e = lane >> 1;
         double x = __builtin_bit_cast(double, ((unsigned long long)other << 32) | half);
         if (nb < 0) x = buf[lane < 6 ? 0 : m - 1];
+        else if (!ok) x = __builtin_nan("");
         buf[e < 3 ? e - 3 : m + e - 3] = x;
     }
     return ok;
@@ -243,35 +260,36 @@ template <int R> constexpr int kResPad = R + 4;
 template <int R> __host__ __device__ constexpr int res_copy(int waves) { return waves * kOutLanes * R + 2 * kResPad<R> + 2; }
 template <int R> constexpr size_t res_lds_bytes(int waves) { return 2 * (size_t)res_copy<R>(waves) * sizeof(double); }
 
-// waves: the wavefronts that own cells; with ONE false and alpha = max|u| the block has one more.
-template <int K, int FLUX, bool FAST, bool CNU, int R, bool ONE>
-__global__ __launch_bounds__(kResThreads) void resident_kernel(ResArgs a, int waves)
+// The block's part: `waves` wavefronts that own cells; with ONE false and alpha = max|u| one more
+// takes part, and `threads` counts them all.  lds, s_mx (4 words) and s_alpha: the block's LDS.  A
+// wait in vain leaves NaN behind.
+template <int K, int FLUX, bool FAST, bool CNU, int R, bool ONE, int GROUP>
+__device__ __forceinline__ void resident_part(const ResPart &a, const ResCoef *coef, int waves, int threads,
+                                              double *lds, unsigned long long *s_mx, double *s_alpha)
 {
     constexpr int H = K - 1, PAD = kResPad<R>;
-    extern __shared__ double lds[];
-    __shared__ unsigned long long s_mx[4];   // block maxima of |u|, in turn
-    __shared__ double s_alpha;
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int cap = waves * kOutLanes * R, copy = res_copy<R>(waves);
     double *cur = lds + PAD, *nxt = cur + copy;
-    const long long base = (long long)blockIdx.x * a.M;
-    const int m = (int)min((long long)a.M, a.n - base);
+    const long long base = a.base;
+    const int m = a.m;
     const int w0 = wv * kOutLanes * R, c0 = w0 + (lane - 1) * R;   // the lane's first cell in the block
     const bool owned = lane >= 1 && lane <= kOutLanes;
-    const bool amax = FLUX == LF && a.amax != 0, per = a.periodic != 0;
+    const bool amax = FLUX == LF && a.amax, per = a.per;
     const bool comm = !ONE && wv >= waves;   // the extra wavefront
+    const bool tiny = ONE && per && m < 2 * kResHalo + 2;   // a cell has several images past the ends
 
     // the initial state and its halo (other cells of the copies: zero)
-    for (int j = tid; j < 2 * copy; j += blockDim.x) lds[j] = 0.0;
+    for (int j = tid; j < 2 * copy; j += threads) lds[j] = 0.0;
     if (tid < 4) s_mx[tid] = 0ull;
     __syncthreads();
     double x0 = 0.0;
-    for (int j = tid - kResHalo; j < m + kResHalo; j += blockDim.x) {
+    for (int j = tid - kResHalo; j < m + kResHalo; j += threads) {
         const double x = a.u[cell_index(base + j, a.n, per)];
         cur[j] = x;
         if (j >= 0 && j < m) {
             x0 = max_f64(x0, fabs(x));
-            if constexpr (!ONE) a.saved[base + j] = x;
+            if (!ONE && a.saved) a.saved[base + j] = x;
         }
     }
     if (amax) {
@@ -294,7 +312,7 @@ __global__ __launch_bounds__(kResThreads) void resident_kernel(ResArgs a, int wa
         const int j = c0 + t;
         mine[t] = owned && j < m;
         at[t] = mine[t] ? j : spare;
-        image[t] = !mine[t] ? spare : (per ? (j < kResHalo ? m + j : (j >= m - kResHalo ? j - m : spare)) : spare);
+        image[t] = !mine[t] || tiny ? spare : (per ? (j < kResHalo ? m + j : (j >= m - kResHalo ? j - m : spare)) : spare);
         const long long g = base + j, gc = g < 0 ? 0 : (g < a.n ? g : a.n - 1);
         if constexpr (CNU) {
             wd[t] = a.width[gc];
@@ -322,15 +340,22 @@ __global__ __launch_bounds__(kResThreads) void resident_kernel(ResArgs a, int wa
         const unsigned tag = a.tag + (unsigned)q;
         __syncthreads();   // cur and its maximum are complete
         if (amax && tid == 0) s_mx[(q + 2) & 3] = 0ull;
+        if (tiny) {
+            if (tid < 2 * kResHalo) {
+                const int j = tid < kResHalo ? tid - kResHalo : m + tid - kResHalo;
+                cur[j] = cur[cell_index(j, m, true)];
+            }
+            __syncthreads();
+        }
         double v[R + 2 * H], vl[R], vr[R], vr_left = 0.0, vl_right = 0.0;
         if (!comm) {
             if constexpr (!ONE) {
                 if (q > 0 && (read_lo || read_hi)) {
                     // (these wavefronts first: theirs is the longer way)
                     __builtin_amdgcn_s_setprio(2);
-                    if (!gather_halo(a, tag, polls, cur, m, read_lo, read_hi)) {
+                    if (!gather_halo(a, tag, polls, cur, read_lo, read_hi)) {
                         polls = 1;
-                        if (lane == 0) atomicOr(a.status, (unsigned long long)RES_TIMEOUT);
+                        if (a.status && lane == 0) atomicOr(a.status, (unsigned long long)RES_TIMEOUT);
                     }
                     __builtin_amdgcn_wave_barrier();
                 }
@@ -342,16 +367,16 @@ __global__ __launch_bounds__(kResThreads) void resident_kernel(ResArgs a, int wa
             vr_left = shfl_up1(vr[R - 1]);
             vl_right = shfl_down1(vl[0]);
         } else {
-            double x = 0.0;
-            if (!gather_max(a, tag, polls, s_mx[q & 3], &x)) {
+            double x = __builtin_nan("");
+            if (!gather_max<GROUP>(a, tag, polls, s_mx[q & 3], &x)) {
                 polls = 1;
-                if (lane == 0) atomicOr(a.status, (unsigned long long)RES_TIMEOUT);
+                if (a.status && lane == 0) atomicOr(a.status, (unsigned long long)RES_TIMEOUT);
             }
-            if (lane == 0) s_alpha = x;
+            if (lane == 0) *s_alpha = x;
         }
         if (!ONE && amax) {
             __syncthreads();   // the line's maximum is known
-            alpha = s_alpha;
+            alpha = *s_alpha;
         }
         if (comm) {
             if (q + 1 == stages) break;
@@ -370,7 +395,7 @@ __global__ __launch_bounds__(kResThreads) void resident_kernel(ResArgs a, int wa
                     if (t == gl) f[t + 1] = f[t];
             }
         }
-        const ResCoef &co = a.coef[st];
+        const ResCoef &co = coef[st];
         if (st == 0) {
 #pragma unroll
             for (int t = 0; t < R; ++t) u0[t] = v[H + t];
@@ -422,7 +447,7 @@ __global__ __launch_bounds__(kResThreads) void resident_kernel(ResArgs a, int wa
                     }
                 }
             } else {
-                unsigned long long *line = res_words(a, tag + 1) + blockIdx.x * kResLine;
+                unsigned long long *line = res_words(a, tag + 1) + a.self * kResLine;
 #pragma unroll
                 for (int t = 0; t < R; ++t) {
                     const int j = c0 + t;
@@ -453,7 +478,128 @@ __global__ __launch_bounds__(kResThreads) void resident_kernel(ResArgs a, int wa
         nxt = sw;
         if (++st == a.order) st = 0;
     }
-    if (__any(bad) && lane == 0) atomicOr(a.status, (unsigned long long)RES_NONFINITE);
+    if (a.status && __any(bad) && lane == 0) atomicOr(a.status, (unsigned long long)RES_NONFINITE);
+}
+
+// One line over the whole grid.
+template <int K, int FLUX, bool FAST, bool CNU, int R, bool ONE>
+__global__ __launch_bounds__(kResThreads) void resident_kernel(ResArgs a, int waves)
+{
+    extern __shared__ double lds[];
+    __shared__ unsigned long long s_mx[4];   // block maxima of |u|, in turn
+    __shared__ double s_alpha;
+    const int b = blockIdx.x, B = gridDim.x;
+    ResPart p;
+    p.u = a.u;
+    p.saved = a.saved;
+    p.n = a.n;
+    p.base = (long long)b * a.M;
+    p.m = (int)min((long long)a.M, a.n - p.base);
+    p.order = a.order;
+    p.nsteps = a.nsteps;
+    p.per = a.periodic != 0;
+    p.amax = a.amax != 0;
+    p.eps = a.eps;
+    p.alpha = a.alpha;
+    p.xmin = a.xmin;
+    p.rx = a.rx;
+    p.width = a.width;
+    p.cnu = a.cnu;
+    p.words = a.words;
+    p.words_per = kResMaxBlocks * kResLine;
+    p.self = b;
+    p.left = b > 0 ? b - 1 : (p.per ? B - 1 : -1);
+    p.right = b + 1 < B ? b + 1 : (p.per ? 0 : -1);
+    p.g0 = 0;
+    p.group = B;
+    p.tag = a.tag;
+    p.polls = a.polls;
+    p.status = a.status;
+    resident_part<K, FLUX, FAST, CNU, R, ONE, kResMaxBlocks>(p, a.coef, waves, blockDim.x, lds, s_mx, &s_alpha);
+}
+
+// ---- an ensemble of periodic lines (kernels_1d_fast.hpp's batch), each on a block or a few ----
+// Block i of the table works on cells [base, base + m) of one line for nsteps RK3 steps: 16 bytes
+// of memory traffic per cell and launch instead of 64 per cell and step.  The blocks of one line
+// are neighbours in the table, and a block takes the table entry of its turn to start, so at any
+// time at most one line has some of its blocks waiting for others that have not started: the lines
+// ahead of it run to their ends and make room.  Two blocks of eight wavefronts share a CU; one
+// computes while the other waits for its exchange.
+constexpr int kBatchResWaves = 8;
+constexpr int kBatchResGroup = 64;      // blocks per line at most
+struct ResBlock {
+    long long off;                      // the line's first cell in the flat state
+    int line, n, k, base, m;            // the line, its length and order; this block's cells
+    int g0, group, pad;                 // the line's blocks [g0, g0 + group)
+    double h, xmin, rx;
+};
+struct BatchResArgs {
+    double *u;
+    const ResBlock *blocks;
+    unsigned *ticket;                   // starts counted so far
+    unsigned ticket0;                   // ... before this launch
+    int nsteps, amax, polls;
+    double eps, alpha;
+    unsigned long long *words;
+    unsigned words_per, tag;
+};
+
+template <int FLUX, int R>
+__global__ __launch_bounds__(64 * kBatchResWaves) __attribute__((amdgpu_waves_per_eu(4))) void batch_resident_kernel(
+    BatchResArgs a)
+{
+    extern __shared__ double lds[];
+    __shared__ unsigned long long s_mx[4];
+    __shared__ double s_alpha;
+    __shared__ ResCoef s_coef[3];
+    __shared__ unsigned s_turn;
+    const int wv = threadIdx.x >> 6;
+    if (threadIdx.x == 0) s_turn = atomicAdd(a.ticket, 1u) - a.ticket0;
+    __syncthreads();
+    const int turn = __builtin_amdgcn_readfirstlane((int)s_turn);
+    const ResBlock &b = a.blocks[turn];
+    const int waves = (b.m + kOutLanes * R - 1) / (kOutLanes * R);
+    const int threads = 64 * (waves + (b.group > 1 && a.amax ? 1 : 0));
+    if (threadIdx.x < 3) s_coef[threadIdx.x] = res_coef(RK3_1 + (int)threadIdx.x, b.h);
+    if (64 * wv >= threads) return;   // (whole wavefronts; a barrier counts those that are left)
+    ResPart p;
+    p.u = a.u + b.off;
+    p.saved = nullptr;
+    p.n = b.n;
+    p.base = b.base;
+    p.m = b.m;
+    p.order = 3;
+    p.nsteps = a.nsteps;
+    p.per = true;
+    p.amax = a.amax != 0;
+    p.eps = a.eps;
+    p.alpha = a.alpha;
+    p.xmin = b.xmin;
+    p.rx = b.rx;
+    p.width = p.cnu = nullptr;
+    p.words = a.words;
+    p.words_per = a.words_per;
+    p.self = turn;
+    p.left = b.base > 0 ? turn - 1 : b.g0 + b.group - 1;
+    p.right = b.base + b.m < b.n ? turn + 1 : b.g0;
+    p.g0 = b.g0;
+    p.group = b.group;
+    p.tag = a.tag;
+    p.polls = a.polls;
+    p.status = nullptr;
+#define HRW_RES_PART(K)                                                                                       \
+    if (b.group == 1)                                                                                         \
+        resident_part<K, FLUX, true, false, R, true, kBatchResGroup>(p, s_coef, waves, threads, lds, s_mx, &s_alpha); \
+    else                                                                                                      \
+        resident_part<K, FLUX, true, false, R, false, kBatchResGroup>(p, s_coef, waves, threads, lds, s_mx, &s_alpha)
+    if (b.k == 3) {
+        HRW_RES_PART(3);
+    } else if (b.k == 2) {
+        HRW_RES_PART(2);
+    } else {
+        HRW_RES_PART(1);
+    }
+#undef HRW_RES_PART
 }
 
 }  // namespace hrw

@@ -47,6 +47,8 @@ struct ResPlan {
 hipError_t launch_resident_k1(int flux, bool fast, const ResPlan &pl, const ResArgs &a, hipStream_t s);
 hipError_t launch_resident_k2(int flux, bool fast, const ResPlan &pl, const ResArgs &a, hipStream_t s);
 hipError_t launch_resident_k3(int flux, bool fast, const ResPlan &pl, const ResArgs &a, hipStream_t s);
+// nsteps RK3 steps of every line of a batch in one launch, r cells per lane (2 or 4).
+hipError_t launch_batch_resident(int flux, int r, long long blocks, const BatchResArgs &a, hipStream_t s);
 // LDS-tile 1D stage (EXACT form, and the FAST LDS variant).
 void launch_tile_1d(int k, int flux, bool periodic, bool fast, bool alphamax, const Stage1DArgs &a,
                     hipStream_t s);

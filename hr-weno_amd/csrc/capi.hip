@@ -1365,7 +1365,7 @@ static int ode_read_status(hrw_ode_s *o, unsigned long long *bad)
 // lane per block, which hide each other's latency; more blocks cost alpha's exchange more (64:
 // 1.6 us, 128: 1.7, 256: 2.3), so with it and the FAST form, whose cells are cheap, two cells per
 // lane come in earlier.  False: the line does not fit.
-static bool resident_split(long long n, bool exact, bool amax, bool nonuniform, ResPlan *pl)
+static bool resident_split(long long n, int order, bool exact, bool amax, bool nonuniform, ResPlan *pl)
 {
     const int most_waves = kResThreads / 64;
     auto one = [&](int r) {
@@ -1376,20 +1376,22 @@ static bool resident_split(long long n, bool exact, bool amax, bool nonuniform, 
     };
     if (n <= 10 * kOutLanes) return one(1);
     if (!exact && !nonuniform && n <= (amax ? 12 : 9) * 2 * kOutLanes) return one(2);
+    const int both = 2 * res_extra(order);   // cells a block computes past its ends
     // blocks of `waves` wavefronts, at most `blocks` of them; or, with `blocks` of them, as many
     // wavefronts as it takes, at most `waves`
     auto several = [&](int r, int waves, int blocks) {
-        const long long per = (long long)waves * kOutLanes * r, nb = (n + per - 1) / per;
+        const long long per = (long long)waves * kOutLanes * r - both, nb = (n + per - 1) / per;
         if (nb > blocks) return false;
         const long long m = (n + nb - 1) / nb;   // cells per block
         pl->r = r;
         pl->blocks = (int)((n + m - 1) / m);
-        pl->waves = (int)((m + kOutLanes * r - 1) / (kOutLanes * r));
-        return n - m * (pl->blocks - 1) >= kResHalo;
+        pl->waves = (int)((m + both + kOutLanes * r - 1) / (kOutLanes * r));
+        return n - m * (pl->blocks - 1) >= kResEdge;
     };
     const int cap = most_waves - (amax ? 1 : 0);
     auto widen = [&](int r, int waves) {   // all blocks, `waves` wavefronts at most
-        const long long w = (n + (long long)kResMaxBlocks * kOutLanes * r - 1) / ((long long)kResMaxBlocks * kOutLanes * r);
+        const long long m = (n + kResMaxBlocks - 1) / kResMaxBlocks + both;
+        const long long w = (m + kOutLanes * r - 1) / (kOutLanes * r);
         return w <= waves && several(r, (int)w, kResMaxBlocks);
     };
     if (nonuniform) return several(1, 7, kResMaxBlocks) || widen(1, cap);
@@ -1407,7 +1409,7 @@ static bool resident_plan(const hrw_ode_s *o, int64_t nsteps, ResPlan *pl)
     if (p->kind != PROB_BURGERS1D || p->variant != 0 || p->cells_per_lane != 0) return false;
     const bool exact = p->arith != HRW_ARITH_FAST;
     if (!p->d_cnu && (p->d_width || (!exact && !near_linear_grid(p->xmin, p->rx, p->neq)))) return false;
-    if (p->neq < 8 || !resident_split(p->neq, exact, p->alphamax(), p->d_cnu != nullptr, pl)) return false;
+    if (p->neq < 8 || !resident_split(p->neq, o->order, exact, p->alphamax(), p->d_cnu != nullptr, pl)) return false;
     // (a launch's first stage must not be its last: blocks read each other's initial cells)
     if (pl->blocks > device_cus() || (pl->blocks > 1 && !o->res_words) || nsteps * o->order < 2 || nsteps >= (1 << 26)) return false;
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
@@ -2040,7 +2042,7 @@ static int batch_resident_blocks(hrw_batch_s *b)
 {
     const int r = b->res_r = *std::max_element(b->h_n.begin(), b->h_n.end()) <= 2048 ? 2 : 4;
     const int waves = kBatchResWaves - (b->alphamax() ? 1 : 0);   // (one for the maxima)
-    const long long most = (long long)waves * kOutLanes * r, single = (long long)kBatchResWaves * kOutLanes * r;
+    const long long most = (long long)waves * kOutLanes * r - 2 * res_extra(3), single = (long long)kBatchResWaves * kOutLanes * r;
     std::vector<int> lines((size_t)b->nlines);
     for (int l = 0; l < b->nlines; ++l) lines[(size_t)l] = l;
     std::sort(lines.begin(), lines.end(), [b](int x, int y) { return b->h_n[x] != b->h_n[y] ? b->h_n[x] > b->h_n[y] : x < y; });

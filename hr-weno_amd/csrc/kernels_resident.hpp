@@ -5,15 +5,17 @@
 // in LDS and registers for every step of the call (src/hrweno_tvdode.f90:136-171): block b owns M
 // consecutive cells, its lanes R consecutive cells each, and a stage reads the block's LDS copy of
 // the stage input and writes the other copy.  One block needs nothing else.  Several blocks (at
-// most one per CU, so that all come to be resident) exchange, after each stage, the three cells at
-// each of their ends with their neighbours and the block maxima of |u| (alpha = max|u|) with every
-// block.
+// most one per CU, so that all come to be resident) exchange, after each step, the cells at each of
+// their ends that the next step's stages reach (three per stage) with their neighbours, and after
+// each stage the block maxima of |u| (alpha = max|u|) with every block.  Within a step they compute
+// the cells past their ends that the later stages need themselves: the same values as their owners',
+// operation for operation.
 //
 // An exchange takes 1.4 us between neighbours and 1.6 / 1.7 / 2.3 us among 64 / 128 / 256 blocks
 // (each block's words on a cache line of their own; packed, writers and readers of one line queue
 // up: 2.3 / 2.7 / 3.1).  What does not wait for it runs beside it: the reconstruction of a stage
 // needs no alpha, so one wavefront more per block sees to the maxima while the others reconstruct,
-// and only the wavefronts that read a halo wait for the neighbours' cells.
+// and only the wavefronts that read a halo wait for the neighbours' cells, once a step.
 //
 // The exchange takes no fence.  A double travels as two 64-bit words, each half of it beside the
 // 32-bit number of the exchange; a maximum (a non-negative double) as one word with a bit of the
@@ -36,9 +38,12 @@
 
 namespace hrw {
 
-constexpr int kResHalo = 3;        // cells exchanged at each end (a face needs K = 3 each side)
+constexpr int kResHalo = 3;        // cells a stage reaches past each end (a face needs K = 3 each side)
+constexpr int kResEdge = 9;        // cells exchanged at each end at most (the three stages of a step)
 constexpr int kResMaxBlocks = 256;
-constexpr int kResLine = 16;       // words per block and exchange: 12 of edge cells, 1 maximum
+// words per block and exchange: the maximum on a cache line of its own (read by every block), from
+// word 16 on the first and the last kResEdge cells
+constexpr int kResLine = 64;
 constexpr int kResThreads = 1024;
 constexpr size_t kResWords = 4 * (size_t)kResMaxBlocks * kResLine;   // one object's exchange words
 constexpr unsigned kResFirstTag = 4;   // the number after which cleared words read as not arrived
@@ -68,7 +73,7 @@ struct ResArgs {
     double *u;                     // state, read at the start and written at the end
     double *saved;                 // several blocks: receives the initial state
     long long n;
-    int M;                         // cells per block (the last block: what is left, >= kResHalo)
+    int M;                         // cells per block (the last block: what is left, >= kResEdge)
     int order, nsteps, periodic, amax;
     double eps, alpha, xmin, rx;
     ResCoef coef[3];               // of the step's stages
@@ -104,6 +109,16 @@ __device__ __forceinline__ void word_store(unsigned long long *p, unsigned long 
 {
     __hip_atomic_store(p, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+// cell_index in 32 bits (a line here has fewer than 2^31 cells, and i lies near it).
+__device__ __forceinline__ int line_cell(long long i, long long n, bool periodic)
+{
+    const int j = (int)i, c = (int)n;
+    if (j >= 0 && j < c) return j;
+    if (!periodic) return j < 0 ? 0 : c - 1;
+    const int r = j % c;
+    return r < 0 ? r + c : r;
+}
+
 // The words of exchange `tag`; block b's line starts at word b*kResLine.
 __device__ __forceinline__ unsigned long long *res_words(const ResPart &a, unsigned tag)
 {
@@ -200,13 +215,13 @@ __device__ __forceinline__ bool gather_max(const ResPart &a, unsigned tag, int p
     const int lane = threadIdx.x & 63, B = a.group;
     const unsigned long long ph = tag_phase(tag);
     unsigned long long *all = res_words(a, tag);
-    if (lane == 0) word_store(all + a.self * kResLine + 12, mine | ph);
+    if (lane == 0) word_store(all + a.self * kResLine, mine | ph);
     const unsigned long long *words = all + a.g0 * kResLine;
     for (int q = 0; q < polls; ++q) {
         unsigned long long w[N], miss = 0;
 #pragma unroll
         for (int i = 0; i < N; ++i)   // (lanes past the last block read its word)
-            w[i] = i == 0 || 64 * i < B ? word_load(words + min(64 * i + lane, B - 1) * kResLine + 12) : ph;
+            w[i] = i == 0 || 64 * i < B ? word_load(words + min(64 * i + lane, B - 1) * kResLine) : ph;
         double x = 0.0;
 #pragma unroll
         for (int i = 0; i < N; ++i) {
@@ -222,41 +237,46 @@ __device__ __forceinline__ bool gather_max(const ResPart &a, unsigned tag, int p
     return false;
 }
 
-// A wavefront that reads a halo waits for the neighbours' end cells and puts them around buf: lanes
-// 0..5 the left neighbour's last three cells, lanes 6..11 the right one's first three.  An end of
-// the line repeats its end cell (src/hrweno_weno.f90:171-173).  False when the polls ran out.
-__device__ __forceinline__ bool gather_halo(const ResPart &a, unsigned tag, int polls, double *buf, bool lo, bool hi)
+// A wavefront that reads a halo waits for the neighbours' end cells, `width` of them each, and puts
+// them around buf: word 2e + half of the left neighbour's last cells by lanes 0 .. 2 width - 1, of
+// the right one's first cells by as many lanes from 32 on.  An end of the line repeats its end cell
+// (src/hrweno_weno.f90:171-173).  False when the polls ran out (the halo is NaN then).
+__device__ __forceinline__ bool gather_halo(const ResPart &a, unsigned tag, int polls, int width, double *buf, bool lo,
+                                            bool hi)
 {
-    const int lane = threadIdx.x & 63, m = a.m;
-    const bool use = lane < 12 && (lane < 6 ? lo : hi);
-    const int nb = lane < 6 ? a.left : a.right;
+    const int lane = threadIdx.x & 63, m = a.m, w = lane & 31;
+    const bool left = lane < 32, use = w < 2 * width && (left ? lo : hi);
+    const int nb = left ? a.left : a.right;
     const bool wait = use && nb >= 0;
-    const unsigned long long *p = res_words(a, tag) + (wait ? nb * kResLine + (lane < 6 ? lane + 6 : lane - 6) : 0);
-    unsigned long long w = 0;
+    // (a block's words: its first cells, then its last ones)
+    const unsigned long long *p =
+        res_words(a, tag) + (wait ? nb * kResLine + 16 + (left ? 2 * (kResEdge + kResEdge - width) : 0) + w : 0);
+    unsigned long long x = 0;
     bool ok = false;
     for (int q = 0; q < polls; ++q) {
-        if (wait) w = word_load(p);
-        if (__all(!wait || (unsigned)w == tag)) {
+        if (wait) x = word_load(p);
+        if (__all(!wait || (unsigned)x == tag)) {
             ok = true;
             break;
         }
     }
-    const unsigned half = (unsigned)(w >> 32);   // words 2e and 2e + 1: the halves of cell e
+    const unsigned half = (unsigned)(x >> 32);
     const unsigned other = (unsigned)__builtin_amdgcn_update_dpp(0, (int)half, 0xB1, 0xF, 0xF, true);   // lane ^ 1
     if (use && !(lane & 1)) {
-        const int e = lane >> 1;
-        double x = __builtin_bit_cast(double, ((unsigned long long)other << 32) | half);
-        if (nb < 0) x = buf[lane < 6 ? 0 : m - 1];
-        else if (!ok) x = __builtin_nan("");
-        buf[e < 3 ? e - 3 : m + e - 3] = x;
+        double c = __builtin_bit_cast(double, ((unsigned long long)other << 32) | half);
+        if (nb < 0) c = buf[left ? 0 : m - 1];
+        else if (!ok) c = __builtin_nan("");
+        buf[(left ? -width : m) + (w >> 1)] = c;
     }
     return ok;
 }
 
-// LDS: two copies of the block's cells with kResPad cells on each side (the three halo cells, and
-// room for what the wave-edge lanes read beyond them, which feeds no cell), and after each copy one
-// cell more that takes the writes of cells that are not the block's.
-template <int R> constexpr int kResPad = R + 4;
+// LDS: two copies of the block's cells with kResPad cells on each side (the halo, and room for what
+// the wave-edge lanes read beyond it, which feeds no cell), and after each copy one cell more that
+// takes the writes of cells the block does not keep.
+template <int R> constexpr int kResPad = R + kResEdge + 1;
+// Cells past each end that a block of several computes in a step's first stage.
+__host__ __device__ constexpr int res_extra(int order) { return kResHalo * (order - 1); }
 template <int R> __host__ __device__ constexpr int res_copy(int waves) { return waves * kOutLanes * R + 2 * kResPad<R> + 2; }
 template <int R> constexpr size_t res_lds_bytes(int waves) { return 2 * (size_t)res_copy<R>(waves) * sizeof(double); }
 
@@ -273,23 +293,36 @@ __device__ __forceinline__ void resident_part(const ResPart &a, const ResCoef *c
     double *cur = lds + PAD, *nxt = cur + copy;
     const long long base = a.base;
     const int m = a.m;
-    const int w0 = wv * kOutLanes * R, c0 = w0 + (lane - 1) * R;   // the lane's first cell in the block
+    const int extra = ONE ? 0 : res_extra(a.order), width = extra + kResHalo;
+    const int w0 = wv * kOutLanes * R - extra, c0 = w0 + (lane - 1) * R;   // the lane's first cell in the block
     const bool owned = lane >= 1 && lane <= kOutLanes;
     const bool amax = FLUX == LF && a.amax, per = a.per;
     const bool comm = !ONE && wv >= waves;   // the extra wavefront
     const bool tiny = ONE && per && m < 2 * kResHalo + 2;   // a cell has several images past the ends
 
-    // the initial state and its halo (other cells of the copies: zero)
-    for (int j = tid; j < 2 * copy; j += threads) lds[j] = 0.0;
+    // the initial state and its halo, R + 1 loads in flight per thread; what the copies hold beyond
+    // feeds no cell (EXACT: zero, so that no lane takes the divides over it)
+    if (!FAST || CNU)
+        for (int j = tid; j < 2 * copy; j += threads) lds[j] = 0.0;
     if (tid < 4) s_mx[tid] = 0ull;
     __syncthreads();
     double x0 = 0.0;
-    for (int j = tid - kResHalo; j < m + kResHalo; j += threads) {
-        const double x = a.u[cell_index(base + j, a.n, per)];
-        cur[j] = x;
-        if (j >= 0 && j < m) {
-            x0 = max_f64(x0, fabs(x));
-            if (!ONE && a.saved) a.saved[base + j] = x;
+    for (int j0 = tid - width; j0 < m + width; j0 += (R + 1) * threads) {
+        double x[R + 1];
+#pragma unroll
+        for (int i = 0; i <= R; ++i) {
+            const int j = j0 + i * threads;
+            if (j < m + width) x[i] = a.u[line_cell(base + j, a.n, per)];
+        }
+#pragma unroll
+        for (int i = 0; i <= R; ++i) {
+            const int j = j0 + i * threads;
+            if (j >= m + width) continue;
+            cur[j] = x[i];
+            if (j >= 0 && j < m) {
+                x0 = max_f64(x0, fabs(x[i]));
+                if (!ONE && a.saved) a.saved[base + j] = x[i];
+            }
         }
     }
     if (amax) {
@@ -298,8 +331,8 @@ __device__ __forceinline__ void resident_part(const ResPart &a, const ResCoef *c
     }
 
     // what does not change with the steps: cell widths (FAST: their reciprocals), the non-uniform
-    // grid's coefficients, which cells are this lane's, where it writes them (others: `spare`) and
-    // (the only block of a line) their images past its ends
+    // grid's coefficients, which cells are the block's, where the lane writes its cells (`spare`:
+    // those it does not keep) and (the only block of a line) their images past its ends
     const int spare = cap + PAD;
     double wd[R];
     [[maybe_unused]] double ci[CNU ? R * K * (K + 1) : 1];
@@ -310,26 +343,29 @@ __device__ __forceinline__ void resident_part(const ResPart &a, const ResCoef *c
 #pragma unroll
     for (int t = 0; t < R; ++t) {
         const int j = c0 + t;
-        mine[t] = owned && j < m;
-        at[t] = mine[t] ? j : spare;
+        const long long g = base + j;
+        const int gc = line_cell(g, a.n, per);
+        mine[t] = owned && j >= 0 && j < m;
+        at[t] = owned && j >= -extra && j < m + extra && (per || (g >= 0 && g < a.n)) ? j : spare;
         image[t] = !mine[t] || tiny ? spare : (per ? (j < kResHalo ? m + j : (j >= m - kResHalo ? j - m : spare)) : spare);
-        const long long g = base + j, gc = g < 0 ? 0 : (g < a.n ? g : a.n - 1);
         if constexpr (CNU) {
             wd[t] = a.width[gc];
 #pragma unroll
-            for (int q = 0; q < K * (K + 1); ++q) ci[t * K * (K + 1) + q] = a.cnu[gc * (K * (K + 1)) + q];
+            for (int q = 0; q < K * (K + 1); ++q) ci[t * K * (K + 1) + q] = a.cnu[(long long)gc * (K * (K + 1)) + q];
         } else {
             const double w = linear_edge(a.xmin, a.rx, gc + 1) - linear_edge(a.xmin, a.rx, gc);
             wd[t] = FAST ? fma_(inv_rx, fma_(-w, inv_rx, 1.0), inv_rx) : w;
         }
     }
-    // zero-gradient ends (example1:103-104): the lane that holds cell 0, and cell n-1
-    const long long gl = a.n - 1 - base - c0;
-    const bool first = !per && base + c0 == 0 && owned, last = !per && owned && gl >= 0 && gl < R;
-    // this wavefront owns end cells of the block / reads halo cells / holds an end of the line
-    const bool own_end = (wv == 0 || w0 + kOutLanes * R > m - kResHalo) && w0 < m;
+    // zero-gradient ends (example1:103-104): the lane's cell that is cell 0, and cell n-1 (-1: none)
+    const long long gf = -base - c0, gl = a.n - 1 - base - c0;
+    const int first = !per && owned && gf >= 0 && gf < R ? (int)gf : -1;
+    const int last = !per && owned && gl >= 0 && gl < R ? (int)gl : -1;
+    // this wavefront owns end cells that are exchanged (or have images) / reads halo cells / holds
+    // an end of the line
+    const bool own_end = w0 < m && (wv == 0 || w0 + kOutLanes * R > m - width);
     const bool read_lo = wv == 0, read_hi = w0 + 63 * R + H > m;
-    const bool line_end = __any(first || last);
+    const bool line_end = __any(first >= 0 || last >= 0);
 
     const int stages = a.order * a.nsteps;
     double u0[R];
@@ -343,21 +379,22 @@ __device__ __forceinline__ void resident_part(const ResPart &a, const ResCoef *c
         if (tiny) {
             if (tid < 2 * kResHalo) {
                 const int j = tid < kResHalo ? tid - kResHalo : m + tid - kResHalo;
-                cur[j] = cur[cell_index(j, m, true)];
+                cur[j] = cur[line_cell(j, m, true)];
             }
             __syncthreads();
         }
         double v[R + 2 * H], vl[R], vr[R], vr_left = 0.0, vl_right = 0.0;
         if (!comm) {
             if constexpr (!ONE) {
-                if (q > 0 && (read_lo || read_hi)) {
+                if (st == 0 && q > 0 && (read_lo || read_hi)) {
                     // (these wavefronts first: theirs is the longer way)
                     __builtin_amdgcn_s_setprio(2);
-                    if (!gather_halo(a, tag, polls, cur, read_lo, read_hi)) {
+                    if (!gather_halo(a, tag, polls, width, cur, read_lo, read_hi)) {
                         polls = 1;
                         if (a.status && lane == 0) atomicOr(a.status, (unsigned long long)RES_TIMEOUT);
                     }
                     __builtin_amdgcn_wave_barrier();
+                    __builtin_amdgcn_s_setprio(0);
                 }
             }
 #pragma unroll
@@ -388,12 +425,12 @@ __device__ __forceinline__ void resident_part(const ResPart &a, const ResCoef *c
         for (int t = 1; t < R; ++t) f[t] = face_flux<K, FLUX, FAST, CNU>(vr[t - 1], vl[t], alpha);
         f[R] = face_flux<K, FLUX, FAST, CNU>(vr[R - 1], vl_right, alpha);
         if (line_end) {
-            if (first) f[0] = f[1];
-            if (last) {
 #pragma unroll
-                for (int t = 0; t < R; ++t)
-                    if (t == gl) f[t + 1] = f[t];
-            }
+            for (int t = 0; t < R; ++t)
+                if (t == first) f[t] = f[t + 1];
+#pragma unroll
+            for (int t = 0; t < R; ++t)
+                if (t == last) f[t + 1] = f[t];
         }
         const ResCoef &co = coef[st];
         if (st == 0) {
@@ -432,38 +469,36 @@ __device__ __forceinline__ void resident_part(const ResPart &a, const ResCoef *c
         }
 #pragma unroll
         for (int t = 0; t < R; ++t) nxt[at[t]] = un[t];
-        if (own_end) {
-            // the next stage's halos: the only block's own images, or words for the neighbours
-            if constexpr (ONE) {
-                if (per) {
+        if (line_end) {   // the line's ends repeat their end cells (src/hrweno_weno.f90:171-173)
 #pragma unroll
-                    for (int t = 0; t < R; ++t) nxt[image[t]] = un[t];
-                } else if (line_end) {   // (src/hrweno_weno.f90:171-173)
-                    if (first) nxt[-1] = nxt[-2] = nxt[-3] = un[0];
-                    if (last) {
+            for (int t = 0; t < R; ++t) {
+                if (t == first) nxt[-1] = nxt[-2] = nxt[-3] = un[t];
+                if (t == last) nxt[m] = nxt[m + 1] = nxt[m + 2] = un[t];
+            }
+        }
+        if constexpr (ONE) {
+            if (own_end && per) {
 #pragma unroll
-                        for (int t = 0; t < R; ++t)
-                            if (t == gl) nxt[m] = nxt[m + 1] = nxt[m + 2] = un[t];
-                    }
+                for (int t = 0; t < R; ++t) nxt[image[t]] = un[t];
+            }
+        } else if (own_end && st + 1 == a.order) {
+            // words for the neighbours' next step
+            unsigned long long *line = res_words(a, tag + 1) + a.self * kResLine + 16;
+#pragma unroll
+            for (int t = 0; t < R; ++t) {
+                const int j = c0 + t;
+                const unsigned long long bits = __builtin_bit_cast(unsigned long long, un[t]);
+                const unsigned long long wl = (bits << 32) | (tag + 1);
+                const unsigned long long wh = (bits & 0xffffffff00000000ull) | (tag + 1);
+                if (mine[t] && j < width) {
+                    word_store(line + 2 * j, wl);
+                    word_store(line + 2 * j + 1, wh);
                 }
-            } else {
-                unsigned long long *line = res_words(a, tag + 1) + a.self * kResLine;
-#pragma unroll
-                for (int t = 0; t < R; ++t) {
-                    const int j = c0 + t;
-                    const unsigned long long bits = __builtin_bit_cast(unsigned long long, un[t]);
-                    const unsigned long long wl = (bits << 32) | (tag + 1);
-                    const unsigned long long wh = (bits & 0xffffffff00000000ull) | (tag + 1);
-                    if (mine[t] && j < kResHalo) {
-                        word_store(line + 2 * j, wl);
-                        word_store(line + 2 * j + 1, wh);
-                    }
-                    if (mine[t] && j >= m - kResHalo) {
-                        word_store(line + 6 + 2 * (j - (m - kResHalo)), wl);
-                        word_store(line + 7 + 2 * (j - (m - kResHalo)), wh);
-                    }
+                if (mine[t] && j >= m - width) {
+                    unsigned long long *e = line + 2 * (j - m + 2 * kResEdge);
+                    word_store(e, wl);
+                    word_store(e + 1, wh);
                 }
-                __builtin_amdgcn_s_setprio(0);
             }
         }
         if (amax) {
@@ -558,7 +593,7 @@ __global__ __launch_bounds__(64 * kBatchResWaves) __attribute__((amdgpu_waves_pe
     __syncthreads();
     const int turn = __builtin_amdgcn_readfirstlane((int)s_turn);
     const ResBlock &b = a.blocks[turn];
-    const int waves = (b.m + kOutLanes * R - 1) / (kOutLanes * R);
+    const int waves = (b.m + (b.group > 1 ? 2 * res_extra(3) : 0) + kOutLanes * R - 1) / (kOutLanes * R);
     const int threads = 64 * (waves + (b.group > 1 && a.amax ? 1 : 0));
     if (threadIdx.x < 3) s_coef[threadIdx.x] = res_coef(RK3_1 + (int)threadIdx.x, b.h);
     if (64 * wv >= threads) return;   // (whole wavefronts; a barrier counts those that are left)

@@ -45,7 +45,7 @@ FLUXES = [(LF, -1.0), (LF, 2.0), (GOD, -1.0)]
 @pytest.mark.parametrize("top", [2048, 9000])
 def test_line_lengths(hh, dev, flux, alpha, top):
     """Two cells per lane (no line above 2048 cells) and four."""
-    ns = [1, 2, 3, 5, 7, 8, 9, 61, 62, 63, 64, 123, 124, 125, 247, 248, 249, 991, 992, 993, 1735, 1736, 1737, 1983,
+    ns = [1, 2, 3, 5, 7, 8, 9, 61, 62, 63, 64, 123, 124, 125, 247, 248, 249, 991, 992, 993, 1723, 1724, 1735, 1736, 1737, 1983,
           1984, 1985, top]
     ns = [n for n in ns if n <= top]
     for k in (1, 2, 3):
@@ -56,11 +56,11 @@ def test_line_lengths(hh, dev, flux, alpha, top):
 def test_split_lines(hh, dev, flux, alpha):
     """Lines over 2 to 64 blocks, with short ones between them; more blocks than the chip holds."""
     rng = np.random.default_rng(4)
-    ns = [111104, 40000, 3473, 5000, 3970, 100, 17, 65536, 20001] + list(rng.integers(2000, 30000, 60))
+    ns = [110336, 40000, 3448, 3449, 3473, 5000, 3970, 100, 17, 65536, 20001] + list(rng.integers(2000, 30000, 60))
     both(hh, dev, ns, [2 + i % 2 for i in range(len(ns))], flux, alpha, 3)
 
 
-@pytest.mark.parametrize("n", [111105, 130000])
+@pytest.mark.parametrize("n", [110337, 126209])
 def test_lines_that_do_not_fit_take_the_stages(hh, dev, n):
     both(hh, dev, [n, 300], [3, 2], LF, -1.0, 2)
 

@@ -63,13 +63,13 @@ def test_orders(hh, dev, n, order, k, arith):
 
 # the steps of the split: 96 blocks of 7 wavefronts (one, two cells per lane), 160 of 12, 256 blocks
 # of more, four cells per lane, and just past what fits
-@pytest.mark.parametrize("n", [41664, 41665, 83329, 111105, 190465, 238081, 476161, 952320, 952321, 1015808, 1015809])
+@pytest.mark.parametrize("n", [40512, 40513, 82177, 108033, 187393, 236161, 473089, 949248, 949249, 1012736, 1012737])
 @pytest.mark.parametrize("flux,bc,arith", [(LF, PER, "fast"), (GOD, ZG, "fast"), (LF, ZG, "exact"), (GOD, PER, "exact")])
 def test_large(hh, dev, n, flux, bc, arith):
     same(run(hh, dev, n, flux, bc, 3, arith, 3, 3, False), run(hh, dev, n, flux, bc, 3, arith, 3, 3, True))
 
 
-@pytest.mark.parametrize("n", [40, 620, 621, 5000, 111105, 238081])
+@pytest.mark.parametrize("n", [40, 620, 621, 5000, 108033, 235009])
 @pytest.mark.parametrize("flux", [LF, GOD])
 @pytest.mark.parametrize("k,arith", [(2, "fast"), (3, "fast"), (3, "exact")])
 def test_nonuniform(hh, dev, n, flux, k, arith):

@@ -39,8 +39,29 @@ static void l1d_x(int flux, bool per, bool fast, bool amax, const Stage1DArgs &a
     if (flux == LF) l1d_p<K, LF>(per, fast, amax, a, s);
     else l1d_p<K, GODUNOV>(per, fast, amax, a, s);
 }
-// Rows per wavefront: the tuned value, else the fewest (at least 8) that let every wavefront
-// of the launch be resident at once.
+// Rows per wavefront of an untuned 2D launch.  A wavefront takes about ty + 1.5 row times (its
+// prologue reconstructs two rows); with w wavefronts on a SIMD a row takes 1, 1.4, 2, 2.7 times what
+// it takes alone (0.6 us FAST, 1.05 us EXACT: latency, then FP64 issue), and wavefronts past the
+// resident ones run in further turns.  The ty with the least (ty + 1.5) * that is taken; measured us
+// per stage with 8 rows at least, and so: 250 x 250 FAST 8.7, 5.1, EXACT 12.3, 6.2; 500 x 500 FAST
+// 9.1, 6.8; 1000 x 1000 FAST 15.1, 12.2, EXACT 23.9, 19.1; 2048 x 2048 as before (18 rows).
+static int rows_per_wave(int n2, int nstrips, int resident)
+{
+    const long long simds = 4LL * device_cus();
+    auto slowdown = [](long long w) { return w <= 1 ? 1.0 : (w == 2 ? 1.4 : 2.0 + 0.67 * (double)(w - 3)); };
+    int best = 1;
+    double least = 1e300;
+    for (int ty = 1; ty <= std::max(64, (int)(n2 * (long long)nstrips / (simds * resident)) + 1); ty = ty < 64 ? ty + 1 : ty + ty / 16) {
+        const long long w = ((long long)nstrips * ((n2 + ty - 1) / ty) + simds - 1) / simds;   // per SIMD
+        const double cost = (ty + 1.5) * ((double)(w / resident) * slowdown(resident) +
+                                          (w % resident ? slowdown(w % resident) : 0.0));
+        if (cost < least) {
+            least = cost;
+            best = ty;
+        }
+    }
+    return best;
+}
 template <int K, int BC, bool FAST>
 static void l2d(Stage2DArgs a, hipStream_t s)
 {
@@ -51,9 +72,7 @@ static void l2d(Stage2DArgs a, hipStream_t s)
                     hipSuccess || per_cu <= 0)
                 per_cu = 4;
         }
-        const long long slots = (long long)per_cu * device_cus() * (kBlock / 64);
-        const long long bands = std::max<long long>(1, slots / a.nstrips);
-        a.ty = (int)std::max<long long>(8, (a.n2 + bands - 1) / bands);
+        a.ty = rows_per_wave(a.n2, a.nstrips, per_cu);
     }
     const long long nsy = (a.n2 + a.ty - 1) / a.ty;
     const long long waves = nsy * a.nstrips;

@@ -1113,6 +1113,7 @@ struct hrw_ode_s {
     hrw_integrand_fn fu = nullptr;        // a callback integrand
     void *ctx = nullptr;
     hipStream_t stream = nullptr;
+    std::vector<double *> blocks;          // the allocations that hold every buffer below
     double *ui = nullptr, *ui2 = nullptr, *udot = nullptr;
     double *S = nullptr;                   // mstvd: current state
     double *ring_u[4] = {}, *ring_L[4] = {};
@@ -1164,37 +1165,54 @@ static void ms_tape_clear(hrw_ode_s *o, bool keep_storage = false)
 static int ode_free_adjoint(hrw_ode_s *o);
 hrw_ode_s::~hrw_ode_s()
 {
-    dfree(ui);
-    dfree(ui2);
-    dfree(udot);
-    dfree(S);
-    for (auto &b : ring_u) dfree(b);
-    for (auto &b : ring_L) dfree(b);
-    dfree(slots);
-    dfree(d_bad);
+    for (auto &b : blocks) dfree(b);
     ms_tape_clear(this);
     for (auto &b : ms_start) dfree(b);
     for (auto &b : ms_lam) dfree(b);
     ode_free_adjoint(this);
 }
 
+// The buffers in few allocations: a hipMalloc of more than 1 MiB and its hipFree cost tens of us,
+// whatever the size (hundreds with 11 of them, which a program that runs many short multistep
+// integrations pays for each object); smaller ones come from the runtime's pool for 1 us.  So small
+// buffers share blocks of up to 1 MiB and large ones one block.  udot: only an integrand callback
+// needs it; the exchange words: only a line of several blocks.
 static int ode_alloc(hrw_ode_s *o)
 {
-    CALL(dalloc(&o->ui, o->neq));
-    CALL(dalloc(&o->ui2, o->neq));
-    CALL(dalloc(&o->udot, o->neq));
-    if (o->method == METHOD_MS) {
-        CALL(dalloc(&o->S, o->neq));
-        for (auto &b : o->ring_u) CALL(dalloc(&b, o->neq));
-        for (auto &b : o->ring_L) CALL(dalloc(&b, o->neq));
-    }
-    // (the exchange words of a line of several blocks, behind the slots)
-    const bool exchange = o->p && o->method == METHOD_RK && o->p->kind == PROB_BURGERS1D && o->neq > 10 * kOutLanes;
+    const size_t state = ((size_t)o->neq + 31) / 32 * 32;   // 256-byte aligned
     const size_t slots = (size_t)3 * kNSlot * kSlotStride;
-    CALL(dalloc(&o->slots, slots + (exchange ? kResWords : 0)));
-    if (exchange) o->res_words = o->slots + slots;
-    CALL(dalloc(&o->d_bad, 1));
-    return HRW_OK;
+    const bool exchange = o->p && o->method == METHOD_RK && o->p->kind == PROB_BURGERS1D && o->neq > 10 * kOutLanes;
+    const size_t states = 2 + (o->fu ? 1 : 0) + (o->method == METHOD_MS ? 9 : 0);
+    const size_t all = states * state + slots + 32 + (exchange ? kResWords : 0), small = (1 << 20) / sizeof(double);
+    double *next = nullptr;
+    size_t left = 0, later = all;
+    int rc = HRW_OK;
+    auto take = [&](size_t count) -> double * {
+        if (count > left) {
+            left = state > small ? later : std::max(count, std::min(later, small));
+            next = nullptr;
+            if (rc == HRW_OK) rc = dalloc(&next, left);
+            if (rc != HRW_OK) return nullptr;
+            o->blocks.push_back(next);
+        }
+        double *q = next;
+        next += count;
+        left -= count;
+        later -= count;
+        return q;
+    };
+    o->ui = take(state);
+    o->ui2 = take(state);
+    if (o->fu) o->udot = take(state);
+    if (o->method == METHOD_MS) {
+        o->S = take(state);
+        for (auto &b : o->ring_u) b = take(state);
+        for (auto &b : o->ring_L) b = take(state);
+    }
+    o->slots = reinterpret_cast<unsigned long long *>(take(slots));
+    o->d_bad = reinterpret_cast<unsigned long long *>(take(32));
+    if (exchange) o->res_words = reinterpret_cast<unsigned long long *>(take(kResWords));
+    return rc;
 }
 
 static int ode_new(int method, int order, hrw_problem_s *p, hrw_integrand_fn fu, void *ctx,
@@ -1605,17 +1623,27 @@ static int ms_integrate(hrw_ode_s *o, double *u, double *t, double tout, double 
     if (o->istate == 1) {                              // :236-249, 4 RK3 starting steps
         if (rec) CALL(ms_record(o, o->S));
         int fe = 0;
-        for (int c = 4; c >= 1; --c) {
-            HIP_TRY(hipMemcpyAsync(o->ring_u[col(c)], o->S, bytes, hipMemcpyDeviceToDevice, o->stream));
-            CALL(ode_rhs(o, seq, *t, o->S, o->ring_L[col(c)]));
-            CALL(rk_step(o, seq, *t, dt, o->S, nullptr));   // order 3
-            if (rec) {   // the step's inner stage inputs (still in ui, ui2) and its result
-                const int q = 2 * (4 - c);
-                HIP_TRY(hipMemcpyAsync(o->ms_start[q], o->ui, bytes, hipMemcpyDeviceToDevice, o->stream));
-                HIP_TRY(hipMemcpyAsync(o->ms_start[q + 1], o->ui2, bytes, hipMemcpyDeviceToDevice, o->stream));
+        for (int c = 4; c >= 1 && !o->fu; --c) {
+            // fused: the first stage writes L(u_n) beside its result, and the last one u_{n+1} into
+            // the column's buffer, which then changes places with the state (recording: the inner
+            // stage inputs go straight to their place on the tape)
+            const int r = col(c), q = 2 * (4 - c);
+            double *y1 = rec ? o->ms_start[q] : o->ui, *y2 = rec ? o->ms_start[q + 1] : o->ui2;
+            CALL(ode_stage(o, seq, RK3_1, *t, dt, o->S, o->S, y1, nullptr, nullptr, o->ring_L[r]));
+            CALL(ode_stage(o, seq, RK3_2, *t + dt, dt, y1, o->S, y2));
+            CALL(ode_stage(o, seq, RK3_3, *t + dt / 2, dt, y2, o->S, o->ring_u[r]));
+            std::swap(o->S, o->ring_u[r]);
+            if (rec) {
                 CALL(ms_record(o, o->S));
                 o->ms_dts.push_back(dt);
             }
+            *t = *t + dt;
+            fe += 3;
+        }
+        for (int c = 4; c >= 1 && o->fu; --c) {
+            HIP_TRY(hipMemcpyAsync(o->ring_u[col(c)], o->S, bytes, hipMemcpyDeviceToDevice, o->stream));
+            CALL(ode_rhs(o, seq, *t, o->S, o->ring_L[col(c)]));
+            CALL(rk_step(o, seq, *t, dt, o->S, nullptr));   // order 3
             *t = *t + dt;
             fe += 3;
         }

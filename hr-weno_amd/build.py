@@ -37,6 +37,7 @@ UNITS = [
     ("launch_resident.hip", ["-DHRW_K=2"], "launch_resident_k2.o"),
     ("launch_resident.hip", ["-DHRW_K=3"], "launch_resident_k3.o"),
     ("launch_batch_resident.hip", [], "launch_batch_resident.o"),
+    ("launch_adjoint_resident.hip", [], "launch_adjoint_resident.o"),
     ("launch_kernels.hip", [], "launch_kernels.o"),
     ("launch_adjoint.hip", [], "launch_adjoint.o"),
 ]

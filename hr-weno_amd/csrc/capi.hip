@@ -68,6 +68,17 @@ static inline hipStream_t S(hrw_stream_t s) { return reinterpret_cast<hipStream_
 
 constexpr int kMaxDevices = 64;
 
+// Whether the stream is being captured (a capture would freeze what changes from launch to launch).
+static bool capturing(hipStream_t s)
+{
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cs) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    return cs != hipStreamCaptureStatusNone;
+}
+
 static bool is_done(double t, double tout, double dt)   // src/hrweno_tvdode.f90:273-284
 {
     return (t - tout) * std::copysign(1.0, dt) > 0.0;
@@ -1106,6 +1117,21 @@ static int gen_vjp(const hrw_problem_s *p, GenScratch &g, hipStream_t st, const 
 
 enum { METHOD_RK = 1, METHOD_MS = 2 };
 
+// What the launches whose blocks wait for each other need of an object (kernels_resident.hpp): the
+// exchange words (kResWords; none: one block only), the status word, the next exchange number,
+// whether both are clear, and the polls of a wait (about 0.2 s; HRW_RESIDENT_POLLS at the object's
+// creation sets them for tests).
+struct ResLink {
+    unsigned long long *words = nullptr, *status = nullptr;
+    unsigned tag = 0;
+    bool clear = false;
+    int polls = 1 << 18;
+    ResLink()
+    {
+        if (const char *e = std::getenv("HRW_RESIDENT_POLLS")) polls = std::atoi(e);
+    }
+};
+
 struct hrw_ode_s {
     int method = METHOD_RK, order = 3, fevals = 0, istate = 0, arith = HRW_ARITH_FAST;
     int64_t neq = 0;
@@ -1135,14 +1161,11 @@ struct hrw_ode_s {
     double *ms_lam[8] = {};
     GenScratch gen;
     bool check_finite = true;              // integrate ends with a scan of u for NaN/Inf
-    unsigned long long *d_bad = nullptr;   // the scan's result word
-    // whole-integration kernel: its exchange words (kResWords, behind the slots), the next exchange
-    // number, whether words and result word are clear, whether it ran in this call and its result's
-    // scan, the polls of a wait (about 0.2 s; HRW_RESIDENT_POLLS at creation sets them for tests)
-    unsigned long long *res_words = nullptr, res_bad = 0;
-    unsigned res_tag = 0;
-    bool res_clear = false, res_ran = false;
-    int res_polls = 1 << 18;
+    // whole-integration kernel (its status word is the scan's result word too), whether it ran in
+    // this call, and its scan of the result
+    ResLink link;
+    unsigned long long res_bad = 0;
+    bool res_ran = false;
     ~hrw_ode_s();
 };
 // Drop the recording; keep_storage: its blocks go to the pool for the next recording.
@@ -1210,8 +1233,8 @@ static int ode_alloc(hrw_ode_s *o)
         for (auto &b : o->ring_L) b = take(state);
     }
     o->slots = reinterpret_cast<unsigned long long *>(take(slots));
-    o->d_bad = reinterpret_cast<unsigned long long *>(take(32));
-    if (exchange) o->res_words = reinterpret_cast<unsigned long long *>(take(kResWords));
+    o->link.status = reinterpret_cast<unsigned long long *>(take(32));
+    if (exchange) o->link.words = reinterpret_cast<unsigned long long *>(take(kResWords));
     return rc;
 }
 
@@ -1238,7 +1261,6 @@ static int ode_new(int method, int order, hrw_problem_s *p, hrw_integrand_fn fu,
         return rc;
     }
     o->istate = 1;   // :93, :199
-    if (const char *e = std::getenv("HRW_RESIDENT_POLLS")) o->res_polls = std::atoi(e);
     *out = o;
     return HRW_OK;
 }
@@ -1366,11 +1388,11 @@ static int64_t count_steps(double &t, double tout, double dt)
 }
 
 // The result word of a scan or of the whole-integration kernel, once the stream is done.
-static int ode_read_status(hrw_ode_s *o, unsigned long long *bad)
+static int read_status(ResLink &l, unsigned long long *bad, hipStream_t s)
 {
-    HIP_TRY(hipMemcpyAsync(bad, o->d_bad, sizeof *bad, hipMemcpyDeviceToHost, o->stream));
-    HIP_TRY(hipStreamSynchronize(o->stream));
-    if (*bad) o->res_clear = false;   // cleared before the next whole-integration launch
+    HIP_TRY(hipMemcpyAsync(bad, l.status, sizeof *bad, hipMemcpyDeviceToHost, s));
+    HIP_TRY(hipStreamSynchronize(s));
+    if (*bad) l.clear = false;   // cleared before the next whole-integration launch
     return HRW_OK;
 }
 
@@ -1382,7 +1404,9 @@ static int ode_read_status(hrw_ode_s *o, unsigned long long *bad)
 // exchange) as long as it beats the exchange of several; then about 7 wavefronts of one cell per
 // lane per block, which hide each other's latency; more blocks cost alpha's exchange more (64:
 // 1.6 us, 128: 1.7, 256: 2.3), so with it and the FAST form, whose cells are cheap, two cells per
-// lane come in earlier.  False: the line does not fit.
+// lane come in earlier, and five before four take more than twelve wavefronts (900,000 cells: four
+// 5.1 us, 1,000,003: five 4.6; 1,150,000 4.6 / 9.7).  Eight take three wavefronts per SIMD
+// (1,300,000: 6.9 / 10.4; Godunov 5.7 / 8.4).  False: the line does not fit.
 static bool resident_split(long long n, int order, bool exact, bool amax, bool nonuniform, ResPlan *pl)
 {
     const int most_waves = kResThreads / 64;
@@ -1414,93 +1438,99 @@ static bool resident_split(long long n, int order, bool exact, bool amax, bool n
     };
     if (nonuniform) return several(1, 7, kResMaxBlocks) || widen(1, cap);
     if (amax && !exact)
-        return several(1, 7, 96) || several(2, 7, 96) || several(2, 12, 160) || widen(2, cap) || widen(4, cap);
-    return several(1, 7, kResMaxBlocks) || widen(1, exact ? 12 : cap) || widen(2, cap) || widen(4, cap);
+        return several(1, 7, 96) || several(2, 7, 96) || several(2, 12, 160) || widen(2, cap) || widen(4, 12) || widen(5, cap) || widen(8, 11);
+    return several(1, 7, kResMaxBlocks) || widen(1, exact ? 12 : cap) || widen(2, cap) || widen(4, cap) || (!exact && (widen(5, cap) || widen(8, amax ? 11 : 12)));
 }
 
-// Whether nsteps steps of o take it, and how.  Left to the launches per stage: problems tuned to a
+// Whether nsteps steps of p take it, and how.  Left to the launches per stage: problems tuned to a
 // kernel, cell widths without their coefficients and FAST lines far from the origin (the tile
 // kernel's arithmetic), and calls under stream capture.
-static bool resident_plan(const hrw_ode_s *o, int64_t nsteps, ResPlan *pl)
+static bool resident_plan(const hrw_problem_s *p, int order, int64_t nsteps, const ResLink &l, hipStream_t s, ResPlan *pl)
 {
-    const hrw_problem_s *p = o->p;
     if (p->kind != PROB_BURGERS1D || p->variant != 0 || p->cells_per_lane != 0) return false;
     const bool exact = p->arith != HRW_ARITH_FAST;
     if (!p->d_cnu && (p->d_width || (!exact && !near_linear_grid(p->xmin, p->rx, p->neq)))) return false;
-    if (p->neq < 8 || !resident_split(p->neq, o->order, exact, p->alphamax(), p->d_cnu != nullptr, pl)) return false;
+    if (p->neq < 8 || !resident_split(p->neq, order, exact, p->alphamax(), p->d_cnu != nullptr, pl)) return false;
     // (a launch's first stage must not be its last: blocks read each other's initial cells)
-    if (pl->blocks > device_cus() || (pl->blocks > 1 && !o->res_words) || nsteps * o->order < 2 || nsteps >= (1 << 26)) return false;
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(o->stream, &cs) != hipSuccess) {
-        (void)hipGetLastError();
-        return false;
-    }
-    return cs == hipStreamCaptureStatusNone;
+    if (pl->blocks > device_cus() || (pl->blocks > 1 && !l.words) || nsteps * order < 2 || nsteps >= (1 << 26)) return false;
+    return !capturing(s);
 }
 
 // Held while a launch whose blocks wait for each other is in flight on the device: two of them at
 // once could each hold CUs the other's missing blocks need.  A call that finds it taken (another
-// thread is in such an integrate) uses one launch per stage.
+// thread is in such a call) uses one launch per stage.
 static std::mutex g_resident_mu[kMaxDevices];
-
-// nsteps steps of o on u by resident_kernel.  *ran = false, and u as it was, when the device is
-// taken or refuses the launch, or when the blocks waited for each other in vain (another process's
-// kernels kept some of them off the device).
-static int rk_resident(hrw_ode_s *o, const ResPlan &pl, double *u, int64_t nsteps, double dt, bool *ran)
+static bool resident_alone(std::unique_lock<std::mutex> &lock)
 {
-    *ran = false;
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return false;
+    lock = std::unique_lock<std::mutex>(g_resident_mu[dev], std::try_to_lock);
+    return lock.owns_lock();
+}
+
+// A recording's buffers (ResArgs).
+struct ResTape {
+    double *states = nullptr, *alpha = nullptr;
+    long long stride = 0;
+};
+
+// nsteps steps of p from `in` to `out` (may be `in`) by resident_kernel; `saved` receives the
+// initial state.  *ran = false, and nothing written but `saved`, `out` and the recording, when the
+// device is taken or refuses the launch, or when the blocks waited for each other in vain (another
+// process's kernels kept some of them off the device).  *saved_in: `saved` was written.  `bad` null:
+// the state of one block's result is not asked for, and nothing waits for it.
+static int resident_run(const hrw_problem_s *p, int order, double dt, const ResPlan &pl, ResLink &l,
+                        const double *in, double *out, double *saved, int64_t nsteps, const ResTape &tape,
+                        hipStream_t s, unsigned long long *bad, bool *saved_in, bool *ran)
+{
+    *ran = *saved_in = false;
     std::unique_lock<std::mutex> alone;
-    if (pl.blocks > 1) {
-        int dev = 0;
-        HIP_TRY(hipGetDevice(&dev));
-        if (dev < 0 || dev >= kMaxDevices) return HRW_OK;
-        alone = std::unique_lock<std::mutex>(g_resident_mu[dev], std::try_to_lock);
-        if (!alone.owns_lock()) return HRW_OK;
-    }
-    const hrw_problem_s *p = o->p;
+    if (pl.blocks > 1 && !resident_alone(alone)) return HRW_OK;
     ResArgs a{};
-    a.u = u;
-    a.saved = o->ui;
+    a.in = in;
+    a.out = out;
+    a.saved = saved;
+    a.tape = tape.states;
+    a.tape_stride = tape.stride;
+    a.alpha_rec = tape.alpha;
     a.n = p->neq;
     a.M = (int)((p->neq + pl.blocks - 1) / pl.blocks);
-    a.order = o->order;
+    a.order = order;
     a.nsteps = (int)nsteps;
     a.periodic = p->bc == HRW_BC_PERIODIC;
     a.amax = p->alphamax();
     static const int stage_id[3][3] = {{RK1, RK1, RK1}, {RK2_1, RK2_2, RK2_2}, {RK3_1, RK3_2, RK3_3}};
-    for (int i = 0; i < 3; ++i) a.coef[i] = res_coef(stage_id[o->order - 1][i], dt);
+    for (int i = 0; i < 3; ++i) a.coef[i] = res_coef(stage_id[order - 1][i], dt);
     a.eps = p->eps;
     a.alpha = p->alpha;
     a.xmin = p->xmin;
     a.rx = p->rx;
     a.width = p->d_width;
     a.cnu = p->d_cnu;
-    a.words = o->res_words;
-    a.status = o->d_bad;
-    a.polls = o->res_polls;
-    const unsigned used = (unsigned)a.nsteps * (unsigned)o->order;
-    if (!o->res_clear || o->res_tag > 0xffffffffu - used) {
-        if (o->res_words)
-            fill_u64_kernel<<<grid_for((long long)kResWords, 256, 64), 256, 0, o->stream>>>(o->res_words, kResWords);
-        fill_u64_kernel<<<1, 64, 0, o->stream>>>(o->d_bad, 1);
-        o->res_tag = kResFirstTag;
-        o->res_clear = true;
+    a.words = l.words;
+    a.status = pl.blocks > 1 || bad ? l.status : nullptr;
+    a.polls = l.polls;
+    const unsigned used = (unsigned)a.nsteps * (unsigned)order;
+    if (!l.clear || l.tag > 0xffffffffu - used) {
+        if (l.words)
+            fill_u64_kernel<<<grid_for((long long)kResWords, 256, 64), 256, 0, s>>>(l.words, kResWords);
+        fill_u64_kernel<<<1, 64, 0, s>>>(l.status, 1);
+        l.tag = kResFirstTag;
+        l.clear = true;
     }
-    a.tag = o->res_tag;
-    o->res_tag += used;
+    a.tag = l.tag;
+    l.tag += used;
     const bool fast = p->arith == HRW_ARITH_FAST;
-    const hipError_t e = p->k == 1   ? launch_resident_k1(p->numflux, fast, pl, a, o->stream)
-                         : p->k == 2 ? launch_resident_k2(p->numflux, fast, pl, a, o->stream)
-                                     : launch_resident_k3(p->numflux, fast, pl, a, o->stream);
+    const hipError_t e = p->k == 1   ? launch_resident_k1(p->numflux, fast, pl, a, s)
+                         : p->k == 2 ? launch_resident_k2(p->numflux, fast, pl, a, s)
+                                     : launch_resident_k3(p->numflux, fast, pl, a, s);
     if (e != hipSuccess) return HRW_OK;   // (not launched)
-    unsigned long long bad = 0;
-    CALL(ode_read_status(o, &bad));
-    if (bad & RES_TIMEOUT) {
-        HIP_TRY(hipMemcpyAsync(u, o->ui, o->neq * sizeof(double), hipMemcpyDeviceToDevice, o->stream));
-        return HRW_OK;
-    }
-    *ran = o->res_ran = true;
-    o->res_bad = bad;
+    *saved_in = saved != nullptr;
+    unsigned long long word = 0;
+    if (a.status) CALL(read_status(l, &word, s));
+    if (word & RES_TIMEOUT) return HRW_OK;
+    if (bad) *bad = word;
+    *ran = true;
     return HRW_OK;
 }
 
@@ -1516,8 +1546,15 @@ static int rk_integrate(hrw_ode_s *o, double *u, double *t, double tout, double 
         const int64_t nsteps = count_steps(t1, tout, dt);
         ResPlan pl;
         bool ran = false;
-        if (resident_plan(o, nsteps, &pl)) CALL(rk_resident(o, pl, u, nsteps, dt, &ran));
+        if (resident_plan(o->p, o->order, nsteps, o->link, o->stream, &pl)) {
+            bool saved = false;
+            CALL(resident_run(o->p, o->order, dt, pl, o->link, u, u, pl.blocks > 1 ? o->ui : nullptr, nsteps, ResTape{},
+                              o->stream, &o->res_bad, &saved, &ran));
+            if (saved && !ran)
+                HIP_TRY(hipMemcpyAsync(u, o->ui, o->neq * sizeof(double), hipMemcpyDeviceToDevice, o->stream));
+        }
         if (ran) {
+            o->res_ran = true;
             *t = t1;
             o->fevals += o->order * (int)nsteps;
             if (o->istate == 1) o->istate = 2;         // :176
@@ -1740,10 +1777,10 @@ static int ode_check_finite(hrw_ode_s *o, const double *u)
 {
     unsigned long long bad = o->res_bad;
     if (!o->res_ran) {   // (else the integration has scanned its result)
-        fill_u64_kernel<<<1, 64, 0, o->stream>>>(o->d_bad, 1);
-        nonfinite_kernel<<<grid_for(o->neq, kBlock * 8, 4096), kBlock, 0, o->stream>>>(u, o->neq, o->d_bad);
+        fill_u64_kernel<<<1, 64, 0, o->stream>>>(o->link.status, 1);
+        nonfinite_kernel<<<grid_for(o->neq, kBlock * 8, 4096), kBlock, 0, o->stream>>>(u, o->neq, o->link.status);
         LAUNCH_CHECK();
-        CALL(ode_read_status(o, &bad));
+        CALL(read_status(o->link, &bad, o->stream));
     }
     if (bad) return fail(HRW_ERR_STATE, "non-finite state: u holds NaN or Inf after integrate");
     return HRW_OK;
@@ -2316,10 +2353,7 @@ extern "C" int hrw_batch_step(hrw_batch_t b, double *u, int64_t nsteps, double *
     if (((uintptr_t)u & 15u) != 0) return fail(HRW_ERR_ARG, "the batch state must be 16-byte aligned");
     if (nsteps == 0) return HRW_OK;
     BatchCall order(b);
-    // (a capture would freeze the exchange numbers)
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    const bool capturing = hipStreamIsCapturing(b->stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone;
-    if (b->resident && b->res_blocks > 0 && !capturing) {
+    if (b->resident && b->res_blocks > 0 && !capturing(b->stream)) {
         CALL(batch_resident_steps(b, u, nsteps));
     } else if (use_graph) {
         CALL(batch_seed(b, u));
@@ -2515,6 +2549,16 @@ struct hrw_adjoint_s {
     int64_t nsteps = 0, nseg = 0, flat = 0;
     double dt = 0.0;
     std::vector<double *> ckpt, Y;
+    double *ystore = nullptr;     // Y's storage, one block
+    long long ystride = 0;
+    ResLink link;                 // one line: the forward in one launch
+    double *link_store = nullptr;
+    // one line, every stage input kept: the reverse in one launch, its exchange words and the
+    // number of the last launch
+    AresPlan ares{};              // (blocks 0: it does not fit)
+    unsigned long long *ares_words = nullptr;
+    size_t ares_count = 0;
+    unsigned ares_tag = 0;
     double *lamA = nullptr, *lamB = nullptr;
     unsigned long long *sets = nullptr;
     size_t set_words = 0;
@@ -2565,8 +2609,8 @@ struct hrw_adjoint_s {
     {
         if (side) (void)hipStreamSynchronize(side);
         for (auto &c : ckpt) dfree(c);
-        for (auto &y : Y) dfree(y);
         for (auto &y : Y1) dfree(y);
+        dfree(ystore); dfree(link_store); dfree(ares_words);
         dfree(lamA); dfree(lamB); dfree(sets); dfree(alpha_rec);
         dfree(sets1); dfree(alpha_rec1); dfree(sink);
         if (ev_a) (void)hipEventDestroy(ev_a);
@@ -2618,6 +2662,49 @@ struct hrw_adjoint_s {
     }
 };
 
+// The adjoint covers the fused 1D Burgers problems on a linear grid, with either flux and either
+// kind of ends; periodic Lax-Friedrichs lines take the register-blocked reverse kernel
+// (adjoint_stage_kernel), the others the general pass (rhs_vjp_kernel).
+static bool adjoint_problem_ok(const hrw_problem_s *p)
+{
+    return p->kind == PROB_BURGERS1D && !p->d_width && !p->d_cnu;
+}
+static bool adjoint_fast_form(const hrw_problem_s *p)
+{
+    return p->bc == HRW_BC_PERIODIC && p->numflux == HRW_FLUX_LAX_FRIEDRICHS;
+}
+
+// How a line of n cells is split for the reverse in one launch: one block, or blocks of one or two
+// groups of four chunks, at most one per CU.  blocks = 0: it does not take it.  Measured on 10 RK3
+// steps, us per reversed stage against one launch per stage: Lax-Friedrichs with alpha = max|u| 300
+// cells 2.6 / 7.6, 5000 4.8 / 7.7, 100,000 5.7 / 7.9, 200,000 6.2 / 7.9; Godunov 1.7 / 4.3, 3.0 /
+// 4.8, 3.1 / 4.9, 4.0 / 5.5.  Beyond two groups per block a wavefront has several chunks in turn,
+// and a stage takes what the launch takes (2^20 cells 16.2 / 16.5): those lines are left to it.
+static AresPlan ares_split(long long n, bool lfp, bool amax)
+{
+    AresPlan pl{};
+    const int chunk = lfp ? kAresChunk<true> : kAresChunk<false>;
+    const long long nc = (n + chunk - 1) / chunk, groups = (nc + 3) / 4;
+    pl.units = (int)(lfp ? nc / 4 + nc % 4 : groups);
+    if (nc <= kAresWaves) {
+        pl.blocks = 1;
+        pl.M = groups * 4 * chunk;
+        pl.chunks = (int)nc;
+    } else {
+        // (a last block of one or two cells, fewer than are exchanged, would need a wavefront more
+        // in the block before: that split is left)
+        const int most = std::min(kResMaxBlocks, device_cus());
+        for (int g = 1; g <= 2 && !pl.blocks; ++g) {
+            pl.M = 4LL * g * chunk;
+            pl.chunks = 4 * g;
+            const long long nb = (n + pl.M - 1) / pl.M;
+            if (nb <= most && n - (nb - 1) * pl.M >= kAresHalo) pl.blocks = (int)nb;
+        }
+    }
+    pl.lds = ares_lds_bytes(pl.chunks, chunk, pl.units, amax);
+    return pl;
+}
+
 static int adjoint_chunks(hrw_adjoint_s *a, const std::vector<int> &ncells);
 static int adjoint_alloc(hrw_adjoint_s *a, const std::vector<int> &ncells)
 {
@@ -2626,7 +2713,24 @@ static int adjoint_alloc(hrw_adjoint_s *a, const std::vector<int> &ncells)
     for (auto &c : a->ckpt) CALL(dalloc(&c, (size_t)a->flat));
     const int ny = a->nsteps > 0 ? a->order * a->m - 1 : 0;
     a->Y.assign((size_t)ny, nullptr);
-    for (auto &y : a->Y) CALL(dalloc(&y, (size_t)a->flat));
+    a->ystride = (a->flat + 31) / 32 * 32;
+    CALL(dalloc(&a->ystore, std::max<size_t>(1, (size_t)ny * (size_t)a->ystride)));
+    for (int i = 0; i < ny; ++i) a->Y[(size_t)i] = a->ystore + (long long)i * a->ystride;
+    if (!a->b) {   // (exchange words: only a line of several blocks)
+        const size_t words = a->flat > 10 * kOutLanes ? kResWords : 0;
+        CALL(dalloc(&a->link_store, 32 + words));
+        a->link.status = reinterpret_cast<unsigned long long *>(a->link_store);
+        if (words) a->link.words = a->link.status + 32;
+        const int64_t stages = a->nsteps * a->order;
+        if (a->nseg == 1 && a->p->k >= 2 && a->flat >= 16 && stages >= 2 && stages < (1 << 28))
+            a->ares = ares_split(a->flat, adjoint_fast_form(a->p), a->alphamax());
+        if (a->ares.blocks > 1) {
+            a->ares_count = (size_t)stages * ((size_t)a->ares.blocks * kAresLine + (a->alphamax() ? 2 * (size_t)a->ares.units : 0));
+            CALL(dalloc(&a->ares_words, a->ares_count));
+            fill_u64_kernel<<<grid_for((long long)a->ares_count, 256, 4096), 256>>>(a->ares_words, (long long)a->ares_count);
+            LAUNCH_CHECK();
+        }
+    }
     CALL(dalloc(&a->lamA, (size_t)a->flat));
     CALL(dalloc(&a->lamB, (size_t)a->flat));
     a->set_words = a->b ? (size_t)a->b->nlines : (size_t)kNSlot * kSlotStride;
@@ -2728,17 +2832,6 @@ static int auto_ckpt(int64_t nsteps, int order, int64_t flat)
     return (int)lo;
 }
 
-// The adjoint covers the fused 1D Burgers problems on a linear grid, with either flux and either
-// kind of ends; periodic Lax-Friedrichs lines take the register-blocked reverse kernel
-// (adjoint_stage_kernel), the others the general pass (rhs_vjp_kernel).
-static bool adjoint_problem_ok(const hrw_problem_s *p)
-{
-    return p->kind == PROB_BURGERS1D && !p->d_width && !p->d_cnu;
-}
-static bool adjoint_fast_form(const hrw_problem_s *p)
-{
-    return p->bc == HRW_BC_PERIODIC && p->numflux == HRW_FLUX_LAX_FRIEDRICHS;
-}
 static const char *kAdjointCovers = "the adjoint covers 1D Burgers problems on a linear grid";
 
 extern "C" int hrw_adjoint_create(hrw_problem_t p, int order, double dt, int64_t nsteps,
@@ -2944,8 +3037,23 @@ extern "C" int hrw_adjoint_forward(hrw_adjoint_t a, const double *u0, double *uN
     hipStream_t s = a->strm();
     std::unique_ptr<BatchCall> order(a->b ? new BatchCall(a->b) : nullptr);
     if (a->side) HIP_TRY(hipStreamSynchronize(a->side));   // (idle unless a call failed midway)
-    HIP_TRY(hipMemcpyAsync(a->ckpt[0], u0, bytes, hipMemcpyDeviceToDevice, s));
     a->recorded = false;
+    ResPlan pl;
+    bool saved = false;
+    if (!a->b && a->nseg == 1 && resident_plan(a->p, a->order, a->nsteps, a->link, s, &pl)) {
+        // the recording keeps every stage input: they and their alphas come out of one launch
+        // (ckpt[1], u_N again, is read by no reverse)
+        bool ran = false;
+        const ResTape tape{a->ystore, a->arec(0), a->ystride};
+        CALL(resident_run(a->p, a->order, a->dt, pl, a->link, u0, uN, a->ckpt[0], a->nsteps, tape, s, nullptr, &saved, &ran));
+        if (ran) {
+            a->buf_seg[0] = 0;
+            a->buf_seg[1] = -1;
+            a->recorded = true;
+            return HRW_OK;
+        }
+    }
+    if (!saved) HIP_TRY(hipMemcpyAsync(a->ckpt[0], u0, bytes, hipMemcpyDeviceToDevice, s));
     for (int64_t g = 0; g < a->nseg; ++g) CALL(adjoint_segment(a, g, true, 0, s));
     a->buf_seg[0] = a->nseg - 1;
     a->buf_seg[1] = -1;
@@ -3024,6 +3132,64 @@ static int adjoint_stage(hrw_adjoint_s *a, int64_t s, int64_t q, int k, const do
     return HRW_OK;
 }
 
+// The reverse of the whole recording from gN to g0 (may be gN) in one launch.  *ran = false when it
+// does not take it, or when the blocks waited in vain: gN is then in lamA if *saved.
+static int adjoint_resident(hrw_adjoint_s *a, const double *gN, double *g0, bool *saved, bool *ran)
+{
+    *ran = *saved = false;
+    const AresPlan &pl = a->ares;
+    const hrw_problem_s *p = a->p;
+    if (!pl.blocks || a->R != 2 || p->variant != 0 || p->cells_per_lane != 0 || pl.blocks > device_cus() ||
+        capturing(a->stream))
+        return HRW_OK;
+    std::unique_lock<std::mutex> alone;
+    if (pl.blocks > 1 && !resident_alone(alone)) return HRW_OK;
+    AresArgs g{};
+    g.x0 = a->ckpt[0];
+    g.tape = a->ystore;
+    g.tape_stride = a->ystride;
+    g.alpha_rec = a->arec(0);
+    g.g = gN;
+    g.out = g0;
+    g.saved = a->lamA;
+    g.n = p->neq;
+    g.M = (int)pl.M;
+    g.chunks = pl.chunks;
+    g.order = a->order;
+    g.nsteps = (int)a->nsteps;
+    g.periodic = p->bc == HRW_BC_PERIODIC;
+    g.constw = exact_linear_grid(p->xmin, p->rx, p->neq) ? 1 : 0;
+    g.eps = p->eps;
+    g.alpha = p->alpha;
+    g.xmin = p->xmin;
+    g.rx = p->rx;
+    g.dt = a->dt;
+    g.words = a->ares_words;
+    g.units = pl.units;
+    g.status = a->link.status;
+    g.polls = a->link.polls;
+    if (pl.blocks > 1) {
+        if (!a->link.clear) {
+            if (a->link.words)
+                fill_u64_kernel<<<grid_for((long long)kResWords, 256, 64), 256, 0, a->stream>>>(a->link.words, kResWords);
+            fill_u64_kernel<<<1, 64, 0, a->stream>>>(a->link.status, 1);
+            a->link.tag = kResFirstTag;
+            a->link.clear = true;
+        }
+        if (a->ares_tag == 0xffffffffu) {
+            fill_u64_kernel<<<grid_for((long long)a->ares_count, 256, 4096), 256, 0, a->stream>>>(a->ares_words, (long long)a->ares_count);
+            a->ares_tag = 0;
+        }
+        g.tag = ++a->ares_tag;
+    }
+    if (launch_adjoint_resident(p->k, !a->general, p->numflux, p->alphamax(), pl, g, a->stream) != hipSuccess) return HRW_OK;
+    *saved = true;
+    unsigned long long word = 0;
+    if (pl.blocks > 1) CALL(read_status(a->link, &word, a->stream));
+    *ran = !(word & RES_TIMEOUT);
+    return HRW_OK;
+}
+
 extern "C" int hrw_adjoint_backward(hrw_adjoint_t a, const double *gN, double *g0)
 {
     if (!a) return fail(HRW_ERR_ARG, "null adjoint");
@@ -3036,6 +3202,12 @@ extern "C" int hrw_adjoint_backward(hrw_adjoint_t a, const double *gN, double *g
     double *lam = g0, *A = a->lamA, *B = a->lamB;
     a->owed.clear();
     if (a->side) HIP_TRY(hipStreamSynchronize(a->side));   // (idle unless a call failed midway)
+    if (!a->b && a->nseg == 1) {
+        bool saved = false, ran = false;
+        CALL(adjoint_resident(a, gN, g0, &saved, &ran));
+        if (ran) return HRW_OK;
+        if (saved) gN = A;
+    }
     if (gN != g0) HIP_TRY(hipMemcpyAsync(g0, gN, bytes, hipMemcpyDeviceToDevice, st));
     // With two stage-input buffers the segments' recomputation overlaps the reverse: while
     // segment s is reversed from buffer k on st, segment s-1 is recomputed into the other on the

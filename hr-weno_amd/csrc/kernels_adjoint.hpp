@@ -224,15 +224,19 @@ __device__ __forceinline__ PendAt pend_at(unsigned tag, const LineRec &r, int i)
     return PendAt{khi == tag ? (int)(0xffffffffu - klo) : -1, d};
 }
 
-// Reverse of one K = 3 reconstruction of cell i from its window x[0..4] = v_{i-2..i+2}.  The
-// cotangents of the two faces come from face_cot(vr, vl, ir, il, sgr, sgl), which sets
-// sgr = vr-bar * ir and sgl = vl-bar * il (ir, il: the reciprocals of the two sums of weights,
-// sr = 6 sum_r (d_r Q_r), vr = nr/sr).  The triple pieces are rebuilt from the window for each
-// cell (cheaper in registers than carrying them between cells).  The window cotangent is added
-// to acc[0..4].
-template <class FaceCot>
-__device__ __forceinline__ void weno5_vjp(double eps12, const double *x, FaceCot &&face_cot,
-                                          double *acc)
+// Reverse of one K = 3 reconstruction of cell i from its window x[0..4] = v_{i-2..i+2}, in two
+// parts: what the window alone gives, and the window cotangent from the faces' cotangents.  The
+// triple pieces are rebuilt from the window for each cell (cheaper in registers than carrying them
+// between cells).
+struct Weno5Rev {
+    double vr, vl, ir, il;            // the faces, and the reciprocals of their two sums of weights,
+                                      // sr = 6 sum_r (d_r Q_r), vr = nr/sr
+    double a0, a1, m0, m2, l2;        // the weights' numerators (right a0, a1, m2; left m0, a1, l2)
+    double dr0, dr1, dr2, dl0, dl1, dl2;   // 6x candidate minus 6x face
+    double P0, P1, P2;                // -4/p_r
+    double t0, t1, t2, x0, e1, y2;    // 13 D, 3 X, 3 E, 3 Y of the indicators
+};
+__device__ __forceinline__ void weno5_rev_window(double eps12, const double *x, Weno5Rev &w)
 {
     // T(i-2) = x0..x2 (beta_2, right cand P2, left cand P1), T(i-1) = x1..x3 (beta_1, P1, P0),
     // T(i) = x2..x4 (beta_0, P0, Pm); with D = a - 2b + c, E = a - c:
@@ -243,11 +247,11 @@ __device__ __forceinline__ void weno5_vjp(double eps12, const double *x, FaceCot
     const double Y2 = fma_(2.0, D2, -E2), X0 = fma_(2.0, D0, E0);
     // (13 D and 3 Y, 3 E, 3 X are kept for the reverse: 26 D pb = 13 D (2 pb) and 6 Y pb =
     // 3 Y (2 pb) exactly, with 2 pb formed directly below)
-    const double t2 = 13.0 * D2, t1 = 13.0 * D1, t0 = 13.0 * D0;
-    const double y2 = 3.0 * Y2, e1 = 3.0 * E1, x0 = 3.0 * X0;
-    const double p2 = eps12 + fma_(y2, Y2, t2 * D2);
-    const double p1 = eps12 + fma_(e1, E1, t1 * D1);
-    const double p0 = eps12 + fma_(x0, X0, t0 * D0);
+    w.t2 = 13.0 * D2, w.t1 = 13.0 * D1, w.t0 = 13.0 * D0;
+    w.y2 = 3.0 * Y2, w.e1 = 3.0 * E1, w.x0 = 3.0 * X0;
+    const double p2 = eps12 + fma_(w.y2, Y2, w.t2 * D2);
+    const double p1 = eps12 + fma_(w.e1, E1, w.t1 * D1);
+    const double p0 = eps12 + fma_(w.x0, X0, w.t0 * D0);
     // 6x candidates: right P0(T(i)), P1(T(i-1)), P2(T(i-2)); left Pm(T(i)), P0(T(i-1)), P1(T(i-2))
     const double cr0 = fma_(5.0, x[3], fma_(2.0, x[2], -x[4]));
     const double cr1 = fma_(5.0, x[2], fma_(2.0, x[3], -x[1]));
@@ -256,46 +260,62 @@ __device__ __forceinline__ void weno5_vjp(double eps12, const double *x, FaceCot
     const double cl1 = fma_(5.0, x[2], fma_(2.0, x[1], -x[3]));
     const double cl2 = fma_(5.0, x[1], fma_(2.0, x[2], -x[0]));
     const double Q0 = p0 * p0, Q1 = p1 * p1, Q2 = p2 * p2;
-    const double m0 = Q1 * Q2, m1 = Q0 * Q2, m2 = Q0 * Q1;
-    const double a0 = 3.0 * m0, a1 = 6.0 * m1, l2 = 3.0 * m2;
-    const double sr = 6.0 * (a0 + a1 + m2), sl = 6.0 * (m0 + a1 + l2);
+    const double m1 = Q0 * Q2;
+    w.m0 = Q1 * Q2, w.m2 = Q0 * Q1;
+    w.a0 = 3.0 * w.m0, w.a1 = 6.0 * m1, w.l2 = 3.0 * w.m2;
+    const double sr = 6.0 * (w.a0 + w.a1 + w.m2), sl = 6.0 * (w.m0 + w.a1 + w.l2);
     // one reciprocal for both faces (sr and sl lie within a factor 3 of each other; see recon3)
     const double i2 = rcp_nr(sr * sl);
-    const double ir = sl * i2, il = sr * i2;
-    const double vr = fma_(a0, cr0, fma_(a1, cr1, m2 * cr2)) * ir;
-    const double vl = fma_(m0, cl0, fma_(a1, cl1, l2 * cl2)) * il;
-    double sgr, sgl;
-    face_cot(vr, vl, ir, il, sgr, sgl);
-    const double vr6 = 6.0 * vr, vl6 = 6.0 * vl;
-    // twice the cotangent of p_r = 12 (eps + beta_r):  -4/p_r [ w-numerator_r sgr (cr_r - 6vr) + ... ]
+    w.ir = sl * i2, w.il = sr * i2;
+    w.vr = fma_(w.a0, cr0, fma_(w.a1, cr1, w.m2 * cr2)) * w.ir;
+    w.vl = fma_(w.m0, cl0, fma_(w.a1, cl1, w.l2 * cl2)) * w.il;
+    const double vr6 = 6.0 * w.vr, vl6 = 6.0 * w.vl;
+    w.dr0 = cr0 - vr6, w.dr1 = cr1 - vr6, w.dr2 = cr2 - vr6;
+    w.dl0 = cl0 - vl6, w.dl1 = cl1 - vl6, w.dl2 = cl2 - vl6;
     const double ipi = -4.0 * rcp_nr(p0 * p1 * p2);
-    const double pb0 = (p1 * p2 * ipi) * fma_(a0 * sgr, cr0 - vr6, (m0 * sgl) * (cl0 - vl6));
-    const double pb1 = (p0 * p2 * ipi) * fma_(a1 * sgr, cr1 - vr6, (a1 * sgl) * (cl1 - vl6));
-    const double pb2 = (p0 * p1 * ipi) * fma_(m2 * sgr, cr2 - vr6, (l2 * sgl) * (cl2 - vl6));
+    w.P0 = p1 * p2 * ipi, w.P1 = p0 * p2 * ipi, w.P2 = p0 * p1 * ipi;
+}
+// sgr = vr-bar * ir, sgl = vl-bar * il; the window cotangent is added to acc[0..4].
+__device__ __forceinline__ void weno5_rev_apply(const Weno5Rev &w, double sgr, double sgl, double *acc)
+{
+    // twice the cotangent of p_r = 12 (eps + beta_r):  -4/p_r [ w-numerator_r sgr (cr_r - 6vr) + ... ]
+    const double pb0 = w.P0 * fma_(w.a0 * sgr, w.dr0, (w.m0 * sgl) * w.dl0);
+    const double pb1 = w.P1 * fma_(w.a1 * sgr, w.dr1, (w.a1 * sgl) * w.dl1);
+    const double pb2 = w.P2 * fma_(w.m2 * sgr, w.dr2, (w.l2 * sgl) * w.dl2);
     // T(i-2): beta_2 (D, Y = 2D - E), candidates P2 (right, m2) and P1 (left, l2)
     {
-        const double Db = t2 * pb2, Yb = y2 * pb2;
-        const double Pr = m2 * sgr, Pl = l2 * sgl;
+        const double Db = w.t2 * pb2, Yb = w.y2 * pb2;
+        const double Pr = w.m2 * sgr, Pl = w.l2 * sgl;
         acc[0] += fma_(2.0, Pr, Db + Yb - Pl);
         acc[1] += fma_(-7.0, Pr, fma_(5.0, Pl, fma_(-4.0, Yb, -2.0 * Db)));
         acc[2] += fma_(11.0, Pr, fma_(2.0, Pl, fma_(3.0, Yb, Db)));
     }
     // T(i-1): beta_1 (D, E), candidates P1 (right, a1) and P0 (left, a1)
     {
-        const double Db = t1 * pb1, Eb = e1 * pb1;
-        const double Pr = a1 * sgr, Pl = a1 * sgl;
+        const double Db = w.t1 * pb1, Eb = w.e1 * pb1;
+        const double Pr = w.a1 * sgr, Pl = w.a1 * sgl;
         acc[1] += fma_(2.0, Pl, Db + Eb - Pr);
         acc[2] += fma_(5.0, Pr + Pl, -2.0 * Db);
         acc[3] += fma_(2.0, Pr, Db - Eb - Pl);
     }
     // T(i): beta_0 (D, X = 2D + E), candidates P0 (right, a0) and Pm (left, m0)
     {
-        const double Db = t0 * pb0, Xb = x0 * pb0;
-        const double Pr = a0 * sgr, Pl = m0 * sgl;
+        const double Db = w.t0 * pb0, Xb = w.x0 * pb0;
+        const double Pr = w.a0 * sgr, Pl = w.m0 * sgl;
         acc[2] += fma_(11.0, Pl, fma_(2.0, Pr, fma_(3.0, Xb, Db)));
         acc[3] += fma_(-7.0, Pl, fma_(5.0, Pr, fma_(-4.0, Xb, -2.0 * Db)));
         acc[4] += fma_(2.0, Pl, Db + Xb - Pr);
     }
+}
+// Both parts: face_cot(vr, vl, ir, il, sgr, sgl) gives the cotangents.
+template <class FaceCot>
+__device__ __forceinline__ void weno5_vjp(double eps12, const double *x, FaceCot &&face_cot, double *acc)
+{
+    Weno5Rev w;
+    weno5_rev_window(eps12, x, w);
+    double sgr, sgl;
+    face_cot(w.vr, w.vl, w.ir, w.il, sgr, sgl);
+    weno5_rev_apply(w, sgr, sgl, acc);
 }
 
 // The Lax-Friedrichs form, for the halved flux cotangents phi3 = (phi_{i-1}, phi_i, phi_{i+1}),
@@ -316,43 +336,62 @@ __device__ __forceinline__ double recon3_vjp(double eps12, const double *x, cons
     return abar;
 }
 
-// Reverse of one K = 2 reconstruction from the pairs (v_{i-1}, v_i) and (v_i, v_{i+1});
-// acc[0..2] = cells i-1..i+1.  The cotangents of the faces come from face_cot as for weno5_vjp.
-template <class FaceCot>
-__device__ __forceinline__ void weno3_vjp(double eps, const Pair2 &p1, const Pair2 &p0,
-                                          FaceCot &&face_cot, double *acc)
+// Reverse of one K = 2 reconstruction from the pairs (v_{i-1}, v_i) and (v_i, v_{i+1}), in two
+// parts as for K = 3; acc[0..2] = cells i-1..i+1.
+struct Weno3Rev {
+    double vr, vl, ir, il;
+    double a0, b1, Q0, Q1;            // the weights' numerators (right a0, Q0; left Q1, b1)
+    double dr0, dr1, dl0, dl1;        // 2x candidate minus 2x face
+    double P0, P1;                    // -2/q_r
+    double d0, d1;                    // 2 (b - a) of the pairs
+};
+__device__ __forceinline__ void weno3_rev_window(double eps, const Pair2 &p1, const Pair2 &p0, Weno3Rev &w)
 {
     const double q0 = eps + p0.B, q1 = eps + p1.B;
-    const double Q0 = q0 * q0, Q1 = q1 * q1;
-    const double a0 = 2.0 * Q1, b1 = 2.0 * Q0;
-    const double sr = 2.0 * (a0 + Q0), sl = 2.0 * (Q1 + b1);
-    const double nr = fma_(a0, p0.S, Q0 * p1.Rr);
-    const double nl = fma_(Q1, p0.Lr, b1 * p1.S);
-    const double ir = rcp_nr(sr), il = rcp_nr(sl);
-    const double vr = nr * ir;
-    const double vl = nl * il;
-    double sgr, sgl;
-    face_cot(vr, vl, ir, il, sgr, sgl);
-    const double vr2 = 2.0 * vr, vl2 = 2.0 * vl;
+    w.Q0 = q0 * q0, w.Q1 = q1 * q1;
+    w.a0 = 2.0 * w.Q1, w.b1 = 2.0 * w.Q0;
+    const double sr = 2.0 * (w.a0 + w.Q0), sl = 2.0 * (w.Q1 + w.b1);
+    const double nr = fma_(w.a0, p0.S, w.Q0 * p1.Rr);
+    const double nl = fma_(w.Q1, p0.Lr, w.b1 * p1.S);
+    w.ir = rcp_nr(sr), w.il = rcp_nr(sl);
+    w.vr = nr * w.ir;
+    w.vl = nl * w.il;
+    const double vr2 = 2.0 * w.vr, vl2 = 2.0 * w.vl;
+    w.dr0 = p0.S - vr2, w.dr1 = p1.Rr - vr2;
+    w.dl0 = p0.Lr - vl2, w.dl1 = p1.S - vl2;
     const double iq = rcp_nr(q0 * q1);
-    // q-bar_r = -2/q_r [ (2x right weight numerator) sgr (cand - 2vr) + ... ]
-    const double qb0 = -2.0 * q1 * iq * fma_(a0 * sgr, p0.S - vr2, (Q1 * sgl) * (p0.Lr - vl2));
-    const double qb1 = -2.0 * q0 * iq * fma_(Q0 * sgr, p1.Rr - vr2, (b1 * sgl) * (p1.S - vl2));
+    w.P0 = -2.0 * q1 * iq, w.P1 = -2.0 * q0 * iq;
     // beta = d^2 with d = b - a = (Rr - S)/2, so d-bar = 2 d q-bar moves -1 to a, +1 to b
+    w.d0 = p0.Rr - p0.S, w.d1 = p1.Rr - p1.S;
+}
+__device__ __forceinline__ void weno3_rev_apply(const Weno3Rev &w, double sgr, double sgl, double *acc)
+{
+    // q-bar_r = -2/q_r [ (2x right weight numerator) sgr (cand - 2vr) + ... ]
+    const double qb0 = w.P0 * fma_(w.a0 * sgr, w.dr0, (w.Q1 * sgl) * w.dl0);
+    const double qb1 = w.P1 * fma_(w.Q0 * sgr, w.dr1, (w.b1 * sgl) * w.dl1);
     // pair (v_i, v_{i+1}): S = a+b, Lr = 3a-b
     {
-        const double Sb = a0 * sgr, Lb = Q1 * sgl;
-        const double dd = (p0.Rr - p0.S) * qb0;
+        const double Sb = w.a0 * sgr, Lb = w.Q1 * sgl;
+        const double dd = w.d0 * qb0;
         acc[1] += fma_(3.0, Lb, Sb - dd);
         acc[2] += Sb - Lb + dd;
     }
     // pair (v_{i-1}, v_i): Rr = 3b-a, S = a+b
     {
-        const double Rb = Q0 * sgr, Sb = b1 * sgl;
-        const double dd = (p1.Rr - p1.S) * qb1;
+        const double Rb = w.Q0 * sgr, Sb = w.b1 * sgl;
+        const double dd = w.d1 * qb1;
         acc[0] += Sb - Rb - dd;
         acc[1] += fma_(3.0, Rb, Sb + dd);
     }
+}
+template <class FaceCot>
+__device__ __forceinline__ void weno3_vjp(double eps, const Pair2 &p1, const Pair2 &p0, FaceCot &&face_cot, double *acc)
+{
+    Weno3Rev w;
+    weno3_rev_window(eps, p1, p0, w);
+    double sgr, sgl;
+    face_cot(w.vr, w.vl, w.ir, w.il, sgr, sgl);
+    weno3_rev_apply(w, sgr, sgl, acc);
 }
 
 // The Lax-Friedrichs form (halved phi3 as for recon3_vjp); abar = the cell's share of alpha-bar.

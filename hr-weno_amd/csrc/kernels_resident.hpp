@@ -70,8 +70,8 @@ __host__ __device__ inline ResCoef res_coef(int stage, double h)
 }
 
 struct ResArgs {
-    double *u;                     // state, read at the start and written at the end
-    double *saved;                 // several blocks: receives the initial state
+    const double *in;              // initial state
+    double *saved;                 // receives the initial state, or nullptr
     long long n;
     int M;                         // cells per block (the last block: what is left, >= kResEdge)
     int order, nsteps, periodic, amax;
@@ -82,11 +82,18 @@ struct ResArgs {
     unsigned long long *status;
     unsigned tag;                  // number of the first exchange (>= kResFirstTag)
     int polls;
+    double *out;                   // final state (may be in)
+    // recording: the output of stage q, but the last, at tape + q*tape_stride, and the alpha of
+    // stage q at alpha_rec[q]; or nullptr
+    double *tape, *alpha_rec;
+    long long tape_stride;
 };
 
 // A block's part of a line: cells [base, base + m) of n, and whom it exchanges with.
 struct ResPart {
-    double *u, *saved;             // the line; saved: receives the initial state, or nullptr
+    const double *in;              // the line
+    double *out, *saved, *tape, *alpha_rec;   // as in ResArgs
+    long long tape_stride;
     long long n, base;
     int m, order, nsteps;
     bool per, amax;
@@ -282,8 +289,8 @@ template <int R> constexpr size_t res_lds_bytes(int waves) { return 2 * (size_t)
 
 // The block's part: `waves` wavefronts that own cells; with ONE false and alpha = max|u| one more
 // takes part, and `threads` counts them all.  lds, s_mx (4 words) and s_alpha: the block's LDS.  A
-// wait in vain leaves NaN behind.
-template <int K, int FLUX, bool FAST, bool CNU, int R, bool ONE, int GROUP>
+// wait in vain leaves NaN behind.  REC: the stages and their alphas are recorded.
+template <int K, int FLUX, bool FAST, bool CNU, int R, bool ONE, int GROUP, bool REC>
 __device__ __forceinline__ void resident_part(const ResPart &a, const ResCoef *coef, int waves, int threads,
                                               double *lds, unsigned long long *s_mx, double *s_alpha)
 {
@@ -307,12 +314,13 @@ __device__ __forceinline__ void resident_part(const ResPart &a, const ResCoef *c
     if (tid < 4) s_mx[tid] = 0ull;
     __syncthreads();
     double x0 = 0.0;
+    bool nan = false;
     for (int j0 = tid - width; j0 < m + width; j0 += (R + 1) * threads) {
         double x[R + 1];
 #pragma unroll
         for (int i = 0; i <= R; ++i) {
             const int j = j0 + i * threads;
-            if (j < m + width) x[i] = a.u[line_cell(base + j, a.n, per)];
+            if (j < m + width) x[i] = a.in[line_cell(base + j, a.n, per)];
         }
 #pragma unroll
         for (int i = 0; i <= R; ++i) {
@@ -321,13 +329,16 @@ __device__ __forceinline__ void resident_part(const ResPart &a, const ResCoef *c
             cur[j] = x[i];
             if (j >= 0 && j < m) {
                 x0 = max_f64(x0, fabs(x[i]));
-                if (!ONE && a.saved) a.saved[base + j] = x[i];
+                nan |= x[i] != x[i];
+                if (a.saved) a.saved[base + j] = x[i];
             }
         }
     }
     if (amax) {
         x0 = row_max(x0);
         if ((lane & 15) == 15) lds_max(&s_mx[0], x0);
+        // (v_max_f64 passes a NaN over; with alpha infinite no flux of the line is finite either)
+        if (__any(nan)) lds_max(&s_mx[0], __builtin_inf());
     }
 
     // what does not change with the steps: cell widths (FAST: their reciprocals), the non-uniform
@@ -383,6 +394,10 @@ __device__ __forceinline__ void resident_part(const ResPart &a, const ResCoef *c
             }
             __syncthreads();
         }
+        if (REC && !comm && q > 0) {   // (from the LDS copy: whole lines of memory at a time)
+            double *y = a.tape + (long long)(q - 1) * a.tape_stride + base;
+            for (int j = tid; j < m; j += 64 * waves) y[j] = cur[j];
+        }
         double v[R + 2 * H], vl[R], vr[R], vr_left = 0.0, vl_right = 0.0;
         if (!comm) {
             if constexpr (!ONE) {
@@ -419,6 +434,7 @@ __device__ __forceinline__ void resident_part(const ResPart &a, const ResCoef *c
             if (q + 1 == stages) break;
             continue;
         }
+        if (REC && amax && base == 0 && tid == 0) a.alpha_rec[q] = alpha;
         double f[R + 1], un[R];
         f[0] = face_flux<K, FLUX, FAST, CNU>(vr_left, vl[0], alpha);
 #pragma unroll
@@ -462,7 +478,7 @@ __device__ __forceinline__ void resident_part(const ResPart &a, const ResCoef *c
 #pragma unroll
             for (int t = 0; t < R; ++t)
                 if (mine[t]) {
-                    a.u[base + c0 + t] = un[t];
+                    a.out[base + c0 + t] = un[t];
                     bad |= !isfinite(un[t]);
                 }
             break;
@@ -517,16 +533,23 @@ __device__ __forceinline__ void resident_part(const ResPart &a, const ResCoef *c
 }
 
 // One line over the whole grid.
-template <int K, int FLUX, bool FAST, bool CNU, int R, bool ONE>
-__global__ __launch_bounds__(kResThreads) void resident_kernel(ResArgs a, int waves)
+// (R = 8: three wavefronts per SIMD and 168 VGPRs)
+template <int K, int FLUX, bool FAST, bool CNU, int R, bool ONE, bool REC>
+__global__ __launch_bounds__(R == 8 ? 768 : kResThreads) void resident_kernel(ResArgs a, int waves)
 {
     extern __shared__ double lds[];
     __shared__ unsigned long long s_mx[4];   // block maxima of |u|, in turn
     __shared__ double s_alpha;
     const int b = blockIdx.x, B = gridDim.x;
     ResPart p;
-    p.u = a.u;
+    p.in = a.in;
+    p.out = a.out;
     p.saved = a.saved;
+    if constexpr (REC) {
+        p.tape = a.tape;
+        p.tape_stride = a.tape_stride;
+        p.alpha_rec = a.alpha_rec;
+    }
     p.n = a.n;
     p.base = (long long)b * a.M;
     p.m = (int)min((long long)a.M, a.n - p.base);
@@ -550,7 +573,7 @@ __global__ __launch_bounds__(kResThreads) void resident_kernel(ResArgs a, int wa
     p.tag = a.tag;
     p.polls = a.polls;
     p.status = a.status;
-    resident_part<K, FLUX, FAST, CNU, R, ONE, kResMaxBlocks>(p, a.coef, waves, blockDim.x, lds, s_mx, &s_alpha);
+    resident_part<K, FLUX, FAST, CNU, R, ONE, kResMaxBlocks, REC>(p, a.coef, waves, blockDim.x, lds, s_mx, &s_alpha);
 }
 
 // ---- an ensemble of periodic lines (kernels_1d_fast.hpp's batch), each on a block or a few ----
@@ -598,7 +621,7 @@ __global__ __launch_bounds__(64 * kBatchResWaves) __attribute__((amdgpu_waves_pe
     if (threadIdx.x < 3) s_coef[threadIdx.x] = res_coef(RK3_1 + (int)threadIdx.x, b.h);
     if (64 * wv >= threads) return;   // (whole wavefronts; a barrier counts those that are left)
     ResPart p;
-    p.u = a.u + b.off;
+    p.in = p.out = a.u + b.off;
     p.saved = nullptr;
     p.n = b.n;
     p.base = b.base;
@@ -624,9 +647,9 @@ __global__ __launch_bounds__(64 * kBatchResWaves) __attribute__((amdgpu_waves_pe
     p.status = nullptr;
 #define HRW_RES_PART(K)                                                                                       \
     if (b.group == 1)                                                                                         \
-        resident_part<K, FLUX, true, false, R, true, kBatchResGroup>(p, s_coef, waves, threads, lds, s_mx, &s_alpha); \
+        resident_part<K, FLUX, true, false, R, true, kBatchResGroup, false>(p, s_coef, waves, threads, lds, s_mx, &s_alpha); \
     else                                                                                                      \
-        resident_part<K, FLUX, true, false, R, false, kBatchResGroup>(p, s_coef, waves, threads, lds, s_mx, &s_alpha)
+        resident_part<K, FLUX, true, false, R, false, kBatchResGroup, false>(p, s_coef, waves, threads, lds, s_mx, &s_alpha)
     if (b.k == 3) {
         HRW_RES_PART(3);
     } else if (b.k == 2) {

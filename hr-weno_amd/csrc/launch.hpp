@@ -11,6 +11,7 @@
 #include "kernels_adjoint_general.hpp"
 #include "kernels_adjoint_blocked.hpp"
 #include "kernels_resident.hpp"
+#include "kernels_adjoint_resident.hpp"
 
 namespace hrw {
 
@@ -38,8 +39,8 @@ void launch_fast_1d_k2(int flux, bool periodic, bool alphamax, bool constw, int 
                        const Stage1DArgs &a, hipStream_t s);
 void launch_fast_1d_k3(int flux, bool periodic, bool alphamax, bool constw, int form, int r,
                        const Stage1DArgs &a, hipStream_t s);
-// A whole rktvd integration in one launch (kernels_resident.hpp): r cells per lane (1, 2, 4; 1 on
-// a non-uniform grid), `waves` wavefronts per block, `blocks` blocks (at most one per CU; the caller
+// A whole rktvd integration in one launch (kernels_resident.hpp): r cells per lane (1, 2, 4 and,
+// FAST, 5, 8; 1 on a non-uniform grid), `waves` wavefronts per block, `blocks` blocks (at most one per CU; the caller
 // sees to it that no other launch whose blocks wait for each other is in flight on the device).
 struct ResPlan {
     int r, waves, blocks;
@@ -49,6 +50,15 @@ hipError_t launch_resident_k2(int flux, bool fast, const ResPlan &pl, const ResA
 hipError_t launch_resident_k3(int flux, bool fast, const ResPlan &pl, const ResArgs &a, hipStream_t s);
 // nsteps RK3 steps of every line of a batch in one launch, r cells per lane (2 or 4).
 hipError_t launch_batch_resident(int flux, int r, long long blocks, const BatchResArgs &a, hipStream_t s);
+// The reverse of a whole recorded integration in one launch (kernels_adjoint_resident.hpp; K = 2, 3):
+// lfp: periodic Lax-Friedrichs; otherwise `flux` (the caller as for launch_resident_k<K>).
+struct AresPlan {
+    int blocks, chunks, units;
+    long long M;
+    size_t lds;
+};
+hipError_t launch_adjoint_resident(int k, bool lfp, int flux, bool alphamax, const AresPlan &pl, const AresArgs &a,
+                                   hipStream_t s);
 // LDS-tile 1D stage (EXACT form, and the FAST LDS variant).
 void launch_tile_1d(int k, int flux, bool periodic, bool fast, bool alphamax, const Stage1DArgs &a,
                     hipStream_t s);

@@ -174,3 +174,26 @@ def test_threads(hh, dev):
     for th in threads:
         th.join()
     assert len(out) == 3 and all(np.array_equal(v, ref) for v in out.values())
+
+
+# five and eight cells per lane (Lax-Friedrichs, Godunov), and just past what fits
+@pytest.mark.parametrize("n", [786433, 1187328, 1187329, 1266688, 1266689, 1393664, 1393665, 1520640, 1520641])
+@pytest.mark.parametrize("flux,bc,k", [(LF, PER, 3), (GOD, ZG, 3), (LF, ZG, 2), (GOD, PER, 1)])
+def test_largest(hh, dev, n, flux, bc, k):
+    same(run(hh, dev, n, flux, bc, k, "fast", 3, 2, False), run(hh, dev, n, flux, bc, k, "fast", 3, 2, True))
+
+
+@pytest.mark.parametrize("value", [math.nan, math.inf, -math.inf])
+@pytest.mark.parametrize("n", [300, 5000])
+def test_nonfinite_line_of_a_batch(hh, dev, n, value):
+    """A line with a non-finite cell is non-finite throughout after a step (alpha is); its neighbours
+    are untouched."""
+    import torch
+    b = hh.BurgersBatch(np.array([n, n, n]), np.array([3, 3, 3]), np.full(3, 1e-3 / n))
+    us = [u0(n), u0(n), u0(n)]
+    us[1][n // 3] = value
+    u = b.pack(us, dev)
+    b.step(u, 2)
+    out = b.unpack(u)
+    assert not np.isfinite(out[1]).any()
+    assert np.isfinite(out[0]).all() and np.array_equal(out[0], out[2])

@@ -1117,12 +1117,54 @@ static int gen_vjp(const hrw_problem_s *p, GenScratch &g, hipStream_t st, const 
 
 enum { METHOD_RK = 1, METHOD_MS = 2 };
 
+// Status words in pinned host memory, a cache line per object: a kernel stores there and the host
+// reads it after the stream's end, without a clearing launch before and a copy after (which cost a
+// call of 100 cells 10 of its 50 us).  One page for the process; an object that finds it full (or
+// not to be had) takes device memory.
+struct StatusPool {
+    static constexpr int kSlots = 1024, kWords = 8;
+    std::mutex mu;
+    unsigned long long *page = nullptr;
+    bool tried = false;
+    std::vector<int> free;
+    unsigned long long *take()
+    {
+        std::lock_guard<std::mutex> lock(mu);
+        if (!tried) {
+            tried = true;
+            void *p = nullptr;
+            if (hipHostMalloc(&p, (size_t)kSlots * kWords * 8, hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent) ==
+                hipSuccess) {
+                page = static_cast<unsigned long long *>(p);
+                for (int i = kSlots - 1; i >= 0; --i) free.push_back(i);
+            } else {
+                (void)hipGetLastError();
+            }
+        }
+        if (free.empty()) return nullptr;
+        const int i = free.back();
+        free.pop_back();
+        return page + (size_t)i * kWords;
+    }
+    void give(unsigned long long *slot)
+    {
+        std::lock_guard<std::mutex> lock(mu);
+        free.push_back((int)((slot - page) / kWords));
+    }
+};
+static StatusPool &status_pool()   // (outlives every object: never destroyed)
+{
+    static StatusPool *pool = new StatusPool;
+    return *pool;
+}
+
 // What the launches whose blocks wait for each other need of an object (kernels_resident.hpp): the
-// exchange words (kResWords; none: one block only), the status word, the next exchange number,
-// whether both are clear, and the polls of a wait (about 0.2 s; HRW_RESIDENT_POLLS at the object's
-// creation sets them for tests).
+// exchange words (kResWords; none: one block only), the two status words, the next exchange number,
+// whether the exchange words are clear, and the polls of a wait (about 0.2 s; HRW_RESIDENT_POLLS at
+// the object's creation sets them for tests).  Every launch that is given the status words is
+// waited for (read_status) before the next.
 struct ResLink {
-    unsigned long long *words = nullptr, *status = nullptr;
+    unsigned long long *words = nullptr, *status = nullptr, *host = nullptr, *dev = nullptr;
     unsigned tag = 0;
     bool clear = false;
     int polls = 1 << 18;
@@ -1130,7 +1172,54 @@ struct ResLink {
     {
         if (const char *e = std::getenv("HRW_RESIDENT_POLLS")) polls = std::atoi(e);
     }
+    ResLink(const ResLink &) = delete;
+    ResLink &operator=(const ResLink &) = delete;
+    ~ResLink()
+    {
+        if (host) status_pool().give(host);
+        dfree(dev);
+    }
+    int alloc()
+    {
+        host = status_pool().take();
+        void *p = nullptr;
+        if (host && hipHostGetDevicePointer(&p, host, 0) == hipSuccess) {
+            status = static_cast<unsigned long long *>(p);
+            return HRW_OK;
+        }
+        (void)hipGetLastError();
+        CALL(dalloc(&dev, 2));
+        status = dev;
+        return HRW_OK;
+    }
+    bool on_host() const { return status != dev; }
 };
+// Before a launch that is given the status words.
+static int clear_status(ResLink &l, hipStream_t s)
+{
+    if (l.on_host()) {
+        for (int i = 0; i < 2; ++i) __atomic_store_n(l.host + i, 0ull, __ATOMIC_RELEASE);
+    } else {
+        fill_u64_kernel<<<1, 64, 0, s>>>(l.status, 2);
+        LAUNCH_CHECK();
+    }
+    return HRW_OK;
+}
+// The status words, once the stream is done: bit i for word i.
+static int read_status(ResLink &l, unsigned *bits, hipStream_t s)
+{
+    unsigned long long w[2];
+    if (l.on_host()) {
+        HIP_TRY(hipStreamSynchronize(s));
+        for (int i = 0; i < 2; ++i) w[i] = __atomic_load_n(l.host + i, __ATOMIC_ACQUIRE);
+    } else {
+        HIP_TRY(hipMemcpyAsync(w, l.status, sizeof w, hipMemcpyDeviceToHost, s));
+        HIP_TRY(hipStreamSynchronize(s));
+    }
+    *bits = (w[0] ? 1u << RES_NONFINITE : 0u) | (w[1] ? 1u << RES_TIMEOUT : 0u);
+    if (w[1]) l.clear = false;   // (the exchange words are cleared before the next launch)
+    return HRW_OK;
+}
 
 struct hrw_ode_s {
     int method = METHOD_RK, order = 3, fevals = 0, istate = 0, arith = HRW_ARITH_FAST;
@@ -1164,8 +1253,7 @@ struct hrw_ode_s {
     // whole-integration kernel (its status word is the scan's result word too), whether it ran in
     // this call, and its scan of the result
     ResLink link;
-    unsigned long long res_bad = 0;
-    bool res_ran = false;
+    bool res_bad = false, res_ran = false;
     ~hrw_ode_s();
 };
 // Drop the recording; keep_storage: its blocks go to the pool for the next recording.
@@ -1206,7 +1294,7 @@ static int ode_alloc(hrw_ode_s *o)
     const size_t slots = (size_t)3 * kNSlot * kSlotStride;
     const bool exchange = o->p && o->method == METHOD_RK && o->p->kind == PROB_BURGERS1D && o->neq > 10 * kOutLanes;
     const size_t states = 2 + (o->fu ? 1 : 0) + (o->method == METHOD_MS ? 9 : 0);
-    const size_t all = states * state + slots + 32 + (exchange ? kResWords : 0), small = (1 << 20) / sizeof(double);
+    const size_t all = states * state + slots + (exchange ? kResWords : 0), small = (1 << 20) / sizeof(double);
     double *next = nullptr;
     size_t left = 0, later = all;
     int rc = HRW_OK;
@@ -1233,9 +1321,8 @@ static int ode_alloc(hrw_ode_s *o)
         for (auto &b : o->ring_L) b = take(state);
     }
     o->slots = reinterpret_cast<unsigned long long *>(take(slots));
-    o->link.status = reinterpret_cast<unsigned long long *>(take(32));
     if (exchange) o->link.words = reinterpret_cast<unsigned long long *>(take(kResWords));
-    return rc;
+    return rc != HRW_OK ? rc : o->link.alloc();
 }
 
 static int ode_new(int method, int order, hrw_problem_s *p, hrw_integrand_fn fu, void *ctx,
@@ -1387,15 +1474,6 @@ static int64_t count_steps(double &t, double tout, double dt)
     return n;
 }
 
-// The result word of a scan or of the whole-integration kernel, once the stream is done.
-static int read_status(ResLink &l, unsigned long long *bad, hipStream_t s)
-{
-    HIP_TRY(hipMemcpyAsync(bad, l.status, sizeof *bad, hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
-    if (*bad) l.clear = false;   // cleared before the next whole-integration launch
-    return HRW_OK;
-}
-
 // ---- the whole integration in one launch (resident_kernel) ----
 // How a line of n cells is split: cells per lane r, wavefronts per block, blocks.  Measured on 40
 // RK3 steps, us per stage against one launch per stage (FAST Lax-Friedrichs with alpha = max|u|):
@@ -1481,7 +1559,7 @@ struct ResTape {
 // the state of one block's result is not asked for, and nothing waits for it.
 static int resident_run(const hrw_problem_s *p, int order, double dt, const ResPlan &pl, ResLink &l,
                         const double *in, double *out, double *saved, int64_t nsteps, const ResTape &tape,
-                        hipStream_t s, unsigned long long *bad, bool *saved_in, bool *ran)
+                        hipStream_t s, bool *bad, bool *saved_in, bool *ran)
 {
     *ran = *saved_in = false;
     std::unique_lock<std::mutex> alone;
@@ -1514,22 +1592,22 @@ static int resident_run(const hrw_problem_s *p, int order, double dt, const ResP
     if (!l.clear || l.tag > 0xffffffffu - used) {
         if (l.words)
             fill_u64_kernel<<<grid_for((long long)kResWords, 256, 64), 256, 0, s>>>(l.words, kResWords);
-        fill_u64_kernel<<<1, 64, 0, s>>>(l.status, 1);
         l.tag = kResFirstTag;
         l.clear = true;
     }
     a.tag = l.tag;
     l.tag += used;
+    if (a.status) CALL(clear_status(l, s));
     const bool fast = p->arith == HRW_ARITH_FAST;
     const hipError_t e = p->k == 1   ? launch_resident_k1(p->numflux, fast, pl, a, s)
                          : p->k == 2 ? launch_resident_k2(p->numflux, fast, pl, a, s)
                                      : launch_resident_k3(p->numflux, fast, pl, a, s);
     if (e != hipSuccess) return HRW_OK;   // (not launched)
     *saved_in = saved != nullptr;
-    unsigned long long word = 0;
-    if (a.status) CALL(read_status(l, &word, s));
-    if (word & RES_TIMEOUT) return HRW_OK;
-    if (bad) *bad = word;
+    unsigned bits = 0;
+    if (a.status) CALL(read_status(l, &bits, s));
+    if (bits & (1u << RES_TIMEOUT)) return HRW_OK;
+    if (bad) *bad = (bits & (1u << RES_NONFINITE)) != 0;
     *ran = true;
     return HRW_OK;
 }
@@ -1770,17 +1848,19 @@ static __global__ __launch_bounds__(kBlock) void nonfinite_kernel(const double *
     for (long long i = (long long)blockIdx.x * kBlock + threadIdx.x; i < n;
          i += (long long)gridDim.x * kBlock)
         b |= !isfinite(u[i]);
-    if (__any(b) && (threadIdx.x & 63) == 0) atomicOr(bad, 1ull);
+    if (__any(b) && (threadIdx.x & 63) == 0) set_status(bad, RES_NONFINITE);
 }
 
 static int ode_check_finite(hrw_ode_s *o, const double *u)
 {
-    unsigned long long bad = o->res_bad;
+    bool bad = o->res_bad;
     if (!o->res_ran) {   // (else the integration has scanned its result)
-        fill_u64_kernel<<<1, 64, 0, o->stream>>>(o->link.status, 1);
+        CALL(clear_status(o->link, o->stream));
         nonfinite_kernel<<<grid_for(o->neq, kBlock * 8, 4096), kBlock, 0, o->stream>>>(u, o->neq, o->link.status);
         LAUNCH_CHECK();
-        CALL(read_status(o->link, &bad, o->stream));
+        unsigned bits = 0;
+        CALL(read_status(o->link, &bits, o->stream));
+        bad = bits != 0;
     }
     if (bad) return fail(HRW_ERR_STATE, "non-finite state: u holds NaN or Inf after integrate");
     return HRW_OK;
@@ -2718,9 +2798,11 @@ static int adjoint_alloc(hrw_adjoint_s *a, const std::vector<int> &ncells)
     for (int i = 0; i < ny; ++i) a->Y[(size_t)i] = a->ystore + (long long)i * a->ystride;
     if (!a->b) {   // (exchange words: only a line of several blocks)
         const size_t words = a->flat > 10 * kOutLanes ? kResWords : 0;
-        CALL(dalloc(&a->link_store, 32 + words));
-        a->link.status = reinterpret_cast<unsigned long long *>(a->link_store);
-        if (words) a->link.words = a->link.status + 32;
+        if (words) {
+            CALL(dalloc(&a->link_store, words));
+            a->link.words = reinterpret_cast<unsigned long long *>(a->link_store);
+        }
+        CALL(a->link.alloc());
         const int64_t stages = a->nsteps * a->order;
         if (a->nseg == 1 && a->p->k >= 2 && a->flat >= 16 && stages >= 2 && stages < (1 << 28))
             a->ares = ares_split(a->flat, adjoint_fast_form(a->p), a->alphamax());
@@ -3169,13 +3251,7 @@ static int adjoint_resident(hrw_adjoint_s *a, const double *gN, double *g0, bool
     g.status = a->link.status;
     g.polls = a->link.polls;
     if (pl.blocks > 1) {
-        if (!a->link.clear) {
-            if (a->link.words)
-                fill_u64_kernel<<<grid_for((long long)kResWords, 256, 64), 256, 0, a->stream>>>(a->link.words, kResWords);
-            fill_u64_kernel<<<1, 64, 0, a->stream>>>(a->link.status, 1);
-            a->link.tag = kResFirstTag;
-            a->link.clear = true;
-        }
+        CALL(clear_status(a->link, a->stream));
         if (a->ares_tag == 0xffffffffu) {
             fill_u64_kernel<<<grid_for((long long)a->ares_count, 256, 4096), 256, 0, a->stream>>>(a->ares_words, (long long)a->ares_count);
             a->ares_tag = 0;
@@ -3184,9 +3260,9 @@ static int adjoint_resident(hrw_adjoint_s *a, const double *gN, double *g0, bool
     }
     if (launch_adjoint_resident(p->k, !a->general, p->numflux, p->alphamax(), pl, g, a->stream) != hipSuccess) return HRW_OK;
     *saved = true;
-    unsigned long long word = 0;
-    if (pl.blocks > 1) CALL(read_status(a->link, &word, a->stream));
-    *ran = !(word & RES_TIMEOUT);
+    unsigned bits = 0;
+    if (pl.blocks > 1) CALL(read_status(a->link, &bits, a->stream));
+    *ran = !(bits & (1u << RES_TIMEOUT));
     return HRW_OK;
 }
 

@@ -252,7 +252,7 @@ __global__ __launch_bounds__(64 * WAVES) void adjoint_resident_kernel(AresArgs a
                 }
                 if (!ok) {
                     polls = 1;
-                    if (lane == 0) atomicOr(a.status, (unsigned long long)RES_TIMEOUT);
+                    if (lane == 0) set_status(a.status, RES_TIMEOUT);
                 }
                 const unsigned half = (unsigned)(x >> 32);
                 const unsigned other = (unsigned)__builtin_amdgcn_update_dpp(0, (int)half, 0xB1, 0xF, 0xF, true);
@@ -436,7 +436,7 @@ __global__ __launch_bounds__(64 * WAVES) void adjoint_resident_kernel(AresArgs a
                 }
                 if (!__all(ok)) {
                     polls = 1;
-                    if (lane == 0) atomicOr(a.status, (unsigned long long)RES_TIMEOUT);
+                    if (lane == 0) set_status(a.status, RES_TIMEOUT);
                 }
                 __syncthreads();
                 if (c == 0 && s_first == base + cell) {

@@ -24,7 +24,7 @@
 // e % 4.  A block publishes e + 4 behind the barrier that follows its reads of e + 2; its
 // neighbours (for the maxima, every block) published those behind a barrier that follows their
 // reads of e: no word is overwritten before it is read.  Numbers go on from launch to launch.  A
-// wait is bounded; a wave that runs out of polls sets a status bit and waits no more, so every
+// wait is bounded; a wave that runs out of polls sets a status word and waits no more, so every
 // launch ends.  The blocks have saved the initial state by then, and the caller goes on from it
 // with one launch per stage.
 //
@@ -48,7 +48,13 @@ constexpr int kResThreads = 1024;
 constexpr size_t kResWords = 4 * (size_t)kResMaxBlocks * kResLine;   // one object's exchange words
 constexpr unsigned kResFirstTag = 4;   // the number after which cleared words read as not arrived
 
-enum { RES_NONFINITE = 1, RES_TIMEOUT = 2 };   // status bits
+// A launch's status: two words that the host has cleared, set by plain stores (they lie in host
+// memory, as a rule).
+enum { RES_NONFINITE = 0, RES_TIMEOUT = 1 };
+__device__ __forceinline__ void set_status(unsigned long long *status, int which)
+{
+    __hip_atomic_store(status + which, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 
 // A stage's combination of u0 (the state at the start of the step), its input us and L = rhs(us):
 // FAST  fma(C, L, fma(A, us - u0, u0))                        (kernels_1d_fast.hpp)
@@ -406,7 +412,7 @@ __device__ __forceinline__ void resident_part(const ResPart &a, const ResCoef *c
                     __builtin_amdgcn_s_setprio(2);
                     if (!gather_halo(a, tag, polls, width, cur, read_lo, read_hi)) {
                         polls = 1;
-                        if (a.status && lane == 0) atomicOr(a.status, (unsigned long long)RES_TIMEOUT);
+                        if (a.status && lane == 0) set_status(a.status, RES_TIMEOUT);
                     }
                     __builtin_amdgcn_wave_barrier();
                     __builtin_amdgcn_s_setprio(0);
@@ -422,7 +428,7 @@ __device__ __forceinline__ void resident_part(const ResPart &a, const ResCoef *c
             double x = __builtin_nan("");
             if (!gather_max<GROUP>(a, tag, polls, s_mx[q & 3], &x)) {
                 polls = 1;
-                if (a.status && lane == 0) atomicOr(a.status, (unsigned long long)RES_TIMEOUT);
+                if (a.status && lane == 0) set_status(a.status, RES_TIMEOUT);
             }
             if (lane == 0) *s_alpha = x;
         }
@@ -529,7 +535,7 @@ __device__ __forceinline__ void resident_part(const ResPart &a, const ResCoef *c
         nxt = sw;
         if (++st == a.order) st = 0;
     }
-    if (a.status && __any(bad) && lane == 0) atomicOr(a.status, (unsigned long long)RES_NONFINITE);
+    if (a.status && __any(bad) && lane == 0) set_status(a.status, RES_NONFINITE);
 }
 
 // One line over the whole grid.

@@ -320,7 +320,6 @@ __device__ __forceinline__ void resident_part(const ResPart &a, const ResCoef *c
     if (tid < 4) s_mx[tid] = 0ull;
     __syncthreads();
     double x0 = 0.0;
-    bool nan = false;
     for (int j0 = tid - width; j0 < m + width; j0 += (R + 1) * threads) {
         double x[R + 1];
 #pragma unroll
@@ -335,7 +334,6 @@ __device__ __forceinline__ void resident_part(const ResPart &a, const ResCoef *c
             cur[j] = x[i];
             if (j >= 0 && j < m) {
                 x0 = max_f64(x0, fabs(x[i]));
-                nan |= x[i] != x[i];
                 if (a.saved) a.saved[base + j] = x[i];
             }
         }
@@ -343,8 +341,6 @@ __device__ __forceinline__ void resident_part(const ResPart &a, const ResCoef *c
     if (amax) {
         x0 = row_max(x0);
         if ((lane & 15) == 15) lds_max(&s_mx[0], x0);
-        // (v_max_f64 passes a NaN over; with alpha infinite no flux of the line is finite either)
-        if (__any(nan)) lds_max(&s_mx[0], __builtin_inf());
     }
 
     // what does not change with the steps: cell widths (FAST: their reciprocals), the non-uniform

@@ -111,3 +111,13 @@ def test_recording_integrate_in_place(hh, dev):
         out.append((u.cpu().numpy(), lam.cpu().numpy(), t))
     same(out[0], out[1])
     assert out[0][2] == out[1][2]
+
+
+@pytest.mark.parametrize("value", [math.nan, math.inf])
+@pytest.mark.parametrize("n", [300, 3001])
+@pytest.mark.parametrize("bc", [PER, ZG])
+def test_nonfinite_state(hh, dev, n, value, bc):
+    u = case(n)[0].copy()
+    u[n // 2] = value
+    a, b = (grad(hh, dev, n, 3, LF, bc, 3, 3, tuned, u=u) for tuned in (False, True))
+    assert np.array_equal(a[0], b[0], equal_nan=True) and np.array_equal(a[1], b[1], equal_nan=True)

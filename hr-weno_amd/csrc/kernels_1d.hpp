@@ -137,6 +137,24 @@ static __global__ __launch_bounds__(kBlock) void maxabs_kernel(const double *__r
     publish_max(m, set, s_red);
 }
 
+// Both for a short line in one block: max|u| into set 0's first slot, the sets' other slots cleared.
+constexpr int kSeedBlock = 1024;
+static __global__ __launch_bounds__(kSeedBlock) void seed_kernel(const double *__restrict__ u, int n,
+                                                                unsigned long long *slots, int nsets)
+{
+    __shared__ double s_red[kSeedBlock / 64];
+    const int t = threadIdx.x;
+    double m = 0.0;
+#pragma unroll 4
+    for (int i = t; i < n; i += kSeedBlock) m = fmax(m, fabs(u[i]));
+    m = wave_max(m);
+    if ((t & 63) == 0) s_red[t >> 6] = m;
+    __syncthreads();
+    if (t >= nsets * kNSlot) return;
+    for (int w = 0; w < kSeedBlock / 64; ++w) m = fmax(m, s_red[w]);
+    slots[t * kSlotStride] = t == 0 ? (unsigned long long)__double_as_longlong(m) : 0ull;
+}
+
 // --------------------------------------------------------------------------------------
 // weno%reconstruct over nlines lines of n cells: element i of line l is v[l*ldv + i*incv].
 struct ReconArgs {

@@ -186,14 +186,30 @@ def test_largest(hh, dev, n, flux, bc, k):
 @pytest.mark.parametrize("value", [math.nan, math.inf, -math.inf])
 @pytest.mark.parametrize("n", [300, 5000])
 def test_nonfinite_line_of_a_batch(hh, dev, n, value):
-    """A line with a non-finite cell is non-finite throughout after a step (alpha is); its neighbours
-    are untouched."""
-    import torch
-    b = hh.BurgersBatch(np.array([n, n, n]), np.array([3, 3, 3]), np.full(3, 1e-3 / n))
+    """A line with a non-finite cell gives what the launches per stage give; its neighbours are untouched."""
     us = [u0(n), u0(n), u0(n)]
     us[1][n // 3] = value
-    u = b.pack(us, dev)
-    b.step(u, 2)
-    out = b.unpack(u)
-    assert not np.isfinite(out[1]).any()
-    assert np.isfinite(out[0]).all() and np.array_equal(out[0], out[2])
+    out = []
+    for per_line in (False, True):
+        b = hh.BurgersBatch(np.array([n, n, n]), np.array([3, 3, 3]), np.full(3, 1e-3 / n))
+        u = b.pack(us, dev)
+        (b.step_per_line if per_line else b.step)(u, 2)
+        out.append(b.unpack(u))
+    for x, y in zip(*out):
+        assert np.array_equal(x, y, equal_nan=True)
+    assert not np.isfinite(out[0][1]).all() and np.isfinite(out[0][0]).all() and np.array_equal(out[0][0], out[0][2])
+
+
+# alpha's seed: one block of 1024 threads, and the launches past its range
+@pytest.mark.parametrize("n", [1, 63, 1023, 1024, 1025, 4097, 32767, 32768, 32769])
+@pytest.mark.parametrize("at", [0, -1])
+def test_seeded_maximum(hh, dev, n, at):
+    """The right-hand side with alpha = max|u| is that with the maximum given as a fixed alpha."""
+    import torch
+    u = u0(n)
+    u[at] = -4.0
+    d = torch.as_tensor(u, device=dev)
+    a, b = (torch.empty_like(d) for _ in range(2))
+    hh.Burgers1D(n).rhs(0.0, d, a)
+    hh.Burgers1D(n, alpha=4.0).rhs(0.0, d, b)
+    assert torch.equal(a, b)

@@ -2195,10 +2195,15 @@ static int batch_chunks(hrw_batch_s *b, int R)
 // Measured, us per RK3 step against one launch per stage: 1024 lines of 256-65536 cells (LF) 163 /
 // 183, the same with the Godunov flux 126 / 183, 475 lines of 454-18274 cells 50 / 73, 256 of
 // 1024-16384 31 / 54, 8 of 30000-65000 13 / 33.  Short lines, which leave the chip half idle, go at
-// two cells per lane (800 lines of 64-2000 cells: 125 us per 8 steps, 140 at four).
+// two cells per lane (800 lines of 64-2000 cells: 125 us per 8 steps, 140 at four)  An ensemble of
+// many rounds of blocks goes at five: a block computes longer for each wait (1024 lines of 256-65536
+// cells 142 us per step, 151 at four; 300 of them, 3.0 M cells, 44 / 47; but 64 lines of 5000-60000
+// 28 / 26; eight cells per lane spill: 229).
 static int batch_resident_blocks(hrw_batch_s *b)
 {
-    const int r = b->res_r = *std::max_element(b->h_n.begin(), b->h_n.end()) <= 2048 ? 2 : 4;
+    const int r = b->res_r = *std::max_element(b->h_n.begin(), b->h_n.end()) <= 2048 ? 2
+                             : b->total < 2900000                                                       ? 4
+                                                                                                        : 5;
     const int waves = kBatchResWaves - (b->alphamax() ? 1 : 0);   // (one for the maxima)
     const long long most = (long long)waves * kOutLanes * r - 2 * res_extra(3), single = (long long)kBatchResWaves * kOutLanes * r;
     std::vector<int> lines((size_t)b->nlines);

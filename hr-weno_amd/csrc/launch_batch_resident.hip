@@ -11,12 +11,16 @@ template <int FLUX, int R> hipError_t run(long long blocks, const BatchResArgs &
     return hipGetLastError();
 }
 
+template <int FLUX> hipError_t run_r(int r, long long blocks, const BatchResArgs &a, hipStream_t s)
+{
+    return r == 2 ? run<FLUX, 2>(blocks, a, s) : r == 4 ? run<FLUX, 4>(blocks, a, s) : run<FLUX, 5>(blocks, a, s);
+}
+
 }  // namespace
 
 hipError_t launch_batch_resident(int flux, int r, long long blocks, const BatchResArgs &a, hipStream_t s)
 {
-    if (flux == LF) return r == 2 ? run<LF, 2>(blocks, a, s) : run<LF, 4>(blocks, a, s);
-    return r == 2 ? run<GODUNOV, 2>(blocks, a, s) : run<GODUNOV, 4>(blocks, a, s);
+    return flux == LF ? run_r<LF>(r, blocks, a, s) : run_r<GODUNOV>(r, blocks, a, s);
 }
 
 }  // namespace hrw

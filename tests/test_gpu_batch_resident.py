@@ -107,3 +107,11 @@ def test_two_batches_on_two_streams(hh, dev):
     ref.step(v, 12)
     torch.cuda.synchronize()
     assert torch.equal(us_d[0], v) and torch.equal(us_d[1], v)
+
+
+# an ensemble of many rounds (five cells per lane): lines at the edges of one block and of two
+@pytest.mark.parametrize("flux,alpha", [(LF, -1.0), (LF, 2.5), (GOD, -1.0)])
+def test_many_rounds(hh, dev, flux, alpha):
+    ns = [61000] * 48 + [2151, 2152, 2153, 2479, 2480, 2481, 4304, 4305, 4306, 4944, 4945, 310, 311, 40, 5]
+    assert sum(ns) > 2900000
+    both(hh, dev, ns, [2 + i % 2 for i in range(len(ns))], flux, alpha, 3)

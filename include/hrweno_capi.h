@@ -307,7 +307,10 @@ int hrw_batch_config(hrw_batch_t b, int *cells_per_lane, int *form);
  * segment, a single line's first backward also takes order*ckpt_every states more when they
  * fit.  Every later backward then recomputes the next segment on a second stream of its own
  * while it reverses the current one, with the same results (its results are ordered on the
- * adjoint's stream as always). */
+ * adjoint's stream as always).  When every stage input is kept, a line that fits on the chip goes
+ * forward, and one of up to 250,000 cells backward, in one launch; over several blocks such a call
+ * returns when its work is done (their waits for each other are checked), and takes one launch per
+ * stage, with the same results, under stream capture or while another such launch is in flight. */
 int hrw_adjoint_create(hrw_problem_t p, int order, double dt, int64_t nsteps, int ckpt_every,
                        hrw_adjoint_t *out);
 /* Every line of a batch (RK3, each line with its own dt; the Lax-Friedrichs flux); runs on

@@ -2192,8 +2192,8 @@ static int batch_chunks(hrw_batch_s *b, int R)
 
 // Block table of the whole-integration kernel: lines longer than a block first (their blocks
 // exchange, and only they have words), each over equal blocks, then the others, the longest first.
-// Measured, us per RK3 step against one launch per stage: 1024 lines of 256-65536 cells (LF) 163 /
-// 183, the same with the Godunov flux 126 / 183, 475 lines of 454-18274 cells 50 / 73, 256 of
+// Measured, us per RK3 step against one launch per stage: 1024 lines of 256-65536 cells (LF) 138 /
+// 183, the same with the Godunov flux 120 / 183, 475 lines of 454-18274 cells 50 / 73, 256 of
 // 1024-16384 31 / 54, 8 of 30000-65000 13 / 33.  Short lines, which leave the chip half idle, go at
 // two cells per lane (800 lines of 64-2000 cells: 125 us per 8 steps, 140 at four)  An ensemble of
 // many rounds of blocks goes at five: a block computes longer for each wait (1024 lines of 256-65536

@@ -60,7 +60,7 @@ def test_orders(hh, dev, n, order, steps, k):
              grad(hh, dev, n, k, flux, bc, order, steps, True, alpha))
 
 
-# around 256 blocks of 4 chunks, of 8, of 36 (2**20), and the largest that fit
+# around 256 blocks of 4 chunks and of 8 (the largest that go back in one launch), and the largest that go forward in one
 @pytest.mark.parametrize("n", [122881, 126976, 126979, 253952, 253955, 700001, 1 << 20, 1187328, 1350000, 1396736, 1400000])
 @pytest.mark.parametrize("flux,bc,alpha", [(LF, PER, -1.0), (LF, ZG, -1.0), (GOD, ZG, -1.0)])
 def test_large(hh, dev, n, flux, bc, alpha):

@@ -27,6 +27,7 @@
 #include "kernels_2d.hpp"
 #include "kernels_adjoint.hpp"
 #include "launch.hpp"
+#include "resident_rules.hpp"
 
 using namespace hrw;
 
@@ -1533,16 +1534,18 @@ static bool resident_split(long long n, int order, bool exact, bool amax, bool n
     return several(1, 7, kResMaxBlocks) || widen(1, exact ? 12 : cap) || widen(2, cap) || widen(4, cap) || (!exact && (widen(5, cap) || widen(8, amax ? 11 : 12)));
 }
 
-// Whether nsteps steps of p take it, and how.  Left to the launches per stage: problems tuned to a
-// kernel, cell widths without their coefficients and FAST lines far from the origin (the tile
-// kernel's arithmetic), and calls under stream capture.
-static bool resident_plan(const hrw_problem_s *p, int order, int64_t nsteps, const ResLink &l, hipStream_t s, ResPlan *pl)
+// Whether nsteps steps of p take it, and how; in_place: the result goes where the initial state is.
+// Left to the launches per stage: problems tuned to a kernel, cell widths without their coefficients
+// and FAST lines far from the origin (the tile kernel's arithmetic), single steps in place over
+// several blocks that do not wait for each other, single stages, and calls under stream capture.
+static bool resident_plan(const hrw_problem_s *p, int order, int64_t nsteps, bool in_place, const ResLink &l, hipStream_t s,
+                          ResPlan *pl)
 {
     if (p->kind != PROB_BURGERS1D || p->variant != 0 || p->cells_per_lane != 0) return false;
     const bool exact = p->arith != HRW_ARITH_FAST;
     if (!p->d_cnu && (p->d_width || (!exact && !near_linear_grid(p->xmin, p->rx, p->neq)))) return false;
     if (p->neq < 8 || !resident_split(p->neq, order, exact, p->alphamax(), p->d_cnu != nullptr, pl)) return false;
-    // (a launch's first stage must not be its last: blocks read each other's initial cells)
+    if (in_place && !resident_in_place(pl->blocks > 1, p->alphamax(), nsteps)) return false;
     if (pl->blocks > device_cus() || (pl->blocks > 1 && !l.words) || nsteps * order < 2 || nsteps >= (1 << 26)) return false;
     return !capturing(s);
 }
@@ -1565,7 +1568,7 @@ struct ResTape {
     long long stride = 0;
 };
 
-// nsteps steps of p from `in` to `out` (may be `in`) by resident_kernel; `saved` receives the
+// nsteps steps of p from `in` to `out` (may be `in` where resident_in_place says so) by resident_kernel; `saved` receives the
 // initial state.  *ran = false, and nothing written but `saved`, `out` and the recording, when the
 // device is taken or refuses the launch, or when the blocks waited for each other in vain (another
 // process's kernels kept some of them off the device).  *saved_in: `saved` was written.  `bad` null:
@@ -1637,7 +1640,7 @@ static int rk_integrate(hrw_ode_s *o, double *u, double *t, double tout, double 
         const int64_t nsteps = count_steps(t1, tout, dt);
         ResPlan pl;
         bool ran = false;
-        if (resident_plan(o->p, o->order, nsteps, o->link, o->stream, &pl)) {
+        if (resident_plan(o->p, o->order, nsteps, true, o->link, o->stream, &pl)) {
             bool saved = false;
             CALL(resident_run(o->p, o->order, dt, pl, o->link, u, u, pl.blocks > 1 ? o->ui : nullptr, nsteps, ResTape{},
                               o->stream, &o->res_bad, &saved, &ran));
@@ -2245,6 +2248,13 @@ static int batch_resident_blocks(hrw_batch_s *b)
     return HRW_OK;
 }
 
+// Whether a call of nsteps steps takes the whole-integration kernel, which works in place.
+static bool batch_resident_fits(const hrw_batch_s *b, int64_t nsteps)
+{
+    return b->resident && b->res_blocks > 0 && resident_in_place(b->res_words_per > 0, b->alphamax(), nsteps) &&
+           !capturing(b->stream);
+}
+
 // nsteps RK3 steps of every line by batch_resident_kernel.
 static int batch_resident_steps(hrw_batch_s *b, double *u, int64_t nsteps)
 {
@@ -2260,7 +2270,7 @@ static int batch_resident_steps(hrw_batch_s *b, double *u, int64_t nsteps)
     a.words_per = b->res_words_per;
     while (nsteps > 0) {
         // (a launch of bounded length: other streams get their turn)
-        a.nsteps = (int)std::min<int64_t>(nsteps, 64);
+        a.nsteps = (int)launch_steps(nsteps, 64);
         const unsigned used = 3u * (unsigned)a.nsteps;
         if (b->res_tag > 0xffffffffu - used) {
             const long long words = 4 * (long long)b->res_words_per;
@@ -2451,7 +2461,7 @@ extern "C" int hrw_batch_step(hrw_batch_t b, double *u, int64_t nsteps, double *
     if (((uintptr_t)u & 15u) != 0) return fail(HRW_ERR_ARG, "the batch state must be 16-byte aligned");
     if (nsteps == 0) return HRW_OK;
     BatchCall order(b);
-    if (b->resident && b->res_blocks > 0 && !capturing(b->stream)) {
+    if (batch_resident_fits(b, nsteps)) {
         CALL(batch_resident_steps(b, u, nsteps));
     } else if (use_graph) {
         CALL(batch_seed(b, u));
@@ -3139,7 +3149,10 @@ extern "C" int hrw_adjoint_forward(hrw_adjoint_t a, const double *u0, double *uN
     a->recorded = false;
     ResPlan pl;
     bool saved = false;
-    if (!a->b && a->nseg == 1 && resident_plan(a->p, a->order, a->nsteps, a->link, s, &pl)) {
+    // (u0 and uN may be one array; where they only overlap, the copy of u0 comes first)
+    const bool in_place = u0 == uN, apart = u0 + a->flat <= uN || uN + a->flat <= u0;
+    if (!a->b && a->nseg == 1 && (in_place || apart) &&
+        resident_plan(a->p, a->order, a->nsteps, in_place, a->link, s, &pl)) {
         // the recording keeps every stage input: they and their alphas come out of one launch
         // (ckpt[1], u_N again, is read by no reverse)
         bool ran = false;

@@ -9,7 +9,9 @@
 // their ends that the next step's stages reach (three per stage) with their neighbours, and after
 // each stage the block maxima of |u| (alpha = max|u|) with every block.  Within a step they compute
 // the cells past their ends that the later stages need themselves: the same values as their owners',
-// operation for operation.
+// operation for operation.  A block may store its result over the input only once its neighbours have
+// loaded their halo cells from it: they have when it has read their words, of the second step's cells
+// or of the first maximum (resident_rules.hpp: a launch of one step without maxima is never in place).
 //
 // An exchange takes 1.4 us between neighbours and 1.6 / 1.7 / 2.3 us among 64 / 128 / 256 blocks
 // (each block's words on a cache line of their own; packed, writers and readers of one line queue
@@ -88,7 +90,7 @@ struct ResArgs {
     unsigned long long *status;
     unsigned tag;                  // number of the first exchange (>= kResFirstTag)
     int polls;
-    double *out;                   // final state (may be in)
+    double *out;                   // final state (may be in: resident_in_place)
     // recording: the output of stage q, but the last, at tape + q*tape_stride, and the alpha of
     // stage q at alpha_rec[q]; or nullptr
     double *tape, *alpha_rec;

@@ -1,0 +1,26 @@
+// resident_rules.hpp -- host rules of the launches whose blocks wait for each other
+// (kernels_resident.hpp).  Plain C++.
+#pragma once
+#include <algorithm>
+#include <cstdint>
+
+namespace hrw {
+
+// Whether a launch of nsteps steps may write its result over its input.  A block loads some of its
+// neighbours' initial cells, so none may store its result before its neighbours have loaded.  With
+// alpha = max|u| every block waits for all maxima in the first stage; otherwise a block first waits
+// for its neighbours at the start of the second step, and a launch of a single step has no wait.
+constexpr bool resident_in_place(bool several_blocks, bool alphamax, int64_t nsteps)
+{
+    return !several_blocks || alphamax || nsteps >= 2;
+}
+
+// Steps of the next launch of a call with `left` steps to go, `most` (3 or more) in one launch: no
+// launch of a single step but for a call of one.
+constexpr int64_t launch_steps(int64_t left, int64_t most)
+{
+    const int64_t n = std::min(left, most);
+    return left - n == 1 ? n - 1 : n;
+}
+
+}  // namespace hrw

@@ -1,0 +1,41 @@
+"""The host rules of the launches whose blocks wait for each other (csrc/resident_rules.hpp), compiled
+for the host: what they must guarantee the kernels for every input."""
+import os
+import subprocess
+
+import pytest
+
+REPO = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+RULES = os.path.join(REPO, "hr-weno_amd", "csrc", "resident_rules.hpp")
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    """expr -> the value of a C++ expression over the rules, one compilation per program."""
+    d = tmp_path_factory.mktemp("rules")
+
+    def run(body):
+        src, exe = d / "rules.cpp", d / "rules"
+        src.write_text(f'#include <cstdio>\n#include "{RULES}"\nusing namespace hrw;\nint main()\n{{\n{body}\nreturn 0;\n}}\n')
+        subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-o", str(exe), str(src)], check=True)
+        out = subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout
+        return [[int(x) for x in line.split()] for line in out.splitlines()]
+    return run
+
+
+def test_one_step_in_place_needs_a_wait(rules):
+    """Several blocks without maxima first wait for each other in the second step."""
+    out = rules("for (int b = 0; b < 2; ++b) for (int a = 0; a < 2; ++a) for (int n = 1; n < 4; ++n)"
+                ' std::printf("%d %d %d %d\\n", b, a, n, (int)resident_in_place(b, a, n));')
+    for several, amax, n, ok in out:
+        assert ok == (not several or amax or n > 1)
+
+
+@pytest.mark.parametrize("most", [3, 64, 1024])
+def test_launches_of_a_call(rules, most):
+    """They add up to the call, none is longer than `most`, and none is a single step but in a call of one."""
+    out = rules(f"for (int64_t n = 1; n < 5 * {most}; ++n) {{ for (int64_t l = n; l > 0;) {{ const int64_t s = launch_steps(l, {most});"
+                ' std::printf("%lld ", (long long)s); l -= s; } std::printf("\\n"); }')
+    for n, steps in enumerate(out, 1):
+        assert sum(steps) == n and max(steps) <= most
+        assert n == 1 or min(steps) >= 2

@@ -1606,8 +1606,7 @@ static int resident_run(const hrw_problem_s *p, int order, double dt, const ResP
     a.polls = l.polls;
     const unsigned used = (unsigned)a.nsteps * (unsigned)order;
     if (!l.clear || l.tag > 0xffffffffu - used) {
-        if (l.words)
-            fill_u64_kernel<<<grid_for((long long)kResWords, 256, 64), 256, 0, s>>>(l.words, kResWords);
+        if (l.words) HIP_TRY(launch_kernel(fill_u64_kernel, grid_for((long long)kResWords, 256, 64), 256, 0, s, l.words, (long long)kResWords));
         l.tag = kResFirstTag;
         l.clear = true;
     }
@@ -1618,7 +1617,8 @@ static int resident_run(const hrw_problem_s *p, int order, double dt, const ResP
     const hipError_t e = p->k == 1   ? launch_resident_k1(p->numflux, fast, pl, a, s)
                          : p->k == 2 ? launch_resident_k2(p->numflux, fast, pl, a, s)
                                      : launch_resident_k3(p->numflux, fast, pl, a, s);
-    if (e != hipSuccess) return HRW_OK;   // (not launched)
+    if (launch_refused(e)) return HRW_OK;
+    if (e != hipSuccess) return fail(HRW_ERR_HIP, "kernel launch failed: %s", hipGetErrorString(e));
     *saved_in = saved != nullptr;
     unsigned bits = 0;
     if (a.status) CALL(read_status(l, &bits, s));
@@ -2274,7 +2274,7 @@ static int batch_resident_steps(hrw_batch_s *b, double *u, int64_t nsteps)
         const unsigned used = 3u * (unsigned)a.nsteps;
         if (b->res_tag > 0xffffffffu - used) {
             const long long words = 4 * (long long)b->res_words_per;
-            fill_u64_kernel<<<grid_for(words, 256, 4096), 256, 0, b->stream>>>(b->res_words, words);
+            HIP_TRY(launch_kernel(fill_u64_kernel, grid_for(words, 256, 4096), 256, 0, b->stream, b->res_words, words));
             b->res_tag = kResFirstTag;
         }
         a.tag = b->res_tag;
@@ -3283,12 +3283,15 @@ static int adjoint_resident(hrw_adjoint_s *a, const double *gN, double *g0, bool
     if (pl.blocks > 1) {
         CALL(clear_status(a->link, a->stream));
         if (a->ares_tag == 0xffffffffu) {
-            fill_u64_kernel<<<grid_for((long long)a->ares_count, 256, 4096), 256, 0, a->stream>>>(a->ares_words, (long long)a->ares_count);
+            HIP_TRY(launch_kernel(fill_u64_kernel, grid_for((long long)a->ares_count, 256, 4096), 256, 0, a->stream, a->ares_words,
+                                  (long long)a->ares_count));
             a->ares_tag = 0;
         }
         g.tag = ++a->ares_tag;
     }
-    if (launch_adjoint_resident(p->k, !a->general, p->numflux, p->alphamax(), pl, g, a->stream) != hipSuccess) return HRW_OK;
+    const hipError_t e = launch_adjoint_resident(p->k, !a->general, p->numflux, p->alphamax(), pl, g, a->stream);
+    if (launch_refused(e)) return HRW_OK;
+    if (e != hipSuccess) return fail(HRW_ERR_HIP, "kernel launch failed: %s", hipGetErrorString(e));
     *saved = true;
     unsigned bits = 0;
     if (pl.blocks > 1) CALL(read_status(a->link, &bits, a->stream));

@@ -28,6 +28,29 @@ inline int device_cus()
     return cus;
 }
 
+// A launch whose refusal the caller acts upon: returns this launch's own error (hipGetLastError would
+// also give one that an earlier call left on the thread, of a launch that went through) and leaves none
+// behind.
+template <class T> struct SameType {
+    using type = T;
+};
+template <class... P>
+hipError_t launch_kernel(void (*kernel)(P...), unsigned blocks, unsigned threads, size_t lds, hipStream_t s,
+                         typename SameType<P>::type... args)
+{
+    void *p[] = {&args...};
+    const hipError_t e =
+        hipLaunchKernel(reinterpret_cast<const void *>(kernel), dim3(blocks), dim3(threads), p, lds, s);
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e;
+}
+// Whether such an error says that the device does not take the launch (it did not start).
+inline bool launch_refused(hipError_t e)
+{
+    return e == hipErrorOutOfMemory || e == hipErrorLaunchOutOfResources || e == hipErrorInvalidConfiguration ||
+           e == hipErrorInvalidValue;
+}
+
 // Register-blocked 1D stage (FAST form).  form: one chunk per wavefront (stage1d_fast_kernel)
 // or persistent with the next chunk's loads issued ahead (stage1d_pf_kernel); r cells per lane
 // (4, 6, 8); constw: every edge of the linear grid is exact, so every width is rx.  One

@@ -8,10 +8,8 @@ template <int K, bool LFP, int FLUX, bool AMAX>
 hipError_t run(const AresPlan &pl, const AresArgs &a, hipStream_t s)
 {
     if (pl.chunks <= 4)
-        adjoint_resident_kernel<K, LFP, FLUX, AMAX, 4><<<pl.blocks, 64 * pl.chunks, pl.lds, s>>>(a);
-    else
-        adjoint_resident_kernel<K, LFP, FLUX, AMAX, 8><<<pl.blocks, 64 * pl.chunks, pl.lds, s>>>(a);
-    return hipGetLastError();
+        return launch_kernel(adjoint_resident_kernel<K, LFP, FLUX, AMAX, 4>, pl.blocks, 64 * pl.chunks, pl.lds, s, a);
+    return launch_kernel(adjoint_resident_kernel<K, LFP, FLUX, AMAX, 8>, pl.blocks, 64 * pl.chunks, pl.lds, s, a);
 }
 template <int K>
 hipError_t run_k(bool lfp, int flux, bool amax, const AresPlan &pl, const AresArgs &a, hipStream_t s)

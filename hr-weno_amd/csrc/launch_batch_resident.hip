@@ -6,9 +6,8 @@ namespace {
 
 template <int FLUX, int R> hipError_t run(long long blocks, const BatchResArgs &a, hipStream_t s)
 {
-    batch_resident_kernel<FLUX, R>
-        <<<(unsigned)blocks, 64 * kBatchResWaves, res_lds_bytes<R>(kBatchResWaves), s>>>(a);
-    return hipGetLastError();
+    return launch_kernel(batch_resident_kernel<FLUX, R>, (unsigned)blocks, 64 * kBatchResWaves,
+                         res_lds_bytes<R>(kBatchResWaves), s, a);
 }
 
 template <int FLUX> hipError_t run_r(int r, long long blocks, const BatchResArgs &a, hipStream_t s)

@@ -14,11 +14,9 @@ hipError_t run(const ResPlan &pl, const ResArgs &a, hipStream_t s)
 {
     const size_t lds = res_lds_bytes<R>(pl.waves);
     if (pl.blocks == 1)
-        resident_kernel<HRW_K, FLUX, FAST, CNU, R, true, REC><<<1, 64 * pl.waves, lds, s>>>(a, pl.waves);
-    else
-        resident_kernel<HRW_K, FLUX, FAST, CNU, R, false, REC>
-            <<<pl.blocks, 64 * (pl.waves + (a.amax ? 1 : 0)), lds, s>>>(a, pl.waves);
-    return hipGetLastError();
+        return launch_kernel(resident_kernel<HRW_K, FLUX, FAST, CNU, R, true, REC>, 1, 64 * pl.waves, lds, s, a, pl.waves);
+    return launch_kernel(resident_kernel<HRW_K, FLUX, FAST, CNU, R, false, REC>, pl.blocks,
+                         64 * (pl.waves + (a.amax ? 1 : 0)), lds, s, a, pl.waves);
 }
 template <int FLUX, bool FAST, bool REC>
 hipError_t run_r(const ResPlan &pl, const ResArgs &a, hipStream_t s)

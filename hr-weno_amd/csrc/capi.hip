@@ -27,7 +27,6 @@
 #include "kernels_2d.hpp"
 #include "kernels_adjoint.hpp"
 #include "launch.hpp"
-#include "resident_rules.hpp"
 
 using namespace hrw;
 
@@ -1173,14 +1172,13 @@ static StatusPool &status_pool()   // (outlives every object: never destroyed)
 }
 
 // What the launches whose blocks wait for each other need of an object (kernels_resident.hpp): the
-// exchange words (kResWords; none: one block only), the two status words, the next exchange number,
-// whether the exchange words are clear, and the polls of a wait (about 0.2 s; HRW_RESIDENT_POLLS at
+// exchange words (kResWords; none: one block only), the two status words, the numbers of its
+// exchanges, and the polls of a wait (about 0.2 s; HRW_RESIDENT_POLLS at
 // the object's creation sets them for tests).  Every launch that is given the status words is
 // waited for (read_status) before the next.
 struct ResLink {
     unsigned long long *words = nullptr, *status = nullptr, *host = nullptr, *dev = nullptr;
-    unsigned tag = 0;
-    bool clear = false;
+    ExchangeNumbers numbers;
     int polls = 1 << 18;
     ResLink()
     {
@@ -1231,7 +1229,7 @@ static int read_status(ResLink &l, unsigned *bits, hipStream_t s)
         HIP_TRY(hipStreamSynchronize(s));
     }
     *bits = (w[0] ? 1u << RES_NONFINITE : 0u) | (w[1] ? 1u << RES_TIMEOUT : 0u);
-    if (w[1]) l.clear = false;   // (the exchange words are cleared before the next launch)
+    if (w[1]) l.numbers.lost();
     return HRW_OK;
 }
 
@@ -1605,13 +1603,11 @@ static int resident_run(const hrw_problem_s *p, int order, double dt, const ResP
     a.status = pl.blocks > 1 || bad ? l.status : nullptr;
     a.polls = l.polls;
     const unsigned used = (unsigned)a.nsteps * (unsigned)order;
-    if (!l.clear || l.tag > 0xffffffffu - used) {
+    if (l.numbers.need_clear(used)) {
         if (l.words) HIP_TRY(launch_kernel(fill_u64_kernel, grid_for((long long)kResWords, 256, 64), 256, 0, s, l.words, (long long)kResWords));
-        l.tag = kResFirstTag;
-        l.clear = true;
+        l.numbers.cleared();
     }
-    a.tag = l.tag;
-    l.tag += used;
+    a.tag = l.numbers.next;
     if (a.status) CALL(clear_status(l, s));
     const bool fast = p->arith == HRW_ARITH_FAST;
     const hipError_t e = p->k == 1   ? launch_resident_k1(p->numflux, fast, pl, a, s)
@@ -1619,6 +1615,7 @@ static int resident_run(const hrw_problem_s *p, int order, double dt, const ResP
                                      : launch_resident_k3(p->numflux, fast, pl, a, s);
     if (launch_refused(e)) return HRW_OK;
     if (e != hipSuccess) return fail(HRW_ERR_HIP, "kernel launch failed: %s", hipGetErrorString(e));
+    l.numbers.launched(used);
     *saved_in = saved != nullptr;
     unsigned bits = 0;
     if (a.status) CALL(read_status(l, &bits, s));
@@ -2117,13 +2114,14 @@ struct hrw_batch_s {
     const double *graph_u = nullptr;
     int graph_R = 0, graph_form = 0;
     // whole-integration kernel: its block table (0 blocks: some line does not fit), cells per lane,
-    // exchange words with the count of started blocks behind them, the next exchange number; used
+    // exchange words with the count of started blocks behind them, the exchanges' numbers; used
     // unless a kernel was chosen (hrw_batch_set_*) or the tuner found one faster
     ResBlock *d_rblocks = nullptr;
     long long res_blocks = 0;
     int res_r = 4;
     unsigned long long *res_words = nullptr;
-    unsigned res_words_per = 0, res_tag = kResFirstTag, res_started = 0;
+    unsigned res_words_per = 0, res_started = 0;
+    ExchangeNumbers res_numbers;
     bool resident = true;
     bool alphamax() const { return numflux == HRW_FLUX_LAX_FRIEDRICHS && alpha < 0; }
     ~hrw_batch_s()
@@ -2243,6 +2241,7 @@ static int batch_resident_blocks(hrw_batch_s *b)
     fill_u64_kernel<<<grid_for((long long)words + 1, 256, 4096), 256, 0, b->stream>>>(b->res_words, (long long)words + 1);
     LAUNCH_CHECK();
     HIP_TRY(hipStreamSynchronize(b->stream));
+    b->res_numbers.cleared();
     b->res_words_per = (unsigned)(exchanging * kResLine);
     b->res_blocks = (long long)t.size();
     return HRW_OK;
@@ -2272,17 +2271,17 @@ static int batch_resident_steps(hrw_batch_s *b, double *u, int64_t nsteps)
         // (a launch of bounded length: other streams get their turn)
         a.nsteps = (int)launch_steps(nsteps, 64);
         const unsigned used = 3u * (unsigned)a.nsteps;
-        if (b->res_tag > 0xffffffffu - used) {
+        if (b->res_numbers.need_clear(used)) {
             const long long words = 4 * (long long)b->res_words_per;
             HIP_TRY(launch_kernel(fill_u64_kernel, grid_for(words, 256, 4096), 256, 0, b->stream, b->res_words, words));
-            b->res_tag = kResFirstTag;
+            b->res_numbers.cleared();
         }
-        a.tag = b->res_tag;
+        a.tag = b->res_numbers.next;
         a.ticket0 = b->res_started;
         const hipError_t e = launch_batch_resident(b->numflux == HRW_FLUX_LAX_FRIEDRICHS ? LF : GODUNOV, b->res_r,
                                                    b->res_blocks, a, b->stream);
         if (e != hipSuccess) return fail(HRW_ERR_HIP, "kernel launch failed: %s", hipGetErrorString(e));
-        b->res_tag += used;
+        b->res_numbers.launched(used);
         b->res_started += (unsigned)b->res_blocks;
         nsteps -= a.nsteps;
     }

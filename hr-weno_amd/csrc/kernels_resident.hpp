@@ -37,6 +37,7 @@
 #include <hip/hip_runtime.h>
 
 #include "kernels_1d_fast.hpp"
+#include "resident_rules.hpp"
 
 namespace hrw {
 
@@ -48,7 +49,6 @@ constexpr int kResMaxBlocks = 256;
 constexpr int kResLine = 64;
 constexpr int kResThreads = 1024;
 constexpr size_t kResWords = 4 * (size_t)kResMaxBlocks * kResLine;   // one object's exchange words
-constexpr unsigned kResFirstTag = 4;   // the number after which cleared words read as not arrived
 
 // A launch's status: two words that the host has cleared, set by plain stores (they lie in host
 // memory, as a rule).

@@ -23,4 +23,23 @@ constexpr int64_t launch_steps(int64_t left, int64_t most)
     return left - n == 1 ? n - 1 : n;
 }
 
+// The numbers of an object's exchanges.  They go on from launch to launch without a gap: a maximum
+// carries one bit of its number, which tells it from the word's last one only if every number in
+// between was published.  So a launch takes its numbers when it has gone through, not when it is
+// tried, and after one whose blocks waited in vain the words are cleared and the numbers start anew.
+constexpr unsigned kResFirstTag = 4;   // the number after which cleared words read as not arrived
+struct ExchangeNumbers {
+    unsigned next = kResFirstTag;
+    bool clear = false;                // the words are clear, or hold the numbers before `next`
+    // Whether the words have to be cleared before a launch of `used` exchanges.
+    bool need_clear(unsigned used) const { return !clear || next > 0xffffffffu - used; }
+    void cleared()
+    {
+        next = kResFirstTag;
+        clear = true;
+    }
+    void launched(unsigned used) { next += used; }
+    void lost() { clear = false; }
+};
+
 }  // namespace hrw

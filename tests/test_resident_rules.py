@@ -39,3 +39,37 @@ def test_launches_of_a_call(rules, most):
     for n, steps in enumerate(out, 1):
         assert sum(steps) == n and max(steps) <= most
         assert n == 1 or min(steps) >= 2
+
+
+@pytest.mark.parametrize("first", [4, 0xffffffff - 300])
+def test_exchange_numbers_leave_no_gap(rules, first):
+    """Launches that are refused, wait in vain or go through, in any order: a maximum's word (one of
+    four in turn, with bit 2 of the number) never reads as arrived before it is published."""
+    out = rules(f"""
+    ExchangeNumbers x;
+    x.cleared();
+    x.next = {first}u;
+    unsigned word[4];
+    // (as if all numbers before had been published)
+    for (unsigned i = 1; i <= 4; ++i) word[(x.next - i) & 3] = x.next == kResFirstTag ? 0 : ((x.next - i) >> 2) & 1;
+    unsigned long long seed = 1;
+    for (int launch = 0; launch < 4000; ++launch) {{
+        seed = seed * 6364136223846793005ull + 1442695040888963407ull;
+        const unsigned used = 2 + (unsigned)(seed >> 33) % 13, what = (unsigned)(seed >> 50) % 4;
+        if (x.need_clear(used)) {{
+            for (unsigned &w : word) w = 0;
+            x.cleared();
+        }}
+        if (what == 0) continue;              // refused: nothing is published
+        for (unsigned q = 0; q < used; ++q) {{
+            const unsigned tag = x.next + q, bit = (tag >> 2) & 1;
+            if (word[tag & 3] == bit) std::printf("%d %u\\n", launch, tag);
+            word[tag & 3] = bit;
+        }}
+        x.launched(used);
+        if (what == 1) {{                      // some waited in vain: the words hold anything
+            for (unsigned &w : word) w = (seed >> 40) & 1;
+            x.lost();
+        }}
+    }}""")
+    assert out == []

@@ -1171,19 +1171,22 @@ static StatusPool &status_pool()   // (outlives every object: never destroyed)
     return *pool;
 }
 
+// The polls of a wait: `usual`, or what HRW_RESIDENT_POLLS says when the object is created (for tests).
+static int resident_polls(int usual)
+{
+    const char *e = std::getenv("HRW_RESIDENT_POLLS");
+    return e ? std::atoi(e) : usual;
+}
+
 // What the launches whose blocks wait for each other need of an object (kernels_resident.hpp): the
 // exchange words (kResWords; none: one block only), the two status words, the numbers of its
-// exchanges, and the polls of a wait (about 0.2 s; HRW_RESIDENT_POLLS at
-// the object's creation sets them for tests).  Every launch that is given the status words is
+// exchanges, and the polls of a wait (about 0.2 s).  Every launch that is given the status words is
 // waited for (read_status) before the next.
 struct ResLink {
     unsigned long long *words = nullptr, *status = nullptr, *host = nullptr, *dev = nullptr;
     ExchangeNumbers numbers;
-    int polls = 1 << 18;
-    ResLink()
-    {
-        if (const char *e = std::getenv("HRW_RESIDENT_POLLS")) polls = std::atoi(e);
-    }
+    int polls = resident_polls(1 << 18);
+    ResLink() = default;
     ResLink(const ResLink &) = delete;
     ResLink &operator=(const ResLink &) = delete;
     ~ResLink()
@@ -2120,6 +2123,9 @@ struct hrw_batch_s {
     long long res_blocks = 0;
     int res_r = 4;
     unsigned long long *res_words = nullptr;
+    unsigned long long *res_status = nullptr;
+    int *d_rfirst = nullptr;
+    int res_lines = 0, res_polls = resident_polls(1 << 23);   // seconds
     unsigned res_words_per = 0, res_started = 0;
     ExchangeNumbers res_numbers;
     bool resident = true;
@@ -2130,7 +2136,7 @@ struct hrw_batch_s {
         dfree(d_off); dfree(d_n); dfree(d_k); dfree(d_cline); dfree(d_cstart);
         dfree(d_h); dfree(d_xmin); dfree(d_rx); dfree(ui); dfree(ui2); dfree(slots);
         dfree(line_slots);
-        dfree(d_rblocks); dfree(res_words);
+        dfree(d_rblocks); dfree(d_rfirst); dfree(res_words);
         if (ev_in) (void)hipEventDestroy(ev_in);
         if (ev_out) (void)hipEventDestroy(ev_out);
         if (own_stream && stream) (void)hipStreamDestroy(stream);
@@ -2212,6 +2218,7 @@ static int batch_resident_blocks(hrw_batch_s *b)
     std::sort(lines.begin(), lines.end(), [b](int x, int y) { return b->h_n[x] != b->h_n[y] ? b->h_n[x] > b->h_n[y] : x < y; });
     if (b->h_n[lines[0]] > most * kBatchResGroup) return HRW_OK;
     std::vector<ResBlock> t;
+    std::vector<int> first;   // of the lines of several blocks
     long long exchanging = 0;
     for (int l : lines) {
         const int n = b->h_n[l];
@@ -2224,6 +2231,8 @@ static int batch_resident_blocks(hrw_batch_s *b)
         q.k = b->h_k[l];
         q.g0 = (int)t.size();
         q.group = group;
+        q.mark = (int)first.size();
+        if (group > 1) first.push_back(q.g0);
         q.h = b->h_dt[l];
         q.xmin = b->h_xmin[l];
         q.rx = b->h_rx[l];
@@ -2236,13 +2245,16 @@ static int batch_resident_blocks(hrw_batch_s *b)
     }
     if ((long long)t.size() > (1 << 24)) return HRW_OK;
     CALL(upload(&b->d_rblocks, t));
-    const size_t words = 4 * (size_t)exchanging * kResLine;
-    CALL(dalloc(&b->res_words, words + 1));
-    fill_u64_kernel<<<grid_for((long long)words + 1, 256, 4096), 256, 0, b->stream>>>(b->res_words, (long long)words + 1);
+    if (!first.empty()) CALL(upload(&b->d_rfirst, first));
+    const size_t words = 4 * (size_t)exchanging * kResLine, all = words + 1 + 2 * first.size();
+    CALL(dalloc(&b->res_words, all));
+    fill_u64_kernel<<<grid_for((long long)all, 256, 4096), 256, 0, b->stream>>>(b->res_words, (long long)all);
     LAUNCH_CHECK();
     HIP_TRY(hipStreamSynchronize(b->stream));
     b->res_numbers.cleared();
     b->res_words_per = (unsigned)(exchanging * kResLine);
+    b->res_status = b->res_words + words + 1;
+    b->res_lines = (int)first.size();
     b->res_blocks = (long long)t.size();
     return HRW_OK;
 }
@@ -2262,11 +2274,24 @@ static int batch_resident_steps(hrw_batch_s *b, double *u, int64_t nsteps)
     a.blocks = b->d_rblocks;
     a.ticket = reinterpret_cast<unsigned *>(b->res_words + 4 * (size_t)b->res_words_per);
     a.amax = b->alphamax();
-    a.polls = 1 << 23;   // seconds
+    a.polls = b->res_polls;
     a.eps = b->eps;
     a.alpha = b->alpha;
     a.words = b->res_words;
     a.words_per = b->res_words_per;
+    a.saved = b->ui;
+    a.status = b->res_status;
+    BatchRecoverArgs r{};
+    r.u = u;
+    r.y1 = b->ui;
+    r.y2 = b->ui2;
+    r.blocks = b->d_rblocks;
+    r.first = b->d_rfirst;
+    r.status = b->res_status;
+    r.amax = a.amax;
+    r.eps = b->eps;
+    r.alpha = b->alpha;
+    const int flux = b->numflux == HRW_FLUX_LAX_FRIEDRICHS ? LF : GODUNOV;
     while (nsteps > 0) {
         // (a launch of bounded length: other streams get their turn)
         a.nsteps = (int)launch_steps(nsteps, 64);
@@ -2278,11 +2303,12 @@ static int batch_resident_steps(hrw_batch_s *b, double *u, int64_t nsteps)
         }
         a.tag = b->res_numbers.next;
         a.ticket0 = b->res_started;
-        const hipError_t e = launch_batch_resident(b->numflux == HRW_FLUX_LAX_FRIEDRICHS ? LF : GODUNOV, b->res_r,
-                                                   b->res_blocks, a, b->stream);
+        const hipError_t e = launch_batch_resident(flux, b->res_r, b->res_blocks, a, b->stream);
         if (e != hipSuccess) return fail(HRW_ERR_HIP, "kernel launch failed: %s", hipGetErrorString(e));
         b->res_numbers.launched(used);
         b->res_started += (unsigned)b->res_blocks;
+        r.nsteps = a.nsteps;
+        if (b->res_lines > 0) HIP_TRY(launch_batch_recover(flux, b->res_lines, r, b->stream));
         nsteps -= a.nsteps;
     }
     return HRW_OK;

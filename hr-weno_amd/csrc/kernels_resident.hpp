@@ -113,7 +113,7 @@ struct ResPart {
     int g0, group;                 // the line's blocks: lines [g0, g0 + group)
     unsigned tag;
     int polls;
-    unsigned long long *status;    // or nullptr
+    unsigned long long *status;    // (of one block: or nullptr)
 };
 
 __device__ __forceinline__ unsigned long long word_load(const unsigned long long *p)
@@ -297,8 +297,10 @@ template <int R> constexpr size_t res_lds_bytes(int waves) { return 2 * (size_t)
 
 // The block's part: `waves` wavefronts that own cells; with ONE false and alpha = max|u| one more
 // takes part, and `threads` counts them all.  lds, s_mx (4 words) and s_alpha: the block's LDS.  A
-// wait in vain leaves NaN behind.  REC: the stages and their alphas are recorded.
-template <int K, int FLUX, bool FAST, bool CNU, int R, bool ONE, int GROUP, bool REC>
+// wait in vain leaves NaN behind, and the wavefront waits no more.  REC: the stages and their alphas are
+// recorded.  SCAN: a result that is not finite is reported.
+constexpr int kInVain = -1;
+template <int K, int FLUX, bool FAST, bool CNU, int R, bool ONE, int GROUP, bool REC, bool SCAN>
 __device__ __forceinline__ void resident_part(const ResPart &a, const ResCoef *coef, int waves, int threads,
                                               double *lds, unsigned long long *s_mx, double *s_alpha)
 {
@@ -409,8 +411,8 @@ __device__ __forceinline__ void resident_part(const ResPart &a, const ResCoef *c
                     // (these wavefronts first: theirs is the longer way)
                     __builtin_amdgcn_s_setprio(2);
                     if (!gather_halo(a, tag, polls, width, cur, read_lo, read_hi)) {
-                        polls = 1;
-                        if (a.status && lane == 0) set_status(a.status, RES_TIMEOUT);
+                        polls = SCAN ? 1 : kInVain;
+                        if (SCAN && a.status && lane == 0) set_status(a.status, RES_TIMEOUT);
                     }
                     __builtin_amdgcn_wave_barrier();
                     __builtin_amdgcn_s_setprio(0);
@@ -425,8 +427,8 @@ __device__ __forceinline__ void resident_part(const ResPart &a, const ResCoef *c
         } else {
             double x = __builtin_nan("");
             if (!gather_max<GROUP>(a, tag, polls, s_mx[q & 3], &x)) {
-                polls = 1;
-                if (a.status && lane == 0) set_status(a.status, RES_TIMEOUT);
+                polls = SCAN ? 1 : kInVain;
+                if (SCAN && a.status && lane == 0) set_status(a.status, RES_TIMEOUT);
             }
             if (lane == 0) *s_alpha = x;
         }
@@ -483,7 +485,7 @@ __device__ __forceinline__ void resident_part(const ResPart &a, const ResCoef *c
             for (int t = 0; t < R; ++t)
                 if (mine[t]) {
                     a.out[base + c0 + t] = un[t];
-                    bad |= !isfinite(un[t]);
+                    bad |= SCAN && !isfinite(un[t]);
                 }
             break;
         }
@@ -533,7 +535,8 @@ __device__ __forceinline__ void resident_part(const ResPart &a, const ResCoef *c
         nxt = sw;
         if (++st == a.order) st = 0;
     }
-    if (a.status && __any(bad) && lane == 0) set_status(a.status, RES_NONFINITE);
+    if (!ONE && !SCAN && polls == kInVain && lane == 0) set_status(a.status, RES_TIMEOUT);
+    if (SCAN && a.status && __any(bad) && lane == 0) set_status(a.status, RES_NONFINITE);
 }
 
 // One line over the whole grid.
@@ -577,7 +580,7 @@ __global__ __launch_bounds__(R == 8 ? 768 : kResThreads) void resident_kernel(Re
     p.tag = a.tag;
     p.polls = a.polls;
     p.status = a.status;
-    resident_part<K, FLUX, FAST, CNU, R, ONE, kResMaxBlocks, REC>(p, a.coef, waves, blockDim.x, lds, s_mx, &s_alpha);
+    resident_part<K, FLUX, FAST, CNU, R, ONE, kResMaxBlocks, REC, true>(p, a.coef, waves, blockDim.x, lds, s_mx, &s_alpha);
 }
 
 // ---- an ensemble of periodic lines (kernels_1d_fast.hpp's batch), each on a block or a few ----
@@ -587,12 +590,18 @@ __global__ __launch_bounds__(R == 8 ? 768 : kResThreads) void resident_kernel(Re
 // time at most one line has some of its blocks waiting for others that have not started: the lines
 // ahead of it run to their ends and make room.  Two blocks of eight wavefronts share a CU; one
 // computes while the other waits for its exchange.
+//
+// Other kernels of the device can still keep a line's blocks off it for longer than a wait lasts.
+// Nobody reads a result on the host, so what waited in vain is made good in the stream: a line of
+// several blocks saves its initial state (8 bytes per cell and launch) and a wait in vain marks it;
+// batch_recover_kernel, launched behind, computes the marked lines anew, each in one block.
 constexpr int kBatchResWaves = 8;
 constexpr int kBatchResGroup = 64;      // blocks per line at most
 struct ResBlock {
     long long off;                      // the line's first cell in the flat state
     int line, n, k, base, m;            // the line, its length and order; this block's cells
-    int g0, group, pad;                 // the line's blocks [g0, g0 + group)
+    int g0, group;                      // the line's blocks [g0, g0 + group)
+    int mark;                           // of a line of several blocks: its number among those
     double h, xmin, rx;
 };
 struct BatchResArgs {
@@ -604,6 +613,8 @@ struct BatchResArgs {
     double eps, alpha;
     unsigned long long *words;
     unsigned words_per, tag;
+    double *saved;                      // receives the initial state of the lines of several blocks
+    unsigned long long *status;         // two status words for each of them
 };
 
 template <int FLUX, int R>
@@ -626,7 +637,7 @@ __global__ __launch_bounds__(64 * kBatchResWaves) __attribute__((amdgpu_waves_pe
     if (64 * wv >= threads) return;   // (whole wavefronts; a barrier counts those that are left)
     ResPart p;
     p.in = p.out = a.u + b.off;
-    p.saved = nullptr;
+    p.saved = b.group > 1 ? a.saved + b.off : nullptr;
     p.n = b.n;
     p.base = b.base;
     p.m = b.m;
@@ -648,12 +659,12 @@ __global__ __launch_bounds__(64 * kBatchResWaves) __attribute__((amdgpu_waves_pe
     p.group = b.group;
     p.tag = a.tag;
     p.polls = a.polls;
-    p.status = nullptr;
+    p.status = b.group > 1 ? a.status + 2 * b.mark : nullptr;
 #define HRW_RES_PART(K)                                                                                       \
     if (b.group == 1)                                                                                         \
-        resident_part<K, FLUX, true, false, R, true, kBatchResGroup, false>(p, s_coef, waves, threads, lds, s_mx, &s_alpha); \
+        resident_part<K, FLUX, true, false, R, true, kBatchResGroup, false, false>(p, s_coef, waves, threads, lds, s_mx, &s_alpha); \
     else                                                                                                      \
-        resident_part<K, FLUX, true, false, R, false, kBatchResGroup, false>(p, s_coef, waves, threads, lds, s_mx, &s_alpha)
+        resident_part<K, FLUX, true, false, R, false, kBatchResGroup, false, false>(p, s_coef, waves, threads, lds, s_mx, &s_alpha)
     if (b.k == 3) {
         HRW_RES_PART(3);
     } else if (b.k == 2) {
@@ -662,6 +673,71 @@ __global__ __launch_bounds__(64 * kBatchResWaves) __attribute__((amdgpu_waves_pe
         HRW_RES_PART(1);
     }
 #undef HRW_RES_PART
+}
+
+// A marked line anew from its saved state, one block per line of several, through memory: per cell
+// the operations of resident_part, so the results are the same.  (It returns at once as a rule; a
+// marked line takes one block's time.)
+struct BatchRecoverArgs {
+    double *u, *y1, *y2;                // the state; stage results (y1 holds the saved states first)
+    const ResBlock *blocks;
+    const int *first;                   // a line's first block in the table
+    unsigned long long *status;
+    int nsteps, amax;
+    double eps, alpha;
+};
+template <int K, int FLUX>
+__device__ __forceinline__ void recover_stage(const ResBlock &b, const BatchRecoverArgs &a, const ResCoef &co, const double *us,
+                                              const double *u0, double *out, double *s_red)
+{
+    constexpr int H = K - 1;
+    const int tid = threadIdx.x, n = b.n;
+    double alpha = a.alpha;
+    if (FLUX == LF && a.amax) {
+        double m = 0.0;
+        for (int i = tid; i < n; i += kResThreads) m = fmax(m, fabs(us[i]));
+        m = __builtin_bit_cast(double, wave_umax(__builtin_bit_cast(unsigned long long, m)));
+        if ((tid & 63) == 0) s_red[tid >> 6] = m;
+        __syncthreads();
+        alpha = 0.0;
+        for (int w = 0; w < kResThreads / 64; ++w) alpha = fmax(alpha, s_red[w]);
+    }
+    const double inv_rx = rcp_nr(b.rx);
+    for (int i = tid; i < n; i += kResThreads) {
+        double v[2 * H + 3], vl[3], vr[3];   // cells i-1-H .. i+1+H; reconstructions of i-1, i, i+1
+#pragma unroll
+        for (int t = 0; t < 2 * H + 3; ++t) v[t] = us[line_cell(i - 1 - H + t, n, true)];
+        lane_recon<K, true, false, 3>(v, a.eps, nullptr, vl, vr);
+        const double f0 = face_flux<K, FLUX, true, false>(vr[0], vl[1], alpha);
+        const double f1 = face_flux<K, FLUX, true, false>(vr[1], vl[2], alpha);
+        const double w = linear_edge(b.xmin, b.rx, i + 1) - linear_edge(b.xmin, b.rx, i);
+        const double L = (f0 - f1) * fma_(inv_rx, fma_(-w, inv_rx, 1.0), inv_rx), x0 = u0[i];
+        out[i] = fma_(co.C, L, fma_(co.A, v[H + 1] - x0, x0));
+    }
+    __syncthreads();
+}
+template <int K, int FLUX>
+__device__ __forceinline__ void recover_line(const ResBlock &b, const BatchRecoverArgs &a, double *s_red)
+{
+    double *u = a.u + b.off, *y1 = a.y1 + b.off, *y2 = a.y2 + b.off;
+    for (int i = threadIdx.x; i < b.n; i += kResThreads) u[i] = y1[i];
+    __syncthreads();
+    for (int q = 0; q < a.nsteps; ++q) {
+        recover_stage<K, FLUX>(b, a, res_coef(RK3_1, b.h), u, u, y1, s_red);
+        recover_stage<K, FLUX>(b, a, res_coef(RK3_2, b.h), y1, u, y2, s_red);
+        recover_stage<K, FLUX>(b, a, res_coef(RK3_3, b.h), y2, u, u, s_red);
+    }
+}
+template <int FLUX> __global__ __launch_bounds__(kResThreads) void batch_recover_kernel(BatchRecoverArgs a)
+{
+    __shared__ double s_red[kResThreads / 64];
+    unsigned long long *mark = a.status + 2 * (size_t)blockIdx.x + RES_TIMEOUT;
+    if (*mark == 0) return;
+    const ResBlock &b = a.blocks[a.first[blockIdx.x]];
+    if (b.k == 3) recover_line<3, FLUX>(b, a, s_red);
+    else if (b.k == 2) recover_line<2, FLUX>(b, a, s_red);
+    else recover_line<1, FLUX>(b, a, s_red);
+    if (threadIdx.x == 0) *mark = 0;
 }
 
 }  // namespace hrw

@@ -73,6 +73,8 @@ hipError_t launch_resident_k2(int flux, bool fast, const ResPlan &pl, const ResA
 hipError_t launch_resident_k3(int flux, bool fast, const ResPlan &pl, const ResArgs &a, hipStream_t s);
 // nsteps RK3 steps of every line of a batch in one launch, r cells per lane (2, 4 or 5).
 hipError_t launch_batch_resident(int flux, int r, long long blocks, const BatchResArgs &a, hipStream_t s);
+// Behind it: the lines of several blocks (`lines` of them) that waited in vain, anew.
+hipError_t launch_batch_recover(int flux, int lines, const BatchRecoverArgs &a, hipStream_t s);
 // The reverse of a whole recorded integration in one launch (kernels_adjoint_resident.hpp; K = 2, 3):
 // lfp: periodic Lax-Friedrichs; otherwise `flux` (the caller as for launch_resident_k<K>).
 struct AresPlan {

@@ -22,4 +22,10 @@ hipError_t launch_batch_resident(int flux, int r, long long blocks, const BatchR
     return flux == LF ? run_r<LF>(r, blocks, a, s) : run_r<GODUNOV>(r, blocks, a, s);
 }
 
+hipError_t launch_batch_recover(int flux, int lines, const BatchRecoverArgs &a, hipStream_t s)
+{
+    return flux == LF ? launch_kernel(batch_recover_kernel<LF>, lines, kResThreads, 0, s, a)
+                      : launch_kernel(batch_recover_kernel<GODUNOV>, lines, kResThreads, 0, s, a);
+}
+
 }  // namespace hrw

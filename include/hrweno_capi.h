@@ -274,8 +274,11 @@ int hrw_batch_size(hrw_batch_t b, int64_t *total, int64_t *offsets);
  * (hrw_batch_synchronize waits for the batch's stream). */
 int hrw_batch_set_stream(hrw_batch_t b, hrw_stream_t stream);
 int hrw_batch_synchronize(hrw_batch_t b);
-/* nsteps SSP-RK3 steps of every line: one launch per stage for all lines; use_graph != 0 replays
- * a captured hipGraph of one step.  t (host, nlines, may be NULL) advances by nsteps*dt[l]. */
+/* nsteps SSP-RK3 steps of every line, enqueued on the batch's stream.  Where every line fits, up to
+ * 64 steps go in one launch with the lines on the chip (a line that its blocks could not finish
+ * together is computed anew in the stream, by one of them); otherwise, in a capture, and with a kernel
+ * chosen below, one launch per stage for all lines, and use_graph != 0 replays a captured hipGraph of
+ * one step.  The results are the same.  t (host, nlines, may be NULL) advances by nsteps*dt[l]. */
 int hrw_batch_step(hrw_batch_t b, double *u, int64_t nsteps, double *t, int use_graph);
 /* The same, each line advanced by its own launches (the one-launch-per-line path). */
 int hrw_batch_step_per_line(hrw_batch_t b, double *u, int64_t nsteps, double *t);

@@ -2216,7 +2216,7 @@ static int batch_resident_blocks(hrw_batch_s *b)
     std::vector<int> lines((size_t)b->nlines);
     for (int l = 0; l < b->nlines; ++l) lines[(size_t)l] = l;
     std::sort(lines.begin(), lines.end(), [b](int x, int y) { return b->h_n[x] != b->h_n[y] ? b->h_n[x] > b->h_n[y] : x < y; });
-    if (b->h_n[lines[0]] > most * kBatchResGroup) return HRW_OK;
+    if (b->h_n[lines[0]] > most * batch_line_blocks(device_cus())) return HRW_OK;
     std::vector<ResBlock> t;
     std::vector<int> first;   // of the lines of several blocks
     long long exchanging = 0;

@@ -596,7 +596,6 @@ __global__ __launch_bounds__(R == 8 ? 768 : kResThreads) void resident_kernel(Re
 // several blocks saves its initial state (8 bytes per cell and launch) and a wait in vain marks it;
 // batch_recover_kernel, launched behind, computes the marked lines anew, each in one block.
 constexpr int kBatchResWaves = 8;
-constexpr int kBatchResGroup = 64;      // blocks per line at most
 struct ResBlock {
     long long off;                      // the line's first cell in the flat state
     int line, n, k, base, m;            // the line, its length and order; this block's cells

@@ -23,6 +23,12 @@ constexpr int64_t launch_steps(int64_t left, int64_t most)
     return left - n == 1 ? n - 1 : n;
 }
 
+// Blocks of one line of a batch at most.  They wait for each other, so all must come to be on the
+// device at once: at most one per CU (two fit on one, which leaves room beside them), and no more than
+// a wavefront gathers the maxima of.
+constexpr int kBatchResGroup = 64;
+constexpr int batch_line_blocks(int cus) { return std::min(kBatchResGroup, cus); }
+
 // The numbers of an object's exchanges.  They go on from launch to launch without a gap: a maximum
 // carries one bit of its number, which tells it from the word's last one only if every number in
 // between was published.  So a launch takes its numbers when it has gone through, not when it is

@@ -41,6 +41,13 @@ def test_launches_of_a_call(rules, most):
         assert n == 1 or min(steps) >= 2
 
 
+def test_blocks_of_a_batch_line_fit_the_device(rules):
+    """One per CU at most, on whole devices and on partitions of them."""
+    out = rules('for (int c = 1; c <= 512; ++c) std::printf("%d %d\\n", c, batch_line_blocks(c));')
+    for cus, blocks in out:
+        assert 1 <= blocks <= min(cus, 64) and (cus < 64 or blocks == 64)
+
+
 @pytest.mark.parametrize("first", [4, 0xffffffff - 300])
 def test_exchange_numbers_leave_no_gap(rules, first):
     """Launches that are refused, wait in vain or go through, in any order: a maximum's word (one of

@@ -1171,12 +1171,8 @@ static StatusPool &status_pool()   // (outlives every object: never destroyed)
     return *pool;
 }
 
-// The polls of a wait: `usual`, or what HRW_RESIDENT_POLLS says when the object is created (for tests).
-static int resident_polls(int usual)
-{
-    const char *e = std::getenv("HRW_RESIDENT_POLLS");
-    return e ? std::atoi(e) : usual;
-}
+// At an object's creation.
+static int resident_polls(int usual) { return resident_polls(std::getenv("HRW_RESIDENT_POLLS"), usual); }
 
 // What the launches whose blocks wait for each other need of an object (kernels_resident.hpp): the
 // exchange words (kResWords; none: one block only), the two status words, the numbers of its

@@ -2,7 +2,9 @@
 // (kernels_resident.hpp).  Plain C++.
 #pragma once
 #include <algorithm>
+#include <climits>
 #include <cstdint>
+#include <cstdlib>
 
 namespace hrw {
 
@@ -21,6 +23,16 @@ constexpr int64_t launch_steps(int64_t left, int64_t most)
 {
     const int64_t n = std::min(left, most);
     return left - n == 1 ? n - 1 : n;
+}
+
+// The polls of a wait: what `text` (the environment variable HRW_RESIDENT_POLLS, or null) says in whole
+// decimal digits, else `usual`.
+inline int resident_polls(const char *text, int usual)
+{
+    if (!text || *text < '0' || *text > '9') return usual;
+    char *end = nullptr;
+    const long v = std::strtol(text, &end, 10);
+    return *end == '\0' && v <= INT_MAX ? (int)v : usual;
 }
 
 // Blocks of one line of a batch at most.  They wait for each other, so all must come to be on the

@@ -65,7 +65,12 @@ enum hrw_bc {
     HRW_BC_INFLOW0_OUTFLOW = 3  /* zero flux in at the low end, upwind f(vr(n)) out at the high end */
 };
 
-/* ---------------------------------------------------------------- runtime ---------- */
+/* ---------------------------------------------------------------- runtime ----------
+ * Integrations that fit on the chip run in one launch whose blocks wait for each other's cells.
+ * The waits are bounded; where they end in vain (other kernels hold the device) the call goes on
+ * with one launch per stage, with the same results.  HRW_RESIDENT_POLLS in the environment, read
+ * when an object is created, sets the polls of a wait (a decimal number; for tests: 0 makes every
+ * wait end in vain). */
 const char *hrw_version(void);
 /* Message of the last failed call on this thread ("" if none). */
 const char *hrw_last_error(void);

@@ -48,6 +48,15 @@ def test_blocks_of_a_batch_line_fit_the_device(rules):
         assert 1 <= blocks <= min(cus, 64) and (cus < 64 or blocks == 64)
 
 
+def test_polls_from_the_environment(rules):
+    """Whole decimal digits count; anything else leaves the usual number."""
+    texts = {"0": 0, "1": 1, "300": 300, "2147483647": 2147483647, "": 77, "x": 77, "12x": 77, "-1": 77, " 3": 77,
+             "2147483648": 77, "99999999999999999999": 77, "1e3": 77}
+    body = "".join(f'std::printf("%d\\n", resident_polls("{t}", 77));' for t in texts)
+    out = rules(body + ' std::printf("%d\\n", resident_polls(nullptr, 77));')
+    assert [x[0] for x in out] == list(texts.values()) + [77]
+
+
 @pytest.mark.parametrize("first", [4, 0xffffffff - 300])
 def test_exchange_numbers_leave_no_gap(rules, first):
     """Launches that are refused, wait in vain or go through, in any order: a maximum's word (one of

@@ -1543,7 +1543,7 @@ static bool resident_plan(const hrw_problem_s *p, int order, int64_t nsteps, boo
     if (!p->d_cnu && (p->d_width || (!exact && !near_linear_grid(p->xmin, p->rx, p->neq)))) return false;
     if (p->neq < 8 || !resident_split(p->neq, order, exact, p->alphamax(), p->d_cnu != nullptr, pl)) return false;
     if (in_place && !resident_in_place(pl->blocks > 1, p->alphamax(), nsteps)) return false;
-    if (pl->blocks > device_cus() || (pl->blocks > 1 && !l.words) || nsteps * order < 2 || nsteps >= (1 << 26)) return false;
+    if (pl->blocks > device_cus() || (pl->blocks > 1 && !l.words) || nsteps * order < 2) return false;
     return !capturing(s);
 }
 
@@ -1565,8 +1565,8 @@ struct ResTape {
     long long stride = 0;
 };
 
-// nsteps steps of p from `in` to `out` (may be `in` where resident_in_place says so) by resident_kernel; `saved` receives the
-// initial state.  *ran = false, and nothing written but `saved`, `out` and the recording, when the
+// nsteps (at most kResLaunchSteps) steps of p from `in` to `out` (may be `in` where resident_in_place
+// says so) by resident_kernel; `saved` receives the initial state.  *ran = false, and nothing written but `saved`, `out` and the recording, when the
 // device is taken or refuses the launch, or when the blocks waited for each other in vain (another
 // process's kernels kept some of them off the device).  *saved_in: `saved` was written.  `bad` null:
 // the state of one block's result is not asked for, and nothing waits for it.
@@ -1633,20 +1633,25 @@ static int rk_integrate(hrw_ode_s *o, double *u, double *t, double tout, double 
     if (o->tape_every > 0) return rk_integrate_taped(o, u, t, tout, dt, itask);
     if (o->p && o->check_finite && itask == 1) {
         double t1 = *t;
-        const int64_t nsteps = count_steps(t1, tout, dt);
+        int64_t left = count_steps(t1, tout, dt);
         ResPlan pl;
-        bool ran = false;
-        if (resident_plan(o->p, o->order, nsteps, true, o->link, o->stream, &pl)) {
-            bool saved = false;
-            CALL(resident_run(o->p, o->order, dt, pl, o->link, u, u, pl.blocks > 1 ? o->ui : nullptr, nsteps, ResTape{},
-                              o->stream, &o->res_bad, &saved, &ran));
-            if (saved && !ran)
-                HIP_TRY(hipMemcpyAsync(u, o->ui, o->neq * sizeof(double), hipMemcpyDeviceToDevice, o->stream));
+        bool ran = resident_plan(o->p, o->order, left, true, o->link, o->stream, &pl);
+        while (ran && left > 0) {
+            const int64_t n = launch_steps(left, kResLaunchSteps);
+            bool saved = false;   // (one block: only the last launch is waited for)
+            CALL(resident_run(o->p, o->order, dt, pl, o->link, u, u, pl.blocks > 1 ? o->ui : nullptr, n, ResTape{},
+                              o->stream, pl.blocks > 1 || n == left ? &o->res_bad : nullptr, &saved, &ran));
+            if (!ran) {
+                if (saved)
+                    HIP_TRY(hipMemcpyAsync(u, o->ui, o->neq * sizeof(double), hipMemcpyDeviceToDevice, o->stream));
+                break;
+            }
+            for (int64_t i = 0; i < n; ++i) *t = *t + dt;
+            o->fevals += o->order * (int)n;
+            left -= n;
         }
-        if (ran) {
+        if (left == 0) {
             o->res_ran = true;
-            *t = t1;
-            o->fevals += o->order * (int)nsteps;
             if (o->istate == 1) o->istate = 2;         // :176
             return HRW_OK;
         }
@@ -2290,7 +2295,7 @@ static int batch_resident_steps(hrw_batch_s *b, double *u, int64_t nsteps)
     const int flux = b->numflux == HRW_FLUX_LAX_FRIEDRICHS ? LF : GODUNOV;
     while (nsteps > 0) {
         // (a launch of bounded length: other streams get their turn)
-        a.nsteps = (int)launch_steps(nsteps, 64);
+        a.nsteps = (int)launch_steps(nsteps, kBatchLaunchSteps);
         const unsigned used = 3u * (unsigned)a.nsteps;
         if (b->res_numbers.need_clear(used)) {
             const long long words = 4 * (long long)b->res_words_per;
@@ -2856,7 +2861,8 @@ static int adjoint_alloc(hrw_adjoint_s *a, const std::vector<int> &ncells)
         if (a->nseg == 1 && a->p->k >= 2 && a->flat >= 16 && stages >= 2 && stages < (1 << 28))
             a->ares = ares_split(a->flat, adjoint_fast_form(a->p), a->alphamax());
         if (a->ares.blocks > 1) {
-            a->ares_count = (size_t)stages * ((size_t)a->ares.blocks * kAresLine + (a->alphamax() ? 2 * (size_t)a->ares.units : 0));
+            // (a launch's tag tells its words from those of the one before)
+            a->ares_count = (size_t)std::min<int64_t>(stages, kResLaunchSteps * a->order) * ((size_t)a->ares.blocks * kAresLine + (a->alphamax() ? 2 * (size_t)a->ares.units : 0));
             CALL(dalloc(&a->ares_words, a->ares_count));
             fill_u64_kernel<<<grid_for((long long)a->ares_count, 256, 4096), 256>>>(a->ares_words, (long long)a->ares_count);
             LAUNCH_CHECK();
@@ -3174,11 +3180,22 @@ extern "C" int hrw_adjoint_forward(hrw_adjoint_t a, const double *u0, double *uN
     const bool in_place = u0 == uN, apart = u0 + a->flat <= uN || uN + a->flat <= u0;
     if (!a->b && a->nseg == 1 && (in_place || apart) &&
         resident_plan(a->p, a->order, a->nsteps, in_place, a->link, s, &pl)) {
-        // the recording keeps every stage input: they and their alphas come out of one launch
-        // (ckpt[1], u_N again, is read by no reverse)
-        bool ran = false;
-        const ResTape tape{a->ystore, a->arec(0), a->ystride};
-        CALL(resident_run(a->p, a->order, a->dt, pl, a->link, u0, uN, a->ckpt[0], a->nsteps, tape, s, nullptr, &saved, &ran));
+        // the recording keeps every stage input: they and their alphas come out of one launch, or
+        // several in turn, each going on from the last stage input (ckpt[1], u_N again, is read by no
+        // reverse)
+        bool ran = true;
+        const double *in = u0;
+        for (int64_t q = 0; ran && q < a->nsteps;) {   // step q
+            const int64_t n = launch_steps(a->nsteps - q, kResLaunchSteps), s0 = q * a->order;
+            double *out = q + n == a->nsteps ? uN : a->Y[(size_t)(s0 + n * a->order - 1)];
+            const ResTape tape{a->ystore + s0 * a->ystride, a->arec(0) + s0, a->ystride};
+            bool kept = false;
+            CALL(resident_run(a->p, a->order, a->dt, pl, a->link, in, out, q == 0 ? a->ckpt[0] : nullptr, n, tape, s, nullptr,
+                              &kept, &ran));
+            saved = saved || kept;
+            in = out;
+            q += n;
+        }
         if (ran) {
             a->buf_seg[0] = 0;
             a->buf_seg[1] = -1;
@@ -3265,8 +3282,8 @@ static int adjoint_stage(hrw_adjoint_s *a, int64_t s, int64_t q, int k, const do
     return HRW_OK;
 }
 
-// The reverse of the whole recording from gN to g0 (may be gN) in one launch.  *ran = false when it
-// does not take it, or when the blocks waited in vain: gN is then in lamA if *saved.
+// The reverse of the whole recording from gN to g0 (may be gN), up to kResLaunchSteps steps per launch.
+// *ran = false when it does not take it, or when the blocks waited in vain: gN is then in lamA if *saved.
 static int adjoint_resident(hrw_adjoint_s *a, const double *gN, double *g0, bool *saved, bool *ran)
 {
     *ran = *saved = false;
@@ -3275,21 +3292,14 @@ static int adjoint_resident(hrw_adjoint_s *a, const double *gN, double *g0, bool
     if (!pl.blocks || a->R != 2 || p->variant != 0 || p->cells_per_lane != 0 || pl.blocks > device_cus() ||
         capturing(a->stream))
         return HRW_OK;
-    std::unique_lock<std::mutex> alone;
-    if (pl.blocks > 1 && !resident_alone(alone)) return HRW_OK;
     AresArgs g{};
-    g.x0 = a->ckpt[0];
-    g.tape = a->ystore;
     g.tape_stride = a->ystride;
-    g.alpha_rec = a->arec(0);
     g.g = gN;
     g.out = g0;
-    g.saved = a->lamA;
     g.n = p->neq;
     g.M = (int)pl.M;
     g.chunks = pl.chunks;
     g.order = a->order;
-    g.nsteps = (int)a->nsteps;
     g.periodic = p->bc == HRW_BC_PERIODIC;
     g.constw = exact_linear_grid(p->xmin, p->rx, p->neq) ? 1 : 0;
     g.eps = p->eps;
@@ -3301,22 +3311,34 @@ static int adjoint_resident(hrw_adjoint_s *a, const double *gN, double *g0, bool
     g.units = pl.units;
     g.status = a->link.status;
     g.polls = a->link.polls;
-    if (pl.blocks > 1) {
-        CALL(clear_status(a->link, a->stream));
-        if (a->ares_tag == 0xffffffffu) {
-            HIP_TRY(launch_kernel(fill_u64_kernel, grid_for((long long)a->ares_count, 256, 4096), 256, 0, a->stream, a->ares_words,
-                                  (long long)a->ares_count));
-            a->ares_tag = 0;
+    for (int64_t left = a->nsteps; left > 0; left -= g.nsteps) {
+        std::unique_lock<std::mutex> alone;
+        if (pl.blocks > 1 && !resident_alone(alone)) return HRW_OK;
+        g.nsteps = (int)launch_steps(left, kResLaunchSteps);
+        const int64_t s0 = (left - g.nsteps) * a->order;   // the first stage of these steps
+        g.x0 = s0 ? a->Y[(size_t)s0 - 1] : a->ckpt[0];
+        g.tape = a->ystore + s0 * a->ystride;
+        g.alpha_rec = a->arec(0) + s0;
+        g.saved = left == a->nsteps ? a->lamA : nullptr;
+        if (pl.blocks > 1) {
+            CALL(clear_status(a->link, a->stream));
+            if (a->ares_tag == 0xffffffffu) {
+                HIP_TRY(launch_kernel(fill_u64_kernel, grid_for((long long)a->ares_count, 256, 4096), 256, 0, a->stream,
+                                      a->ares_words, (long long)a->ares_count));
+                a->ares_tag = 0;
+            }
+            g.tag = ++a->ares_tag;
         }
-        g.tag = ++a->ares_tag;
+        const hipError_t e = launch_adjoint_resident(p->k, !a->general, p->numflux, p->alphamax(), pl, g, a->stream);
+        if (launch_refused(e)) return HRW_OK;
+        if (e != hipSuccess) return fail(HRW_ERR_HIP, "kernel launch failed: %s", hipGetErrorString(e));
+        *saved = true;
+        unsigned bits = 0;
+        if (pl.blocks > 1) CALL(read_status(a->link, &bits, a->stream));
+        if (bits & (1u << RES_TIMEOUT)) return HRW_OK;
+        g.g = g0;
     }
-    const hipError_t e = launch_adjoint_resident(p->k, !a->general, p->numflux, p->alphamax(), pl, g, a->stream);
-    if (launch_refused(e)) return HRW_OK;
-    if (e != hipSuccess) return fail(HRW_ERR_HIP, "kernel launch failed: %s", hipGetErrorString(e));
-    *saved = true;
-    unsigned bits = 0;
-    if (pl.blocks > 1) CALL(read_status(a->link, &bits, a->stream));
-    *ran = !(bits & (1u << RES_TIMEOUT));
+    *ran = true;
     return HRW_OK;
 }
 

@@ -52,7 +52,7 @@ struct AresArgs {
     long long tape_stride;
     const double *g;               // the cotangent of the result
     double *out;                   // that of the initial state (may be g)
-    double *saved;                 // receives g
+    double *saved;                 // receives g, or nullptr
     long long n;
     int M;                         // cells per block, a multiple of four chunks (the last: what is left, >= 3)
     int chunks;                    // = wavefronts of a block
@@ -125,7 +125,7 @@ __global__ __launch_bounds__(64 * WAVES) void adjoint_resident_kernel(AresArgs a
     for (int j = tid - kAresHalo; j < m + kAresHalo; j += threads) {
         const double x = a.g[line_cell(base + j, n, per)];
         L0[j] = x;
-        if (j >= 0 && j < m) a.saved[base + j] = x;
+        if (a.saved && j >= 0 && j < m) a.saved[base + j] = x;
     }
     if (tid < 4) s_peak[tid] = kNone, s_held[tid] = 0;
 

@@ -17,6 +17,12 @@ constexpr bool resident_in_place(bool several_blocks, bool alphamax, int64_t nst
     return !several_blocks || alphamax || nsteps >= 2;
 }
 
+// Steps of a line in one launch at most: some ms (3 to 15 us a step), so that other streams and threads
+// get their turn in a long call, and what is done again after a wait in vain is little.
+constexpr int64_t kResLaunchSteps = 1024;
+// The same of a batch, whose steps take up to some 100 us.
+constexpr int64_t kBatchLaunchSteps = 64;
+
 // Steps of the next launch of a call with `left` steps to go, `most` (3 or more) in one launch: no
 // launch of a single step but for a call of one.
 constexpr int64_t launch_steps(int64_t left, int64_t most)

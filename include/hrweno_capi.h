@@ -66,7 +66,8 @@ enum hrw_bc {
 };
 
 /* ---------------------------------------------------------------- runtime ----------
- * Integrations that fit on the chip run in one launch whose blocks wait for each other's cells.
+ * Integrations that fit on the chip run in one launch per 1024 steps (a batch: 64), whose blocks
+ * wait for each other's cells.
  * The waits are bounded; where they end in vain (other kernels hold the device) the call goes on
  * with one launch per stage, with the same results.  HRW_RESIDENT_POLLS in the environment, read
  * when an object is created, sets the polls of a wait (a decimal number; for tests: 0 makes every
@@ -316,7 +317,7 @@ int hrw_batch_config(hrw_batch_t b, int *cells_per_lane, int *form);
  * fit.  Every later backward then recomputes the next segment on a second stream of its own
  * while it reverses the current one, with the same results (its results are ordered on the
  * adjoint's stream as always).  When every stage input is kept, a line that fits on the chip goes
- * forward, and one of up to 250,000 cells backward, in one launch; over several blocks such a call
+ * forward, and one of up to 250,000 cells backward, in one launch per 1024 steps; over several blocks such a call
  * returns when its work is done (their waits for each other are checked), and takes one launch per
  * stage, with the same results, under stream capture or while another such launch is in flight. */
 int hrw_adjoint_create(hrw_problem_t p, int order, double dt, int64_t nsteps, int ckpt_every,

@@ -1172,16 +1172,18 @@ static StatusPool &status_pool()   // (outlives every object: never destroyed)
 }
 
 // At an object's creation.
+constexpr int kResPolls = 1 << 18;
 static int resident_polls(int usual) { return resident_polls(std::getenv("HRW_RESIDENT_POLLS"), usual); }
 
 // What the launches whose blocks wait for each other need of an object (kernels_resident.hpp): the
 // exchange words (kResWords; none: one block only), the two status words, the numbers of its
-// exchanges, and the polls of a wait (about 0.2 s).  Every launch that is given the status words is
-// waited for (read_status) before the next.
+// exchanges, the polls of a wait (about 0.2 s) and the calls to leave out after one in vain.  Every
+// launch that is given the status words is waited for (read_status) before the next.
 struct ResLink {
     unsigned long long *words = nullptr, *status = nullptr, *host = nullptr, *dev = nullptr;
     ExchangeNumbers numbers;
-    int polls = resident_polls(1 << 18);
+    int polls = resident_polls(kResPolls);
+    BackOff back_off;
     ResLink() = default;
     ResLink(const ResLink &) = delete;
     ResLink &operator=(const ResLink &) = delete;
@@ -1228,7 +1230,10 @@ static int read_status(ResLink &l, unsigned *bits, hipStream_t s)
         HIP_TRY(hipStreamSynchronize(s));
     }
     *bits = (w[0] ? 1u << RES_NONFINITE : 0u) | (w[1] ? 1u << RES_TIMEOUT : 0u);
-    if (w[1]) l.numbers.lost();
+    if (w[1]) {
+        l.numbers.lost();
+        l.back_off.in_vain();
+    }
     return HRW_OK;
 }
 
@@ -1534,8 +1539,9 @@ static bool resident_split(long long n, int order, bool exact, bool amax, bool n
 // Whether nsteps steps of p take it, and how; in_place: the result goes where the initial state is.
 // Left to the launches per stage: problems tuned to a kernel, cell widths without their coefficients
 // and FAST lines far from the origin (the tile kernel's arithmetic), single steps in place over
-// several blocks that do not wait for each other, single stages, and calls under stream capture.
-static bool resident_plan(const hrw_problem_s *p, int order, int64_t nsteps, bool in_place, const ResLink &l, hipStream_t s,
+// several blocks that do not wait for each other, single stages, calls under stream capture, and the
+// first ones after a wait in vain.
+static bool resident_plan(const hrw_problem_s *p, int order, int64_t nsteps, bool in_place, ResLink &l, hipStream_t s,
                           ResPlan *pl)
 {
     if (p->kind != PROB_BURGERS1D || p->variant != 0 || p->cells_per_lane != 0) return false;
@@ -1544,7 +1550,7 @@ static bool resident_plan(const hrw_problem_s *p, int order, int64_t nsteps, boo
     if (p->neq < 8 || !resident_split(p->neq, order, exact, p->alphamax(), p->d_cnu != nullptr, pl)) return false;
     if (in_place && !resident_in_place(pl->blocks > 1, p->alphamax(), nsteps)) return false;
     if (pl->blocks > device_cus() || (pl->blocks > 1 && !l.words) || nsteps * order < 2) return false;
-    return !capturing(s);
+    return !capturing(s) && !(pl->blocks > 1 && l.back_off.skip());
 }
 
 // Held while a launch whose blocks wait for each other is in flight on the device: two of them at
@@ -1619,6 +1625,7 @@ static int resident_run(const hrw_problem_s *p, int order, double dt, const ResP
     unsigned bits = 0;
     if (a.status) CALL(read_status(l, &bits, s));
     if (bits & (1u << RES_TIMEOUT)) return HRW_OK;
+    if (pl.blocks > 1) l.back_off.went();
     if (bad) *bad = (bits & (1u << RES_NONFINITE)) != 0;
     *ran = true;
     return HRW_OK;
@@ -2126,7 +2133,7 @@ struct hrw_batch_s {
     unsigned long long *res_words = nullptr;
     unsigned long long *res_status = nullptr;
     int *d_rfirst = nullptr;
-    int res_lines = 0, res_polls = resident_polls(1 << 23);   // seconds
+    int res_lines = 0, res_polls = resident_polls(kResPolls);
     unsigned res_words_per = 0, res_started = 0;
     ExchangeNumbers res_numbers;
     bool resident = true;
@@ -3290,7 +3297,7 @@ static int adjoint_resident(hrw_adjoint_s *a, const double *gN, double *g0, bool
     const AresPlan &pl = a->ares;
     const hrw_problem_s *p = a->p;
     if (!pl.blocks || a->R != 2 || p->variant != 0 || p->cells_per_lane != 0 || pl.blocks > device_cus() ||
-        capturing(a->stream))
+        capturing(a->stream) || (pl.blocks > 1 && a->link.back_off.skip()))
         return HRW_OK;
     AresArgs g{};
     g.tape_stride = a->ystride;
@@ -3336,6 +3343,7 @@ static int adjoint_resident(hrw_adjoint_s *a, const double *gN, double *g0, bool
         unsigned bits = 0;
         if (pl.blocks > 1) CALL(read_status(a->link, &bits, a->stream));
         if (bits & (1u << RES_TIMEOUT)) return HRW_OK;
+        if (pl.blocks > 1) a->link.back_off.went();
         g.g = g0;
     }
     *ran = true;

@@ -41,6 +41,24 @@ inline int resident_polls(const char *text, int usual)
     return *end == '\0' && v <= INT_MAX ? (int)v : usual;
 }
 
+// After a launch whose blocks waited in vain (a fifth of a second lost), an object's next calls take the
+// launches per stage at once: 1, then 2, 4 .. 256 of them between tries that end so, until one does not.
+struct BackOff {
+    int left = 0, next = 1;
+    bool skip()
+    {
+        if (left == 0) return false;
+        --left;
+        return true;
+    }
+    void in_vain()
+    {
+        left = next;
+        next = std::min(2 * next, 256);
+    }
+    void went() { left = 0, next = 1; }
+};
+
 // Blocks of one line of a batch at most.  They wait for each other, so all must come to be on the
 // device at once: at most one per CU (two fit on one, which leaves room beside them), and no more than
 // a wavefront gathers the maxima of.

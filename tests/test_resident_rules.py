@@ -57,6 +57,30 @@ def test_polls_from_the_environment(rules):
     assert [x[0] for x in out] == list(texts.values()) + [77]
 
 
+def test_back_off(rules):
+    """Calls that would wait in vain every time: few tries; one that does not, and the next is tried again."""
+    out = rules("""
+    BackOff b;
+    int tries = 0;
+    for (int call = 1; call <= 5000; ++call) {
+        if (!b.skip()) {
+            b.in_vain();
+            ++tries;
+            std::printf("%d\\n", call);
+        }
+    }
+    int wait = 0;
+    while (b.skip()) ++wait;
+    b.went();
+    std::printf("%d %d\\n", wait, (int)b.skip());
+    b.in_vain();
+    const int one = b.skip(), two = b.skip();
+    std::printf("%d %d\\n", one, two);""")
+    tries = [x[0] for x in out[:-2]]
+    assert tries[:4] == [1, 3, 6, 11] and len(tries) < 30 and max(b - a for a, b in zip(tries, tries[1:])) == 257
+    assert out[-2][0] <= 256 and out[-2][1] == 0 and out[-1] == [1, 0]
+
+
 @pytest.mark.parametrize("first", [4, 0xffffffff - 300])
 def test_exchange_numbers_leave_no_gap(rules, first):
     """Launches that are refused, wait in vain or go through, in any order: a maximum's word (one of

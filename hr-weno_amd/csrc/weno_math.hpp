@@ -210,16 +210,18 @@ struct Tri3 {
 };
 
 // EXACT: each piece is what beta_exact and weno_cell_exact form for those cells, operation for
-// operation (a product by 2, 4 or 1/4 is exact, so fusing it with the sum it enters changes
-// nothing); formed once and used by three cells.
+// operation (a product by 2 or 1/4 is exact, so fusing it with the sum it enters changes nothing;
+// where 2b overflows, 4b does too, which leaves no finite indicator either way, but 4b may overflow
+// alone, so it is not fused); formed once and used by three cells.
 HRW_HD Tri3 tri3_exact(double a, double b, double c)
 {
     Tri3 t;
     const double D = fma_(-2.0, b, a) + c;
     const double dd = 13.0 / 12 * (D * D);
-    const double b0 = fma_(-4.0, b, 3 * a) + c;
+    const double b4 = 4 * b;
+    const double b0 = (3 * a - b4) + c;
     const double b1 = a - c;
-    const double b2 = fma_(-4.0, b, a) + 3 * c;
+    const double b2 = (a - b4) + 3 * c;
     t.bA = fma_(0.25, b0 * b0, dd);
     t.bB = fma_(0.25, b1 * b1, dd);
     t.bC = fma_(0.25, b2 * b2, dd);

@@ -169,13 +169,33 @@ struct ReconArgs {
     long long incr, ldr;
 };
 
-template <int K, bool NONUNIFORM, bool FAST>
+template <int K, bool NONUNIFORM, bool FAST, bool DIVIDE>
 __device__ __forceinline__ void recon_window(const ReconArgs &a, long long i, const double *x,
-                                             double &vl, double &vr)
+                                             double &vl, double &vr, double &top)
 {
     if constexpr (NONUNIFORM) weno_cell_exact<K>(x, a.eps, a.cnu + i * (K * (K + 1)), vl, vr);
-    else if constexpr (FAST) weno_cell_fast<K>(x, a.eps, vl, vr);
+    else if constexpr (FAST) weno_cell_fast<K, DIVIDE>(x, a.eps, vl, vr, top);
     else weno_cell_exact<K>(x, a.eps, nullptr, vl, vr);
+}
+// A thread's R cells: cell m is i0 + step*m of line l, its window at x + stride*m.  FAST: where a
+// quotient left the range of the shared-reciprocal form, all of them again by the divide (one branch a
+// thread: one a face took 8 % of both sweeps of a 1500 x 1200 state).
+template <int K, bool NONUNIFORM, bool FAST, int R, bool DIVIDE = false>
+__device__ __forceinline__ void recon_cells(const ReconArgs &a, long long l, long long i0, int step, const double *x, int stride)
+{
+    double top = 0.0;
+#pragma unroll
+    for (int m = 0; m < R; ++m) {
+        const long long i = i0 + step * m;
+        if (i >= a.n) break;
+        double vl, vr;
+        recon_window<K, NONUNIFORM, FAST, DIVIDE>(a, i, x + stride * m, vl, vr, top);
+        a.vl[l * a.ldl + i * a.incl] = vl;
+        a.vr[l * a.ldr + i * a.incr] = vr;
+    }
+    if constexpr (FAST && !NONUNIFORM && K > 1 && !DIVIDE) {
+        if (!(top < kQuotTop)) recon_cells<K, NONUNIFORM, FAST, R, true>(a, l, i0, step, x, stride);
+    }
 }
 
 // Lanes along the line (lines whose cells are the nearer neighbours in memory): thread t of a
@@ -193,15 +213,7 @@ __global__ __launch_bounds__(kBlock) void reconstruct_kernel(ReconArgs a)
 #pragma unroll
         for (int w = -(K - 1); w <= K - 1; ++w)
             x[m][w + K - 1] = vline[cell_index(base + kBlock * m + w, a.n, false) * a.incv];
-#pragma unroll
-    for (int m = 0; m < R; ++m) {
-        const long long i = base + kBlock * m;
-        if (i >= a.n) return;
-        double vl, vr;
-        recon_window<K, NONUNIFORM, FAST>(a, i, x[m], vl, vr);
-        a.vl[l * a.ldl + i * a.incl] = vl;
-        a.vr[l * a.ldr + i * a.incr] = vr;
-    }
+    recon_cells<K, NONUNIFORM, FAST, R>(a, l, base, kBlock, x[0], 2 * K - 1);
 }
 
 // Lanes across the lines (lines whose neighbours' cells are nearer in memory than their own, as
@@ -225,15 +237,7 @@ __global__ __launch_bounds__(kBlock) void reconstruct_across_kernel(ReconArgs a)
     double x[R + 2 * H];
 #pragma unroll
     for (int m = 0; m < R + 2 * H; ++m) x[m] = vline[cell_index(i0 - H + m, a.n, false) * a.incv];
-#pragma unroll
-    for (int m = 0; m < R; ++m) {
-        const long long i = i0 + m;
-        if (i >= a.n) return;
-        double vl, vr;
-        recon_window<K, NONUNIFORM, FAST>(a, i, x + m, vl, vr);
-        a.vl[l * a.ldl + i * a.incl] = vl;
-        a.vr[l * a.ldr + i * a.incr] = vr;
-    }
+    recon_cells<K, NONUNIFORM, FAST, R>(a, l, i0, 1, x, 1);
 }
 
 // --------------------------------------------------------------------------------------

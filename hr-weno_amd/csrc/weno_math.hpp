@@ -11,8 +11,8 @@
 //             consolidated over a common denominator (two divides per cell instead of twelve):
 //                 w_r = d_r/q_r / sum_s d_s/q_s  =  d_r*prod_{s!=r} q_s / sum_s d_s*prod_{t!=s} q_t
 //             with q_r = (eps+beta_r)**2.  This is an exact rewrite of the algebra; only the
-//             rounding differs (a few ulp per reconstruction).  The products of two q's stay
-//             finite while |beta| < ~1e77, i.e. for cell-value jumps below ~1e38.
+//             rounding differs (a few ulp per reconstruction).  A face's numerator, of the size
+//             of beta**4 times a cell value, stays finite for cell-value jumps below ~1e33.
 //
 // The coefficient tables follow src/hrweno_weno.f90:12-21 (Shu, ICASE 97-65, Table 2.1 and
 // eqs. 2.58-2.63).  Window convention: x[K-1+m] holds v_{i+m}, m = -(K-1)..K-1.
@@ -268,19 +268,25 @@ HRW_HD void recon2_exact(double eps, const Pair2 &p1, const Pair2 &p0, double &v
     vl = fma_(wt[0], p0.Lr, 0.0) + wt[1] * p1.S;
 }
 
-// A face value over its sum of weights, correctly rounded (quot's range holds: the sum lies above
-// 2^-210 for eps > 2^-52, and below 2^900 while the jumps stay below ~1e33).
-HRW_HD double fast_div(double n, double d)
+// A face value over its sum of weights, by quot; top becomes the largest of itself, |n| and d.  The sum
+// lies above 2^-210 for eps > 2^-52, so while top < kQuotTop (jumps below some 1e33) the quotient is
+// the correctly rounded one, or an ulp off it where |n| lies below 2^-900.  DIVIDE: the divide.
+constexpr double kQuotTop = 0x1p900;
+template <bool DIVIDE> HRW_HD double fast_face(double n, double d, double &top)
 {
 #if defined(__HIP_DEVICE_COMPILE__)
-    return quot(n, d, rcp_nr(d));
-#else
-    return n / d;
+    if constexpr (!DIVIDE) {
+        top = __builtin_fmax(__builtin_fmax(top, __builtin_fabs(n)), d);
+        return quot(n, d, rcp_nr(d));
+    }
 #endif
+    (void)top;
+    return n / d;
 }
 
-// Fast form of one cell on a uniform grid (see the header comment).
-template <int K> HRW_HD void weno_cell_fast(const double *x, double eps, double &vl, double &vr)
+// Fast form of one cell on a uniform grid (see the header comment), its faces by fast_face.
+template <int K, bool DIVIDE>
+HRW_HD void weno_cell_fast(const double *x, double eps, double &vl, double &vr, double &top)
 {
     const double *v = x + (K - 1);
     if constexpr (K == 1) {
@@ -300,8 +306,8 @@ template <int K> HRW_HD void weno_cell_fast(const double *x, double eps, double 
         const double vrr1 = fma_(1.5, v[0], -0.5 * v[-1]);
         const double vlr0 = fma_(1.5, v[0], -0.5 * v[1]);
         const double vlr1 = 0.5 * (v[-1] + v[0]);
-        vr = fast_div(fma_(ar0, vrr0, ar1 * vrr1), ar0 + ar1);
-        vl = fast_div(fma_(al0, vlr0, al1 * vlr1), al0 + al1);
+        vr = fast_face<DIVIDE>(fma_(ar0, vrr0, ar1 * vrr1), ar0 + ar1, top);
+        vl = fast_face<DIVIDE>(fma_(al0, vlr0, al1 * vlr1), al0 + al1, top);
     } else {
         const double vm2 = v[-2], vm1 = v[-1], v0 = v[0], vp1 = v[1], vp2 = v[2];
         // candidate stencils, c3 rows r+1 (right faces) and r (left faces)
@@ -332,9 +338,15 @@ template <int K> HRW_HD void weno_cell_fast(const double *x, double eps, double 
         const double sl = fma_(0.1, m0, fma_(0.6, m1, 0.3 * m2));
         const double nr = fma_(0.3 * m0, vrr0, fma_(0.6 * m1, vrr1, (0.1 * m2) * vrr2));
         const double nl = fma_(0.1 * m0, vlr0, fma_(0.6 * m1, vlr1, (0.3 * m2) * vlr2));
-        vr = fast_div(nr, sr);
-        vl = fast_div(nl, sl);
+        vr = fast_face<DIVIDE>(nr, sr, top);
+        vl = fast_face<DIVIDE>(nl, sl, top);
     }
+}
+template <int K> HRW_HD void weno_cell_fast(const double *x, double eps, double &vl, double &vr)
+{
+    double top = 0.0;
+    weno_cell_fast<K, false>(x, eps, vl, vr, top);
+    if (!(top < kQuotTop)) weno_cell_fast<K, true>(x, eps, vl, vr, top);
 }
 
 // --------------------------------------------------------------------------------------

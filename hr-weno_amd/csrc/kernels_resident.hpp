@@ -144,7 +144,7 @@ __device__ __forceinline__ unsigned long long tag_phase(unsigned tag)   // in a 
     return (unsigned long long)((tag >> 2) & 1) << 63;
 }
 
-// v_max_f64 (a NaN gives the other operand), and the maximum over each row of 16 lanes into its
+// v_max_f64 (a quiet NaN gives the other operand), and the maximum over each row of 16 lanes into its
 // lane 15 (non-negative values; a lane with no source keeps its own).
 __device__ __forceinline__ double max_f64(double x, double y)
 {
@@ -337,7 +337,9 @@ __device__ __forceinline__ void resident_part(const ResPart &a, const ResCoef *c
             if (j >= m + width) continue;
             cur[j] = x[i];
             if (j >= 0 && j < m) {
-                x0 = max_f64(x0, fabs(x[i]));
+                // (a signalling NaN would take x0 with it: its own maximum is a quiet one)
+                const double x1 = fabs(x[i]);
+                x0 = max_f64(x0, max_f64(x1, x1));
                 if (a.saved) a.saved[base + j] = x[i];
             }
         }

@@ -100,6 +100,14 @@ template <class T> static void dfree(T *&p)
     p = nullptr;
 }
 
+// Memory that an object does without (it is faster with it): whether it was had.
+template <class T> static bool try_alloc(T **p, size_t count)
+{
+    if (dalloc(p, count) == HRW_OK) return true;
+    (void)hipGetLastError();
+    return false;
+}
+
 static unsigned grid_for(long long n, int per_block, unsigned cap = 1u << 20)
 {
     long long g = (n + per_block - 1) / per_block;
@@ -1191,18 +1199,22 @@ struct ResLink {
     {
         if (host) status_pool().give(host);
         dfree(dev);
+        dfree(words);
     }
-    int alloc()
+    // exchange: with the exchange words (without them, where there is no memory left, the object takes
+    // one launch per stage)
+    int alloc(bool exchange)
     {
         host = status_pool().take();
         void *p = nullptr;
         if (host && hipHostGetDevicePointer(&p, host, 0) == hipSuccess) {
             status = static_cast<unsigned long long *>(p);
-            return HRW_OK;
+        } else {
+            (void)hipGetLastError();
+            CALL(dalloc(&dev, 2));
+            status = dev;
         }
-        (void)hipGetLastError();
-        CALL(dalloc(&dev, 2));
-        status = dev;
+        if (exchange) (void)try_alloc(&words, kResWords);
         return HRW_OK;
     }
     bool on_host() const { return status != dev; }
@@ -1303,14 +1315,13 @@ hrw_ode_s::~hrw_ode_s()
 // whatever the size (hundreds with 11 of them, which a program that runs many short multistep
 // integrations pays for each object); smaller ones come from the runtime's pool for 1 us.  So small
 // buffers share blocks of up to 1 MiB and large ones one block.  udot: only an integrand callback
-// needs it; the exchange words: only a line of several blocks.
+// needs it.
 static int ode_alloc(hrw_ode_s *o)
 {
     const size_t state = ((size_t)o->neq + 31) / 32 * 32;   // 256-byte aligned
     const size_t slots = (size_t)3 * kNSlot * kSlotStride;
-    const bool exchange = o->p && o->method == METHOD_RK && o->p->kind == PROB_BURGERS1D && o->neq > 10 * kOutLanes;
     const size_t states = 2 + (o->fu ? 1 : 0) + (o->method == METHOD_MS ? 9 : 0);
-    const size_t all = states * state + slots + (exchange ? kResWords : 0), small = (1 << 20) / sizeof(double);
+    const size_t all = states * state + slots, small = (1 << 20) / sizeof(double);
     double *next = nullptr;
     size_t left = 0, later = all;
     int rc = HRW_OK;
@@ -1337,8 +1348,9 @@ static int ode_alloc(hrw_ode_s *o)
         for (auto &b : o->ring_L) b = take(state);
     }
     o->slots = reinterpret_cast<unsigned long long *>(take(slots));
-    if (exchange) o->link.words = reinterpret_cast<unsigned long long *>(take(kResWords));
-    return rc != HRW_OK ? rc : o->link.alloc();
+    if (rc != HRW_OK) return rc;
+    const bool exchange = o->p && o->method == METHOD_RK && o->p->kind == PROB_BURGERS1D && o->neq > 10 * kOutLanes;
+    return o->link.alloc(exchange);
 }
 
 static int ode_new(int method, int order, hrw_problem_s *p, hrw_integrand_fn fu, void *ctx,
@@ -2252,10 +2264,13 @@ static int batch_resident_blocks(hrw_batch_s *b)
         if (group > 1) exchanging = (long long)t.size();
     }
     if ((long long)t.size() > (1 << 24)) return HRW_OK;
-    CALL(upload(&b->d_rblocks, t));
-    if (!first.empty()) CALL(upload(&b->d_rfirst, first));
     const size_t words = 4 * (size_t)exchanging * kResLine, all = words + 1 + 2 * first.size();
-    CALL(dalloc(&b->res_words, all));
+    if (!try_alloc(&b->d_rblocks, t.size()) || !try_alloc(&b->d_rfirst, first.size()) || !try_alloc(&b->res_words, all)) {
+        dfree(b->d_rblocks); dfree(b->d_rfirst);   // (the launches per stage need none of it)
+        return HRW_OK;
+    }
+    HIP_TRY(hipMemcpy(b->d_rblocks, t.data(), t.size() * sizeof(ResBlock), hipMemcpyHostToDevice));
+    if (!first.empty()) HIP_TRY(hipMemcpy(b->d_rfirst, first.data(), first.size() * sizeof(int), hipMemcpyHostToDevice));
     fill_u64_kernel<<<grid_for((long long)all, 256, 4096), 256, 0, b->stream>>>(b->res_words, (long long)all);
     LAUNCH_CHECK();
     HIP_TRY(hipStreamSynchronize(b->stream));
@@ -2693,7 +2708,6 @@ struct hrw_adjoint_s {
     double *ystore = nullptr;     // Y's storage, one block
     long long ystride = 0;
     ResLink link;                 // one line: the forward in one launch
-    double *link_store = nullptr;
     // one line, every stage input kept: the reverse in one launch, its exchange words and the
     // number of the last launch
     AresPlan ares{};              // (blocks 0: it does not fit)
@@ -2751,7 +2765,7 @@ struct hrw_adjoint_s {
         if (side) (void)hipStreamSynchronize(side);
         for (auto &c : ckpt) dfree(c);
         for (auto &y : Y1) dfree(y);
-        dfree(ystore); dfree(link_store); dfree(ares_words);
+        dfree(ystore); dfree(ares_words);
         dfree(lamA); dfree(lamB); dfree(sets); dfree(alpha_rec);
         dfree(sets1); dfree(alpha_rec1); dfree(sink);
         if (ev_a) (void)hipEventDestroy(ev_a);
@@ -2857,30 +2871,35 @@ static int adjoint_alloc(hrw_adjoint_s *a, const std::vector<int> &ncells)
     a->ystride = (a->flat + 31) / 32 * 32;
     CALL(dalloc(&a->ystore, std::max<size_t>(1, (size_t)ny * (size_t)a->ystride)));
     for (int i = 0; i < ny; ++i) a->Y[(size_t)i] = a->ystore + (long long)i * a->ystride;
-    if (!a->b) {   // (exchange words: only a line of several blocks)
-        const size_t words = a->flat > 10 * kOutLanes ? kResWords : 0;
-        if (words) {
-            CALL(dalloc(&a->link_store, words));
-            a->link.words = reinterpret_cast<unsigned long long *>(a->link_store);
-        }
-        CALL(a->link.alloc());
-        const int64_t stages = a->nsteps * a->order;
-        if (a->nseg == 1 && a->p->k >= 2 && a->flat >= 16 && stages >= 2 && stages < (1 << 28))
-            a->ares = ares_split(a->flat, adjoint_fast_form(a->p), a->alphamax());
-        if (a->ares.blocks > 1) {
-            // (a launch's tag tells its words from those of the one before)
-            a->ares_count = (size_t)std::min<int64_t>(stages, kResLaunchSteps * a->order) * ((size_t)a->ares.blocks * kAresLine + (a->alphamax() ? 2 * (size_t)a->ares.units : 0));
-            CALL(dalloc(&a->ares_words, a->ares_count));
-            fill_u64_kernel<<<grid_for((long long)a->ares_count, 256, 4096), 256>>>(a->ares_words, (long long)a->ares_count);
-            LAUNCH_CHECK();
-        }
-    }
     CALL(dalloc(&a->lamA, (size_t)a->flat));
     CALL(dalloc(&a->lamB, (size_t)a->flat));
     a->set_words = a->b ? (size_t)a->b->nlines : (size_t)kNSlot * kSlotStride;
     CALL(dalloc(&a->sets, a->set_words * (size_t)(a->order * a->m + 2)));
     if (!a->b) CALL(dalloc(&a->alpha_rec, (size_t)(a->order * a->m + 1)));
     CALL(adjoint_chunks(a, ncells));
+    return HRW_OK;
+}
+
+// What a line's launches for the whole recording need: the last to be allocated, so that it takes
+// nothing from the rest.
+static int adjoint_alloc_resident(hrw_adjoint_s *a)
+{
+    CALL(a->link.alloc(a->flat > 10 * kOutLanes));
+    const int64_t stages = a->nsteps * a->order;
+    if (a->nseg == 1 && a->p->k >= 2 && a->flat >= 16 && stages >= 2 && stages < (1 << 28))
+        a->ares = ares_split(a->flat, adjoint_fast_form(a->p), a->alphamax());
+    if (a->ares.blocks > 1) {
+        // (a launch's tag tells its words from those of the one before)
+        a->ares_count = (size_t)std::min<int64_t>(stages, kResLaunchSteps * a->order) *
+                        ((size_t)a->ares.blocks * kAresLine + (a->alphamax() ? 2 * (size_t)a->ares.units : 0));
+        if (!try_alloc(&a->ares_words, a->ares_count)) {
+            a->ares.blocks = 0;
+            return HRW_OK;
+        }
+        fill_u64_kernel<<<grid_for((long long)a->ares_count, 256, 4096), 256>>>(a->ares_words, (long long)a->ares_count);
+        LAUNCH_CHECK();
+        HIP_TRY(hipStreamSynchronize(nullptr));
+    }
     return HRW_OK;
 }
 
@@ -3011,6 +3030,7 @@ extern "C" int hrw_adjoint_create(hrw_problem_t p, int order, double dt, int64_t
     CALL(adjoint_alloc(a, std::vector<int>{(int)p->neq}));
     a->general = !adjoint_fast_form(p);
     if (a->general) CALL(a->gen.alloc(p->neq));
+    CALL(adjoint_alloc_resident(a));
     *out = guard.release();
     return HRW_OK;
 }

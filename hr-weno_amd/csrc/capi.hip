@@ -2289,8 +2289,9 @@ static bool batch_resident_fits(const hrw_batch_s *b, int64_t nsteps)
            !capturing(b->stream);
 }
 
-// nsteps RK3 steps of every line by batch_resident_kernel.
-static int batch_resident_steps(hrw_batch_s *b, double *u, int64_t nsteps)
+// *left RK3 steps of every line by batch_resident_kernel; *left: those that remain, where the device
+// refuses a launch.
+static int batch_resident_steps(hrw_batch_s *b, double *u, int64_t *left)
 {
     BatchResArgs a{};
     a.u = u;
@@ -2315,9 +2316,9 @@ static int batch_resident_steps(hrw_batch_s *b, double *u, int64_t nsteps)
     r.eps = b->eps;
     r.alpha = b->alpha;
     const int flux = b->numflux == HRW_FLUX_LAX_FRIEDRICHS ? LF : GODUNOV;
-    while (nsteps > 0) {
+    while (*left > 0) {
         // (a launch of bounded length: other streams get their turn)
-        a.nsteps = (int)launch_steps(nsteps, kBatchLaunchSteps);
+        a.nsteps = (int)launch_steps(*left, kBatchLaunchSteps);
         const unsigned used = 3u * (unsigned)a.nsteps;
         if (b->res_numbers.need_clear(used)) {
             const long long words = 4 * (long long)b->res_words_per;
@@ -2327,12 +2328,13 @@ static int batch_resident_steps(hrw_batch_s *b, double *u, int64_t nsteps)
         a.tag = b->res_numbers.next;
         a.ticket0 = b->res_started;
         const hipError_t e = launch_batch_resident(flux, b->res_r, b->res_blocks, a, b->stream);
+        if (launch_refused(e)) return HRW_OK;
         if (e != hipSuccess) return fail(HRW_ERR_HIP, "kernel launch failed: %s", hipGetErrorString(e));
         b->res_numbers.launched(used);
         b->res_started += (unsigned)b->res_blocks;
         r.nsteps = a.nsteps;
         if (b->res_lines > 0) HIP_TRY(launch_batch_recover(flux, b->res_lines, r, b->stream));
-        nsteps -= a.nsteps;
+        *left -= a.nsteps;
     }
     return HRW_OK;
 }
@@ -2509,9 +2511,9 @@ extern "C" int hrw_batch_step(hrw_batch_t b, double *u, int64_t nsteps, double *
     if (((uintptr_t)u & 15u) != 0) return fail(HRW_ERR_ARG, "the batch state must be 16-byte aligned");
     if (nsteps == 0) return HRW_OK;
     BatchCall order(b);
-    if (batch_resident_fits(b, nsteps)) {
-        CALL(batch_resident_steps(b, u, nsteps));
-    } else if (use_graph) {
+    int64_t left = nsteps;
+    if (batch_resident_fits(b, nsteps)) CALL(batch_resident_steps(b, u, &left));
+    if (left > 0 && use_graph) {
         CALL(batch_seed(b, u));
         if (!b->graph || b->graph_u != u || b->graph_R != b->chunk_R || b->graph_form != b->form) {
             if (b->graph) {
@@ -2531,10 +2533,10 @@ extern "C" int hrw_batch_step(hrw_batch_t b, double *u, int64_t nsteps, double *
             b->graph_R = b->chunk_R;
             b->graph_form = b->form;
         }
-        for (int64_t s = 0; s < nsteps; ++s) HIP_TRY(hipGraphLaunch(b->graph, b->stream));
-    } else {
+        for (int64_t s = 0; s < left; ++s) HIP_TRY(hipGraphLaunch(b->graph, b->stream));
+    } else if (left > 0) {
         CALL(batch_seed(b, u));
-        for (int64_t s = 0; s < nsteps; ++s) CALL(batch_rk3_step(b, u));
+        for (int64_t s = 0; s < left; ++s) CALL(batch_rk3_step(b, u));
     }
     if (t)
         for (int l = 0; l < b->nlines; ++l)
@@ -2636,7 +2638,8 @@ extern "C" int hrw_batch_tune(hrw_batch_t b, const double *u, int *chosen)
         for (int pass = 0; pass < 3; ++pass) {   // (the first warms up)
             (void)hipMemcpyAsync(work, u, b->total * sizeof(double), hipMemcpyDeviceToDevice, b->stream);
             (void)hipEventRecord(e0, b->stream);
-            const int rc = batch_resident_steps(b, work, 3);
+            int64_t left = 3;
+            const int rc = batch_resident_steps(b, work, &left);
             (void)hipEventRecord(e1, b->stream);
             (void)hipEventSynchronize(e1);
             if (rc != HRW_OK) {
@@ -2645,7 +2648,7 @@ extern "C" int hrw_batch_tune(hrw_batch_t b, const double *u, int *chosen)
             }
             float ms = 0.f;
             (void)hipEventElapsedTime(&ms, e0, e1);
-            if (pass > 0) res_ms = std::min(res_ms, ms);
+            if (pass > 0 && left == 0) res_ms = std::min(res_ms, ms);
         }
         b->resident = res_ms < best_ms;
     }

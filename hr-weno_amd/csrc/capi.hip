@@ -1650,7 +1650,9 @@ static int rk_integrate(hrw_ode_s *o, double *u, double *t, double tout, double 
     if (o->istate < 1) return HRW_OK;                  // :126
     if (is_done(*t, tout, dt)) return HRW_OK;          // :127
     if (o->tape_every > 0) return rk_integrate_taped(o, u, t, tout, dt, itask);
-    if (o->p && o->check_finite && itask == 1) {
+    // (the register-blocked kernels, whose arithmetic the FAST form has there, take aligned states)
+    const bool same_form = o->p && (o->p->arith != HRW_ARITH_FAST || o->p->d_cnu || aligned16(u));
+    if (same_form && o->check_finite && itask == 1) {
         double t1 = *t;
         int64_t left = count_steps(t1, tout, dt);
         ResPlan pl;

@@ -171,10 +171,10 @@ struct ReconArgs {
 
 template <int K, bool NONUNIFORM, bool FAST, bool DIVIDE>
 __device__ __forceinline__ void recon_window(const ReconArgs &a, long long i, const double *x,
-                                             double &vl, double &vr, double &top)
+                                             double &vl, double &vr, bool &out)
 {
     if constexpr (NONUNIFORM) weno_cell_exact<K>(x, a.eps, a.cnu + i * (K * (K + 1)), vl, vr);
-    else if constexpr (FAST) weno_cell_fast<K, DIVIDE>(x, a.eps, vl, vr, top);
+    else if constexpr (FAST) weno_cell_fast<K, DIVIDE>(x, a.eps, vl, vr, out);
     else weno_cell_exact<K>(x, a.eps, nullptr, vl, vr);
 }
 // A thread's R cells: cell m is i0 + step*m of line l, its window at x + stride*m.  FAST: where a
@@ -183,18 +183,18 @@ __device__ __forceinline__ void recon_window(const ReconArgs &a, long long i, co
 template <int K, bool NONUNIFORM, bool FAST, int R, bool DIVIDE = false>
 __device__ __forceinline__ void recon_cells(const ReconArgs &a, long long l, long long i0, int step, const double *x, int stride)
 {
-    double top = 0.0;
+    bool out = false;
 #pragma unroll
     for (int m = 0; m < R; ++m) {
         const long long i = i0 + step * m;
         if (i >= a.n) break;
         double vl, vr;
-        recon_window<K, NONUNIFORM, FAST, DIVIDE>(a, i, x + stride * m, vl, vr, top);
+        recon_window<K, NONUNIFORM, FAST, DIVIDE>(a, i, x + stride * m, vl, vr, out);
         a.vl[l * a.ldl + i * a.incl] = vl;
         a.vr[l * a.ldr + i * a.incr] = vr;
     }
     if constexpr (FAST && !NONUNIFORM && K > 1 && !DIVIDE) {
-        if (!(top < kQuotTop)) recon_cells<K, NONUNIFORM, FAST, R, true>(a, l, i0, step, x, stride);
+        if (out) recon_cells<K, NONUNIFORM, FAST, R, true>(a, l, i0, step, x, stride);
     }
 }
 

@@ -268,25 +268,29 @@ HRW_HD void recon2_exact(double eps, const Pair2 &p1, const Pair2 &p0, double &v
     vl = fma_(wt[0], p0.Lr, 0.0) + wt[1] * p1.S;
 }
 
-// A face value over its sum of weights, by quot; top becomes the largest of itself, |n| and d.  The sum
-// lies above 2^-210 for eps > 2^-52, so while top < kQuotTop (jumps below some 1e33) the quotient is
-// the correctly rounded one, or an ulp off it where |n| lies below 2^-900.  DIVIDE: the divide.
-constexpr double kQuotTop = 0x1p900;
-template <bool DIVIDE> HRW_HD double fast_face(double n, double d, double &top)
+// The faces nr/sr, nl/sl by quot; `out` is set where that is not the correctly rounded quotient (or an
+// ulp off it, where the numerator lies below 2^-900): the sums lie above 2^-210 for eps > 2^-52 and
+// within a factor 3 of each other, so their reciprocals are normal numbers while sr < 2^1020, and a
+// numerator that has overflowed (jumps above some 1e33) gives NaN.  DIVIDE: the divide.
+template <bool DIVIDE>
+HRW_HD void fast_faces(double nr, double sr, double nl, double sl, double &vl, double &vr, bool &out)
 {
 #if defined(__HIP_DEVICE_COMPILE__)
     if constexpr (!DIVIDE) {
-        top = __builtin_fmax(__builtin_fmax(top, __builtin_fabs(n)), d);
-        return quot(n, d, rcp_nr(d));
+        vr = quot(nr, sr, rcp_nr(sr));
+        vl = quot(nl, sl, rcp_nr(sl));
+        out = out | __builtin_isunordered(vr, vl) | !(sr < 0x1p1020);
+        return;
     }
 #endif
-    (void)top;
-    return n / d;
+    (void)out;
+    vr = nr / sr;
+    vl = nl / sl;
 }
 
-// Fast form of one cell on a uniform grid (see the header comment), its faces by fast_face.
+// Fast form of one cell on a uniform grid (see the header comment), its faces by fast_faces.
 template <int K, bool DIVIDE>
-HRW_HD void weno_cell_fast(const double *x, double eps, double &vl, double &vr, double &top)
+HRW_HD void weno_cell_fast(const double *x, double eps, double &vl, double &vr, bool &out)
 {
     const double *v = x + (K - 1);
     if constexpr (K == 1) {
@@ -306,8 +310,7 @@ HRW_HD void weno_cell_fast(const double *x, double eps, double &vl, double &vr, 
         const double vrr1 = fma_(1.5, v[0], -0.5 * v[-1]);
         const double vlr0 = fma_(1.5, v[0], -0.5 * v[1]);
         const double vlr1 = 0.5 * (v[-1] + v[0]);
-        vr = fast_face<DIVIDE>(fma_(ar0, vrr0, ar1 * vrr1), ar0 + ar1, top);
-        vl = fast_face<DIVIDE>(fma_(al0, vlr0, al1 * vlr1), al0 + al1, top);
+        fast_faces<DIVIDE>(fma_(ar0, vrr0, ar1 * vrr1), ar0 + ar1, fma_(al0, vlr0, al1 * vlr1), al0 + al1, vl, vr, out);
     } else {
         const double vm2 = v[-2], vm1 = v[-1], v0 = v[0], vp1 = v[1], vp2 = v[2];
         // candidate stencils, c3 rows r+1 (right faces) and r (left faces)
@@ -338,15 +341,14 @@ HRW_HD void weno_cell_fast(const double *x, double eps, double &vl, double &vr, 
         const double sl = fma_(0.1, m0, fma_(0.6, m1, 0.3 * m2));
         const double nr = fma_(0.3 * m0, vrr0, fma_(0.6 * m1, vrr1, (0.1 * m2) * vrr2));
         const double nl = fma_(0.1 * m0, vlr0, fma_(0.6 * m1, vlr1, (0.3 * m2) * vlr2));
-        vr = fast_face<DIVIDE>(nr, sr, top);
-        vl = fast_face<DIVIDE>(nl, sl, top);
+        fast_faces<DIVIDE>(nr, sr, nl, sl, vl, vr, out);
     }
 }
 template <int K> HRW_HD void weno_cell_fast(const double *x, double eps, double &vl, double &vr)
 {
-    double top = 0.0;
-    weno_cell_fast<K, false>(x, eps, vl, vr, top);
-    if (!(top < kQuotTop)) weno_cell_fast<K, true>(x, eps, vl, vr, top);
+    bool out = false;
+    weno_cell_fast<K, false>(x, eps, vl, vr, out);
+    if (out) weno_cell_fast<K, true>(x, eps, vl, vr, out);
 }
 
 // --------------------------------------------------------------------------------------

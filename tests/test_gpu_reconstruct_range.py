@@ -59,6 +59,8 @@ def states(n):
     yield "ordinary", sign * 10.0 ** rng.uniform(-8, 8, n)
     yield "large", sign * 10.0 ** rng.uniform(25, 34, n)
     yield "overflow", sign * 10.0 ** rng.uniform(33.5, 39, n)
+    yield "sums at the overflow", sign * rng.uniform(2e38, 3.6e38, n)
+    yield "they and zeros", sign * rng.uniform(2e38, 3.6e38, n) * (rng.random(n) < 0.5)
     yield "overflow of pairs", sign * 10.0 ** rng.uniform(58, 80, n)
     yield "mixed", sign * 10.0 ** rng.uniform(-320, 60, n)
     yield "flat", np.full(n, 3e37)

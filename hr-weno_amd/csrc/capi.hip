@@ -2221,13 +2221,14 @@ static int batch_chunks(hrw_batch_s *b, int R)
 
 // Block table of the whole-integration kernel: lines longer than a block first (their blocks
 // exchange, and only they have words), each over equal blocks, then the others, the longest first.
-// Measured, us per RK3 step against one launch per stage: 1024 lines of 256-65536 cells (LF) 138 /
-// 183, the same with the Godunov flux 120 / 183, 475 lines of 454-18274 cells 50 / 73, 256 of
-// 1024-16384 31 / 54, 8 of 30000-65000 13 / 33.  Short lines, which leave the chip half idle, go at
-// two cells per lane (800 lines of 64-2000 cells: 125 us per 8 steps, 140 at four)  An ensemble of
-// many rounds of blocks goes at five: a block computes longer for each wait (1024 lines of 256-65536
-// cells 142 us per step, 151 at four; 300 of them, 3.0 M cells, 44 / 47; but 64 lines of 5000-60000
-// 28 / 26; eight cells per lane spill: 229).
+// Measured, us per RK3 step against one launch per stage (12 steps a call, the first 6), Lax-Friedrichs
+// and Godunov: 1024 lines of 256-65536 cells 132 / 175, 108 / 174; 475 of 454-18274 28 / 55, 26 / 56;
+// 256 of 1024-16384 21 / 42, 19 / 43; 8 of 30000-65000 9.1 / 29, 8.0 / 29; 16 of 175-648 4.9 / 30,
+// 4.6 / 31.  Short lines, which leave the chip half idle, go at two cells per lane (800 lines of 64-2000
+// cells: 12.8 us per step, 13.8 at four).  An ensemble of many rounds of blocks goes at five: a block
+// computes longer for each wait, which outweighs the 32 registers that the five-cell kernel spills
+// (four: 8, or 1 with Godunov): 1024 lines 132 us per step, 143 at four; 300 of them, 4.4 M cells,
+// 51 / 56; but 256 lines of 1024-16384 22 / 21; eight cells per lane spill 49: 229.
 static int batch_resident_blocks(hrw_batch_s *b)
 {
     const int r = b->res_r = *std::max_element(b->h_n.begin(), b->h_n.end()) <= 2048 ? 2

@@ -317,9 +317,10 @@ __device__ __forceinline__ void pbe2d_wave(const Stage2DArgs &a)
     }
 }
 
-// Bound by FP64 issue (EXACT: about 290 VALU operations per cell, against 62 for its bytes).
-// 2048 x 2048 cells, per RK3 stage: EXACT 81 us with a divide for every quotient and the triples
-// formed per cell, 58 us with shared triples and reciprocals (weights_exact); FAST 41 us.
+// EXACT: bound by FP64 issue.  402 VALU instructions per cell, 309 of them FP64; the SIMDs issue them in
+// 84 % of the launch's busy cycles (profiles/pbe2d_2048.md).  2048 x 2048 cells, per RK3 stage: 81 us with
+// a divide for every quotient and the triples formed per cell, 58 us with shared triples and reciprocals
+// (weights_exact); FAST 41 us.
 template <int K, int BC, bool FAST>
 __global__ __launch_bounds__(kBlock) void pbe2d_kernel(Stage2DArgs a)
 {

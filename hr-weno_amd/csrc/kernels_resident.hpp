@@ -542,7 +542,8 @@ __device__ __forceinline__ void resident_part(const ResPart &a, const ResCoef *c
 }
 
 // One line over the whole grid.
-// (R = 8: three wavefronts per SIMD and 168 VGPRs)
+// (R = 8: three wavefronts per SIMD and 168 VGPRs.  Spilled VGPRs over several blocks, K = 3: 8-19 of
+// them there, 4-12 at R = 5, EXACT 11-21 at R = 4; a recording has the larger numbers.)
 template <int K, int FLUX, bool FAST, bool CNU, int R, bool ONE, bool REC>
 __global__ __launch_bounds__(R == 8 ? 768 : kResThreads) void resident_kernel(ResArgs a, int waves)
 {

@@ -436,8 +436,9 @@ class MsTvd(_Ode):
 
 class BurgersBatch:
     """Ensemble of independent periodic 1D Burgers lines of uneven length, each with its own
-    WENO order k, grid and time step, advanced together (one launch per RK3 stage for all
-    lines, optionally from a captured hipGraph).  The state is one flat device tensor; line l
+    WENO order k, grid and time step, advanced together (up to 64 steps in one launch with the
+    lines on the chip where they fit, else one launch per RK3 stage for all lines, optionally
+    from a captured hipGraph).  The state is one flat device tensor; line l
     is ``u[offsets[l]:offsets[l] + ncells[l]]``."""
 
     def __init__(self, ncells, k, dt, xmin=None, xmax=None, eps=1e-6, flux=LAX_FRIEDRICHS,
